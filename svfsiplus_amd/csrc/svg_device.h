@@ -210,7 +210,6 @@ unsigned long long coarse_generation(const svg_lhs* L);  // changes when the lev
 // Shared between the translation units.
 void krylov_free(KrylovWork& k);   // every buffer, pinned mirror and event of a Krylov workspace
 int lhs_ensure_trans(svg_lhs* L);  // block-transpose map (pattern must be symmetric)
-int spmv_residual(const svg_lhs* L, const double* K, const double* U, const double* B, double* out, hipStream_t s);
 int lpc_prepare_dev(svg_lhs* L, const double* Val, hipStream_t s);
 // nsc: per-node (sc, 1/sc); sysOf/st: skip the rows of batched systems that stopped iterating.
 int lpc_apply_dev(svg_lpc* N, const svg_lhs* L, const double* V, double* Z, float* Z32, const int* skip,

@@ -1542,13 +1542,6 @@ static void op_apply(const Op& A, const double* x, double* y, const double* b, c
   }
 }
 
-int spmv_residual(const svg_lhs* L, const double* K, const double* U, const double* B, double* out, hipStream_t s)
-{
-  spmv<4, 4, 1>(L, K, U, out, B, nullptr, s, "spmv_res");
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? SVG_OK : hip_check(e, "spmv_residual");
-}
-
 // One restart cycle (gmres.cpp:529-612 / :533-592): up to sD Arnoldi steps with
 // at most LOOKAHEAD steps enqueued beyond the host's last convergence check,
 // then the back substitution and X += sum y_j u_j. Returns after the cycle's

@@ -568,9 +568,51 @@ __global__ __launch_bounds__(BS) void k_layer(int n, int rows, const int* __rest
 }
 
 // ------------------------------------------------------------- backward ---
-// GZ = -(2/B) A^T Res on the FP64 scaled matrix (the transposed block of
-// row j's block k sits at trans[k]); one lane per (row, dof).
-__global__ __launch_bounds__(256) void k_spmvT(int nNo, const int* __restrict__ rowPtr,
+// Res_b = T_b - A Z_b and GZ_b = alpha A^T Res_b on the FP64 scaled matrix for
+// every stacked vector b in one launch: one lane per (row, dof) and NV vectors
+// (blockIdx.y: the next NV), each vector's sums in the block order of a launch
+// of its own. With NV > 1 the matrix is read once for NV vectors; small meshes
+// take NV = 1, whose lanes fill the chip (NV_MIN_LANES). One launch per vector
+// took 9 us for each of 8 vectors on the 15k-tet pipe, most of it latency.
+constexpr size_t NV_MIN_LANES = 1u << 19;  // lanes that fill the chip's 256 CUs 8 wavefronts deep
+
+template <int NV>
+__global__ __launch_bounds__(256) void k_residual_nv(int nNo, int nvec, const int* __restrict__ rowPtr,
+                                                     const int* __restrict__ colPtr, const double* __restrict__ K,
+                                                     const double* __restrict__ Z, const double* __restrict__ T,
+                                                     double* __restrict__ Res)
+{
+#pragma clang fp contract(off)
+  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int row = (int)(k >> 2), i = (int)(k & 3);
+  if (row >= nNo) return;
+  const size_t n4 = (size_t)4 * nNo, b0 = (size_t)blockIdx.y * NV;
+  const int nb = min(NV, nvec - (int)b0);
+  double acc[NV];
+#pragma unroll
+  for (int b = 0; b < NV; b++) acc[b] = 0.0;
+  for (int j = rowPtr[row]; j < rowPtr[row + 1]; j++) {
+    const double2* a = reinterpret_cast<const double2*>(K + 16 * (size_t)j + 4 * i);
+    const double2 a0 = a[0], a1 = a[1];
+    const size_t c = 4 * (size_t)colPtr[j];
+#pragma unroll
+    for (int b = 0; b < NV; b++)
+      if (b < nb) {
+        const double* u = Z + (b0 + b) * n4 + c;
+        double t = acc[b] + a0.x * u[0];
+        t = t + a0.y * u[1];
+        t = t + a1.x * u[2];
+        acc[b] = t + a1.y * u[3];
+      }
+  }
+#pragma unroll
+  for (int b = 0; b < NV; b++)
+    if (b < nb) Res[(b0 + b) * n4 + k] = T[(b0 + b) * n4 + k] - acc[b];
+}
+
+// The transposed block of row j's block k sits at trans[k].
+template <int NV>
+__global__ __launch_bounds__(256) void k_spmvT(int nNo, int nvec, const int* __restrict__ rowPtr,
                                                const int* __restrict__ colPtr, const int* __restrict__ trans,
                                                const double* __restrict__ K, const double* __restrict__ U,
                                                double* __restrict__ Y, double alpha)
@@ -578,13 +620,25 @@ __global__ __launch_bounds__(256) void k_spmvT(int nNo, const int* __restrict__ 
   const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int j = (int)(k >> 2), e = (int)(k & 3);
   if (j >= nNo) return;
-  double acc = 0.0;
+  const size_t n4 = (size_t)4 * nNo, b0 = (size_t)blockIdx.y * NV;
+  const int nb = min(NV, nvec - (int)b0);
+  double acc[NV];
+#pragma unroll
+  for (int b = 0; b < NV; b++) acc[b] = 0.0;
   for (int q = rowPtr[j]; q < rowPtr[j + 1]; q++) {
     const double* a = K + 16 * (size_t)trans[q] + e;
-    const double* u = U + 4 * (size_t)colPtr[q];
-    acc += a[0] * u[0] + a[4] * u[1] + a[8] * u[2] + a[12] * u[3];
+    const double a0 = a[0], a1 = a[4], a2 = a[8], a3 = a[12];
+    const size_t c = 4 * (size_t)colPtr[q];
+#pragma unroll
+    for (int b = 0; b < NV; b++)
+      if (b < nb) {
+        const double* u = U + (b0 + b) * n4 + c;
+        acc[b] += a0 * u[0] + a1 * u[1] + a2 * u[2] + a3 * u[3];
+      }
   }
-  Y[k] = alpha * acc;
+#pragma unroll
+  for (int b = 0; b < NV; b++)
+    if (b < nb) Y[(b0 + b) * n4 + k] = alpha * acc[b];
 }
 
 __global__ __launch_bounds__(256) void k_sqsum(size_t n, const double* __restrict__ x, double* __restrict__ part)
@@ -705,37 +759,56 @@ __global__ __launch_bounds__(BS) void k_layer_bwd(int rows, const float* __restr
 }
 
 // Transposed message passing: Gin[j] += sum_{i : j in row i} A_ij^T (x) GM[i];
-// one lane per (row j, channel c).
+// one lane per (row j, channel c), the block read as two 16-byte words (the
+// row's 16 lanes share it) and two blocks' loads issued before their sums.
+__device__ __forceinline__ void spmmT_block(float4& e, const uint4& lo4, const uint4& hi4, const float4& g)
+{
+  const unsigned r0[2] = {lo4.x, lo4.y}, r1[2] = {lo4.z, lo4.w}, r2[2] = {hi4.x, hi4.y}, r3[2] = {hi4.z, hi4.w};
+  const float gd[4] = {g.x, g.y, g.z, g.w};
+  const unsigned* row[4] = {r0, r1, r2, r3};  // A_ij row d: entries e = 0..3
+#pragma unroll
+  for (int d = 0; d < 4; d++) {
+    e.x = fmaf(lo(row[d][0]), gd[d], e.x);
+    e.y = fmaf(hi(row[d][0]), gd[d], e.y);
+    e.z = fmaf(lo(row[d][1]), gd[d], e.z);
+    e.w = fmaf(hi(row[d][1]), gd[d], e.w);
+  }
+}
+
 __global__ __launch_bounds__(256) void k_spmmT(int n, int rows, const int* __restrict__ rowPtr,
                                                const int* __restrict__ colPtr, const int* __restrict__ trans,
                                                const bf16* __restrict__ A16, const float* __restrict__ GM,
                                                float* __restrict__ Gin)
 {
+  constexpr int UNR = 4;
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int r = (int)(idx >> 4), c = (int)(idx & 15);
   if (r >= rows) return;
   const int b = r / n, j = r - b * n;
   const float* Gb = GM + (size_t)b * n * F + 4 * c;
-  float e0 = 0.f, e1 = 0.f, e2 = 0.f, e3 = 0.f;
-  for (int k = rowPtr[j]; k < rowPtr[j + 1]; k++) {
-    const int i = colPtr[k];
-    const bf16* a = A16 + 16 * (size_t)trans[k];  // A_ij, row-major [d][e]
-    const float4 g = *reinterpret_cast<const float4*>(Gb + (size_t)i * F);
-    const float gd[4] = {g.x, g.y, g.z, g.w};
+  float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int k1 = rowPtr[j + 1];
+  for (int k = rowPtr[j]; k < k1; k += UNR) {
+    uint4 a0[UNR], a1[UNR];
+    float4 g[UNR];
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-      e0 = fmaf(bf2f(a[4 * d + 0]), gd[d], e0);
-      e1 = fmaf(bf2f(a[4 * d + 1]), gd[d], e1);
-      e2 = fmaf(bf2f(a[4 * d + 2]), gd[d], e2);
-      e3 = fmaf(bf2f(a[4 * d + 3]), gd[d], e3);
-    }
+    for (int q = 0; q < UNR; q++)
+      if (k + q < k1) {
+        const uint4* a = reinterpret_cast<const uint4*>(A16 + 16 * (size_t)trans[k + q]);
+        a0[q] = a[0];
+        a1[q] = a[1];
+        g[q] = *reinterpret_cast<const float4*>(Gb + (size_t)colPtr[k + q] * F);
+      }
+#pragma unroll
+    for (int q = 0; q < UNR; q++)
+      if (k + q < k1) spmmT_block(e, a0[q], a1[q], g[q]);
   }
   float4* o = reinterpret_cast<float4*>(Gin + (size_t)r * F + 4 * c);
   float4 v = *o;
-  v.x += e0;
-  v.y += e1;
-  v.z += e2;
-  v.w += e3;
+  v.x += e.x;
+  v.y += e.y;
+  v.z += e.z;
+  v.w += e.w;
   *o = v;
 }
 
@@ -773,15 +846,47 @@ __global__ __launch_bounds__(BS) void k_enc_bwd(int n, int rows, const double* _
     }
 }
 
-// out[e] = sum_p part[p*len + e] (p in order).
-__global__ __launch_bounds__(256) void k_reduce(int nparts, int len, const float* __restrict__ part,
-                                                float* __restrict__ out)
+// out[e] = sum_p part[p*len + e] for two stacked sets of partials in one
+// launch (entries e < len of part, then e < lenB of partB into outB). A
+// workgroup takes 64 entries: wavefront w sums the partials p = w, w + 16, ...
+// in order with eight loads in flight, then the 16 sums are added in order.
+// One lane adding the up to 512 partials of its entry alone waited out a
+// memory latency each: 98 us per launch on the 15k-tet pipe, 0.78 of the 1.18 ms
+// a loss and gradient of 8 vectors took (0.30 ms with this reduction and the
+// residuals of all vectors in one launch).
+constexpr int RD_W = 16;
+
+__global__ __launch_bounds__(64 * RD_W) void k_reduce(int nparts, int len, const float* __restrict__ part,
+                                                      float* __restrict__ out, int lenB,
+                                                      const float* __restrict__ partB, float* __restrict__ outB)
 {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= len) return;
+  __shared__ float red[RD_W][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int nbA = (len + 63) / 64;
+  int e = blockIdx.x * 64 + lane;
+  if ((int)blockIdx.x >= nbA) {
+    e -= nbA * 64;
+    len = lenB;
+    part = partB;
+    out = outB;
+  }
+  const int ec = e < len ? e : len - 1;
   float s = 0.f;
-  for (int p = 0; p < nparts; p++) s += part[(size_t)p * len + e];
-  out[e] = s;
+  for (int p0 = w; p0 < nparts; p0 += 8 * RD_W) {
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = p0 + q * RD_W < nparts ? part[(size_t)(p0 + q * RD_W) * len + ec] : 0.f;
+#pragma unroll
+    for (int q = 0; q < 8; q++) s += v[q];
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && e < len) {
+    float a = red[0][lane];
+#pragma unroll
+    for (int q = 1; q < RD_W; q++) a += red[q][lane];
+    out[e] = a;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_adam(int np, float* __restrict__ p, const float* __restrict__ g,
@@ -1050,12 +1155,19 @@ static int lpc_loss_grad(svg_lpc* N, svg_lhs* L, const double* Val, int nvec, co
   if ((rc = lpc_forward(N, L, nvec, R, N->Z, nullptr, true, nullptr, s))) return rc;
   const double sc = std::sqrt((double)n);
   const unsigned nbv = blocks_for((size_t)4 * n, 256);
-  for (int b = 0; b < nvec; b++) {
-    const size_t o = (size_t)b * 4 * n;
-    // Res = T - A Z (FP64, the solver's SpMV), GZ = -(2/B) A^T Res
-    if ((rc = spmv_residual(L, Val, N->Z + o, (T ? T : R) + o, N->Res + o, s))) return rc;
-    launch("lpc_spmvT", k_spmvT, dim3(nbv), dim3(256), 0, s, n, (const int*)L->d_rowPtr, (const int*)L->d_colPtr,
-           (const int*)L->d_trans, Val, (const double*)(N->Res + o), N->GZ + o, -2.0 / nvec);
+  // Res = T - A Z (FP64, in the solver's SpMV order), GZ = -(2/B) A^T Res
+  const double* Tt = T ? T : R;
+  if ((size_t)4 * rows <= NV_MIN_LANES) {
+    launch("lpc_res", k_residual_nv<1>, dim3(nbv, nvec), dim3(256), 0, s, n, nvec, (const int*)L->d_rowPtr,
+           (const int*)L->d_colPtr, Val, (const double*)N->Z, Tt, N->Res);
+    launch("lpc_spmvT", k_spmvT<1>, dim3(nbv, nvec), dim3(256), 0, s, n, nvec, (const int*)L->d_rowPtr,
+           (const int*)L->d_colPtr, (const int*)L->d_trans, Val, (const double*)N->Res, N->GZ, -2.0 / nvec);
+  } else {
+    launch("lpc_res", k_residual_nv<4>, dim3(nbv, blocks_for(nvec, 4)), dim3(256), 0, s, n, nvec,
+           (const int*)L->d_rowPtr, (const int*)L->d_colPtr, Val, (const double*)N->Z, Tt, N->Res);
+    launch("lpc_spmvT", k_spmvT<4>, dim3(nbv, blocks_for(nvec, 4)), dim3(256), 0, s, n, nvec,
+           (const int*)L->d_rowPtr, (const int*)L->d_colPtr, (const int*)L->d_trans, Val, (const double*)N->Res,
+           N->GZ, -2.0 / nvec);
   }
   launch("lpc_loss", k_sqsum, dim3(256), dim3(256), 0, s, (size_t)rows * 4, (const double*)N->Res, N->sq);
   const unsigned ng = std::min<unsigned>(MAXGRID, blocks_for(rows, TILE));
@@ -1063,17 +1175,18 @@ static int lpc_loss_grad(svg_lpc* N, svg_lhs* L, const double* Val, int nvec, co
   float* g = N->g;
   launch("lpc_bwd", k_dec_bwd, dim3(ng), dim3(BS), 0, s, rows, (const double*)N->GZ, 1.0 / sc, pb + OFF_WD,
          (const bf16*)N->H[NL], N->G, N->part);
-  launch("lpc_bwd", k_reduce, dim3(blocks_for(4 * F, 256)), dim3(256), 0, s, (int)ng, 4 * F,
-         (const float*)N->part, g + OFF_WD);
+  auto reduce = [&](int len, const float* part, float* out, int lenB, const float* partB, float* outB) {
+    launch("lpc_bwd", k_reduce, dim3(blocks_for(len, 64) + blocks_for(lenB, 64)), dim3(64 * RD_W), 0, s, (int)ng, len,
+           part, out, lenB, partB, outB);
+  };
+  reduce(4 * F, N->part, g + OFF_WD, 0, nullptr, nullptr);
   float* Gout = N->G;
   float* Gin = N->G2;
   for (int l = NL - 1; l >= 0; l--) {
     launch("lpc_bwd", k_layer_bwd, dim3(ng), dim3(BS), 0, s, rows, (const float*)Gout, (const bf16*)N->H[l],
            (const bf16*)N->M[l], (const bf16*)N->P[l], pb + OFF_L + l * LSZ, Gin, N->GM, N->part,
            N->part + (size_t)ng * F * 2 * F);
-    launch("lpc_bwd", k_reduce, dim3(blocks_for(F * 2 * F, 256)), dim3(256), 0, s, (int)ng, F * 2 * F,
-           (const float*)N->part, g + OFF_L + l * LSZ);
-    launch("lpc_bwd", k_reduce, dim3(1), dim3(256), 0, s, (int)ng, F, (const float*)(N->part + (size_t)ng * F * 2 * F),
+    reduce(F * 2 * F, N->part, g + OFF_L + l * LSZ, F, N->part + (size_t)ng * F * 2 * F,
            g + OFF_L + l * LSZ + F * 2 * F);
     launch("lpc_bwd", k_spmmT, dim3(blocks_for((size_t)rows * 16, 256)), dim3(256), 0, s, n, rows,
            (const int*)L->d_rowPtr, (const int*)L->d_colPtr, (const int*)L->d_trans, (const bf16*)L->d_val16,
@@ -1082,8 +1195,7 @@ static int lpc_loss_grad(svg_lpc* N, svg_lhs* L, const double* Val, int nvec, co
   }
   launch("lpc_bwd", k_enc_bwd, dim3(ng), dim3(BS), 0, s, n, rows, R, sc, (const bf16*)L->d_diag16,
          (const float*)Gout, N->part);
-  launch("lpc_bwd", k_reduce, dim3(blocks_for(F * NIN, 256)), dim3(256), 0, s, (int)ng, F * NIN,
-         (const float*)N->part, g + OFF_W0);
+  reduce(F * NIN, N->part, g + OFF_W0, 0, nullptr, nullptr);
   SVG_HIP(hipGetLastError());
   SVG_HIP(hipMemcpyAsync(N->h_sq, N->sq, 256 * sizeof(double), hipMemcpyDeviceToHost, s));
   SVG_HIP(hipStreamSynchronize(s));

@@ -87,6 +87,34 @@ def test_lpc_gradient_matches_oracle(torch_cuda):
         assert rel < 1e-5, name  # observed <= 3e-7
 
 
+@pytest.mark.parametrize("nvec", [6, 8])
+def test_lpc_gradient_of_stacked_vectors(torch_cuda, nvec):
+    """A stack large enough that the residual kernels take four vectors per lane
+    (6: with a remainder) gives the mean of the one-vector calls. The forward
+    pass and the FP64 residuals of a vector do not depend on the stack (loss:
+    FP64 summation order only); the gradient's BF16 roundings are unchanged by
+    the factor 1/8, so for 8 vectors only the FP32 summation order differs."""
+    torch = torch_cuda
+    sys = _sys(torch, n=16)
+    net = L.LearnedPC(_params(5))
+    R = _vectors(torch, sys, nvec, 2)
+    lib = _lib.load()
+
+    def call(V):
+        loss, g = C.c_double(), np.empty(L.num_params(), dtype=np.float32)
+        _lib.check(lib.svg_lpc_loss_grad(net.h, sys.lhs.h, sys.Val.data_ptr(), V.shape[0], V.data_ptr(),
+                                         C.byref(loss), g.ctypes.data, _stream()))
+        return loss.value, g.astype(np.float64)
+
+    one = [call(R[b:b + 1].contiguous()) for b in range(nvec)]
+    loss, grad = call(R)
+    want = np.mean([o[0] for o in one])
+    assert abs(loss - want) <= 1e-12 * want
+    if nvec == 8:
+        g = np.mean([o[1] for o in one], axis=0)
+        assert np.linalg.norm(grad - g) <= 1e-5 * np.linalg.norm(g)
+
+
 def test_lpc_training_reduces_loss(torch_cuda):
     torch = torch_cuda
     sys = _sys(torch)
