@@ -511,6 +511,35 @@ __global__ __launch_bounds__(128) void k_b_fluid_tri3(int q0, int qn, const int4
   }
 }
 
+// The nodes of elements gE[0..nFe) (in range) on the host.
+__global__ __launch_bounds__(256) void k_face_parents(int nFe, const int* __restrict__ gE,
+                                                      const int4* __restrict__ ien, int4* __restrict__ out)
+{
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nFe) out[q] = ien[gE[q]];
+}
+
+static int face_parents(const svg_msh* M, int nFe, const int* gE, std::vector<int>& out)
+{
+  int *d_gE = nullptr, *d_out = nullptr;
+  int rc;
+  if ((rc = dev_alloc(&d_gE, (size_t)nFe)) || (rc = dev_alloc(&d_out, (size_t)4 * nFe))) {
+    dev_free(d_gE);
+    return rc;
+  }
+  out.resize((size_t)4 * nFe);
+  hipError_t e = hipMemcpy(d_gE, gE, sizeof(int) * nFe, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_face_parents, dim3(blocks_for(nFe, 256)), dim3(256), 0, 0, nFe, (const int*)d_gE,
+                       reinterpret_cast<const int4*>(M->d_ien0), reinterpret_cast<int4*>(d_out));
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(out.data(), d_out, sizeof(int) * out.size(), hipMemcpyDeviceToHost);
+  dev_free(d_gE);
+  dev_free(d_out);
+  return e == hipSuccess ? SVG_OK : hip_check(e, "svg_face_create: parents");
+}
+
 int construct_fluid_enqueue(svg_msh* M, const svg_fluid_params* p, const double* Ag, const double* Yg,
                             const double* Bf, double* R, double* Val, hipStream_t s)
 {
@@ -577,14 +606,17 @@ extern "C" int svg_face_create(const svg_msh* M, int nFe, const int* faceIEN, co
 {
   if (!M || !faceIEN || !gE || !out || nFe <= 0) return set_error(SVG_ERR_ARG, "svg_face_create: bad argument");
   const svg_lhs* L = M->lhs;
+  for (int e = 0; e < nFe; e++)
+    if (gE[e] < 0 || gE[e] >= M->nEl) return set_error(SVG_ERR_ARG, "svg_face_create: parent element out of range");
+  std::vector<int> parent;
+  int rc = face_parents(M, nFe, gE, parent);
+  if (rc) return rc;
   std::vector<int> ien4((size_t)4 * nFe);
   for (int e = 0; e < nFe; e++) {
-    const int E = gE[e];
-    if (E < 0 || E >= M->nEl) return set_error(SVG_ERR_ARG, "svg_face_create: parent element out of range");
     // the parent's node off the face (gnnb, nn.cpp:586-624)
     int inner = -1, found = 0;
     for (int b = 0; b < 4; b++) {
-      const int Bc = M->ien[4 * (size_t)E + b];
+      const int Bc = parent[4 * (size_t)e + b];
       bool on = false;
       for (int a = 0; a < 3; a++) on = on || (faceIEN[3 * (size_t)e + a] == Bc);
       if (on)
@@ -599,8 +631,7 @@ extern "C" int svg_face_create(const svg_msh* M, int nFe, const int* faceIEN, co
   }
   std::vector<int> color, slots;
   int nColors = 0;
-  int rc = color_elements(M->nNo, nFe, 3, faceIEN, color, &nColors);
-  if (rc) return rc;
+  if ((rc = color_elements(M->nNo, nFe, 3, faceIEN, color, &nColors))) return rc;
   if ((rc = slot_map(nFe, 3, faceIEN, L->rowPtr.data(), L->colPtr.data(), slots))) return rc;
   std::vector<int> off(nColors + 1, 0), order(nFe);
   for (int e = 0; e < nFe; e++) off[color[e] + 1]++;

@@ -300,11 +300,8 @@ struct svg_msh {
   std::vector<int> colorOff;   // nColors+1 offsets into the colour-sorted order
   double* d_x = nullptr;       // (3,nNo)
   int* d_ien = nullptr;        // (4, nEl) in colour-sorted order (int4 per element)
-  int* d_slot = nullptr;       // 16 slots per element, SoA: slot[p*nElPad + e]
   int* d_err = nullptr;        // zero-Jacobian flag (element index + 1)
   int* h_err = nullptr;        // pinned mirror
-  int nElPad = 0;
-  std::vector<int> ien;        // (4, nEl) in the caller's element order (face -> parent lookups)
   // Element-order assembly (construct_fluid): per block slot s of the pattern,
   // the element pairs that add to it, clist[cptr[s] .. cptr[s+1]) = e*16 + 4a + b
   // in increasing element order e, and the per-element record the gather reads.

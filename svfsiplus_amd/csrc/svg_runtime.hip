@@ -443,11 +443,9 @@ int svg_msh_create(const svg_lhs* L, int nEl, const int* IEN, int nNo, const dou
 {
   if (!L || !IEN || !x || !out || nEl <= 0) return set_error(SVG_ERR_ARG, "svg_msh_create: bad argument");
   if (nNo != L->nNo) return set_error(SVG_ERR_ARG, "svg_msh_create: nNo differs from the lhs");
-  std::vector<int> color, slots;
+  std::vector<int> color;
   int nColors = 0;
   int rc = color_elements(nNo, nEl, 4, IEN, color, &nColors);
-  if (rc) return rc;
-  rc = slot_map(nEl, 4, IEN, L->rowPtr.data(), L->colPtr.data(), slots);
   if (rc) return rc;
   // Colour-sorted order (stable: element order inside each colour).
   std::vector<int> off(nColors + 1, 0), order(nEl);
@@ -463,22 +461,18 @@ int svg_msh_create(const svg_lhs* L, int nEl, const int* IEN, int nNo, const dou
   M->nNo = nNo;
   M->nColors = nColors;
   M->colorOff = off;
-  M->nElPad = (nEl + 63) & ~63;
-  M->ien.assign(IEN, IEN + (size_t)4 * nEl);
-  std::vector<int> ien((size_t)4 * nEl), sl((size_t)16 * M->nElPad, 0);
+  std::vector<int> ien((size_t)4 * nEl);
   for (int q = 0; q < nEl; q++) {
     int e = order[q];
     for (int a = 0; a < 4; a++) ien[4 * (size_t)q + a] = IEN[4 * (size_t)e + a];
-    for (int p = 0; p < 16; p++) sl[(size_t)p * M->nElPad + q] = slots[16 * (size_t)e + p];
   }
   if ((rc = dev_alloc(&M->d_x, (size_t)3 * nNo)) || (rc = dev_alloc(&M->d_ien, (size_t)4 * nEl)) ||
-      (rc = dev_alloc(&M->d_slot, (size_t)16 * M->nElPad)) || (rc = dev_alloc(&M->d_err, 1))) {
+      (rc = dev_alloc(&M->d_err, 1))) {
     svg_msh_free(M);
     return rc;
   }
   hipError_t e = hipMemcpy(M->d_x, x, sizeof(double) * 3 * nNo, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(M->d_ien, ien.data(), sizeof(int) * ien.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(M->d_slot, sl.data(), sizeof(int) * sl.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(M->d_err, 0, sizeof(int));
   if (e == hipSuccess) e = hipHostMalloc((void**)&M->h_err, sizeof(int), hipHostMallocDefault);
   if (e != hipSuccess) {
@@ -507,7 +501,6 @@ int svg_msh_free(svg_msh* M)
   if (!M) return SVG_OK;
   dev_free(M->d_x);
   dev_free(M->d_ien);
-  dev_free(M->d_slot);
   dev_free(M->d_err);
   dev_free(M->d_ien0);
   dev_free(M->d_cptr);

@@ -10,12 +10,13 @@
 //
 // Colouring: Jones-Plassmann. Each element has a fixed pseudo-random
 // priority; in each round an uncoloured element whose priority is the
-// largest among the uncoloured elements at all four of its nodes (per-node
-// atomicMax) takes the smallest colour not yet used at its nodes (per-node
+// largest among the uncoloured elements at all four of its nodes (their
+// "head") takes the smallest colour not yet used at its nodes (per-node
 // 256-bit masks). Winners of a round share no node, so no two elements of a
 // colour share a node, and the result is the sequential greedy colouring in
-// decreasing priority order. The colour order is a stable radix sort of the
-// element ids by colour.
+// decreasing priority order. A round looks only at the nodes whose head
+// changed in the round before (k_jp_round). The colour order is a stable radix
+// sort of the element ids by colour.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -83,90 +84,146 @@ __device__ __forceinline__ unsigned mix32(unsigned x)
   return x;
 }
 
-__device__ __forceinline__ unsigned long long prio(int e)
-{
-  return ((unsigned long long)mix32((unsigned)e * 2654435761u + 0x9e3779b9u) << 32) | (unsigned)e;
-}
+// An element's priority: a bijection of its id, so no two are equal.
+__device__ __forceinline__ unsigned prio(int e) { return mix32((unsigned)e * 2654435761u + 0x9e3779b9u); }
 
-__global__ __launch_bounds__(256) void k_jp_propose(int nEl, const int4* __restrict__ ien,
-                                                    const int* __restrict__ color,
-                                                    unsigned long long* __restrict__ best)
-{
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nEl || color[e] >= 0) return;
-  const unsigned long long p = prio(e);
-  const int4 v = ien[e];
-  atomicMax(best + v.x, p);
-  atomicMax(best + v.y, p);
-  atomicMax(best + v.z, p);
-  atomicMax(best + v.w, p);
-}
+// Heads: per node and round parity, (round the node's head last changed << 32)
+// | element, kNoElem when every element of the node is coloured. A node's head
+// changes at most once a round, into the slot of the round's parity, so a
+// reader in round r finds the head before r in the newer of the two slots
+// unless a winner of round r already replaced it (stamp r), and then the node
+// is taken.
+constexpr unsigned kNoElem = 0xffffffffu;
 
-__global__ __launch_bounds__(256) void k_jp_select(int nEl, const int4* __restrict__ ien, int* __restrict__ color,
-                                                   const unsigned long long* __restrict__ best,
-                                                   unsigned long long* __restrict__ used, int* __restrict__ nDone,
-                                                   int* __restrict__ maxColor, int* __restrict__ err)
+// The uncoloured element other than `won` of the highest priority among
+// entries [c0, c1) of a node's element list (clist: 16 e + 4 a + b), by the
+// four lanes of a quad (each every fourth entry, 8 loads in flight).
+__device__ __forceinline__ unsigned jp_scan(const int* __restrict__ clist, int c0, int c1, const int* color, int won,
+                                            int quad)
 {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nEl || color[e] >= 0) return;
-  const unsigned long long p = prio(e);
-  const int4 v = ien[e];
-  if (best[v.x] != p || best[v.y] != p || best[v.z] != p || best[v.w] != p) return;
-  // e holds all four of its nodes this round: no other winner touches their masks
-  const int nd[4] = {v.x, v.y, v.z, v.w};
-  unsigned long long m[CW] = {0, 0, 0, 0};
+  unsigned best = kNoElem, bp = 0;
+  for (int c = c0 + quad; c < c1; c += 32) {
+    int e[8], col[8];
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+    for (int q = 0; q < 8; q++) e[q] = c + 4 * q < c1 ? clist[c + 4 * q] >> 4 : -1;
 #pragma unroll
-    for (int w = 0; w < CW; w++) m[w] |= used[(size_t)CW * nd[a] + w];
-  int c = -1;
-  for (int w = 0; w < CW && c < 0; w++)
-    if (~m[w]) c = 64 * w + __builtin_ctzll(~m[w]);
-  if (c < 0) {
-    atomicOr(err, 2);
-    color[e] = 0x7fffffff;  // leaves the loop; the error is reported
-    atomicAdd(nDone, 1);
-    return;
+    for (int q = 0; q < 8; q++) col[q] = e[q] >= 0 && e[q] != won ? color[e[q]] : 0;
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (col[q] < 0 && (best == kNoElem || prio(e[q]) > bp)) best = (unsigned)e[q], bp = prio(e[q]);
   }
-  color[e] = c;
 #pragma unroll
-  for (int a = 0; a < 4; a++) used[(size_t)CW * nd[a] + c / 64] |= 1ull << (c % 64);
-  atomicAdd(nDone, 1);
-  atomicMax(maxColor, c);
+  for (int o = 1; o < 4; o <<= 1) {
+    const unsigned ob = __shfl_xor(best, o, 4), op = __shfl_xor(bp, o, 4);
+    if (ob != kNoElem && (best == kNoElem || op > bp)) best = ob, bp = op;
+  }
+  return best;
 }
 
-// Colour-sorted element q = order[q0]: its nodes and 16 block slots (binary
-// search of each column in the row's sorted colPtr range).
-__global__ __launch_bounds__(256) void k_slots(int nEl, int nElPad, const int* __restrict__ order,
-                                               const int4* __restrict__ ien, const int* __restrict__ rowPtr,
-                                               const int* __restrict__ colPtr, int4* __restrict__ ienSorted,
-                                               int* __restrict__ slot, int* __restrict__ err)
+// Every node's first head (round 1) and the first list of changed nodes: all.
+__global__ __launch_bounds__(256) void k_jp_heads(int nNo, const int* __restrict__ diagPtr,
+                                                  const int* __restrict__ cptr, const int* __restrict__ clist,
+                                                  const int* __restrict__ color, unsigned long long* __restrict__ head,
+                                                  int* __restrict__ list, int* __restrict__ cnt)
 {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nEl) return;
-  const int4 v = ien[order[q]];
-  ienSorted[q] = v;
-  const int nd[4] = {v.x, v.y, v.z, v.w};
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, v = t >> 2;
+  if (v >= nNo) return;
+  const int s = diagPtr[v];
+  const unsigned e = jp_scan(clist, cptr[s], cptr[s + 1], color, -1, t & 3);
+  if ((t & 3) == 0) {
+    head[2 * (size_t)v] = kNoElem;
+    head[2 * (size_t)v + 1] = (1ull << 32) | e;
+    list[v] = v;
+    if (v == 0) cnt[0] = 0, cnt[1] = nNo, cnt[2] = 0;
+  }
+}
+
+// Round r: 16 lanes per node of `list` (the nodes whose head changed in round
+// r - 1), four per node of its head element e. e wins when it heads all four
+// of its nodes; of the nodes that changed, the first in e's order handles it.
+// The winner takes its colour, and its nodes' new heads (slots of parity r) go
+// to the next list. Lists' lengths rotate through three counters: read
+// (r - 1), written (r), cleared for the next round. What bounds a round is the
+// chain of dependent loads (list, element, heads, masks, colours): about 7 us
+// on any mesh, where the same round over every uncoloured element took 49 us
+// on the 240k-tet pipe (one contended counter above all).
+__global__ __launch_bounds__(256) void k_jp_round(int r, const int4* __restrict__ ien,
+                                                  const int* __restrict__ diagPtr, const int* __restrict__ cptr,
+                                                  const int* __restrict__ clist, int* color,
+                                                  unsigned long long* head, unsigned long long* __restrict__ used,
+                                                  const int* __restrict__ list, int* __restrict__ next,
+                                                  int* __restrict__ cnt, int* __restrict__ maxColor,
+                                                  int* __restrict__ err)
+{
+  const int n = cnt[(r - 1) % 3];
+  int* nNext = cnt + r % 3;
+  if (blockIdx.x == 0 && threadIdx.x == 0) cnt[(r + 1) % 3] = 0;
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 4, a = (threadIdx.x >> 2) & 3, quad = threadIdx.x & 3;
+  const unsigned long long group = 0xffffull << (lane & 48);
+  // whole groups of 16 lanes leave or go on together
+  for (int q = blockIdx.x * 16 + g; q < n; q += gridDim.x * 16) {
+    const int v = list[q];
+    const unsigned e = (unsigned)head[2 * (size_t)v + ((r - 1) & 1)];
+    if (e == kNoElem) continue;
+    const int4 w = ien[e];
+    const int m = a == 0 ? w.x : a == 1 ? w.y : a == 2 ? w.z : w.w;
+    const unsigned long long hp = head[2 * (size_t)m + ((r - 1) & 1)];
+    const unsigned long long hc =
+        __hip_atomic_load(head + 2 * (size_t)m + (r & 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool changed = (int)(hp >> 32) == r - 1;
+    const bool heads = (int)(hc >> 32) != r && (unsigned)(hp > hc ? hp : hc) == e;
+    const unsigned long long ch = __ballot(changed) & group;
+    if ((__ballot(heads) & group) != group) continue;  // e does not head every node
+    if (__shfl(m, (int)__builtin_ctzll(ch), 64) != v) continue;  // another changed node handles e
+    unsigned long long mk[CW];
 #pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int s = rowPtr[nd[a]], e = rowPtr[nd[a] + 1];
+    for (int k = 0; k < CW; k++) {
+      mk[k] = used[(size_t)CW * m + k];
+      mk[k] |= __shfl_xor(mk[k], 4, 16);
+      mk[k] |= __shfl_xor(mk[k], 8, 16);
+    }
+    int c = -1;
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      int lo = s, hi = e;  // first position with colPtr >= nd[b]
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (colPtr[mid] < nd[b])
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      if (lo == e || colPtr[lo] != nd[b]) {
-        atomicOr(err, 4);
-        lo = s;
-      }
-      slot[(size_t)(4 * a + b) * nElPad + q] = lo;
+    for (int k = 0; k < CW; k++)
+      if (c < 0 && ~mk[k]) c = 64 * k + __builtin_ctzll(~mk[k]);
+    if ((threadIdx.x & 15) == 0) {
+      color[e] = c < 0 ? 0x7fffffff : c;  // past 256 colours: reported at the end
+      if (c < 0)
+        atomicOr(err, 2);
+      else if (c > __hip_atomic_load(maxColor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(maxColor, c);
+    }
+    if (quad == 0 && c >= 0) used[(size_t)CW * m + c / 64] |= 1ull << (c % 64);
+    const int s = diagPtr[m];
+    const unsigned ne = jp_scan(clist, cptr[s], cptr[s + 1], color, (int)e, quad);
+    const int m0 = __shfl(m, 0, 16), m1 = __shfl(m, 4, 16), m2 = __shfl(m, 8, 16);
+    const bool twice = (a > 0 && m == m0) || (a > 1 && m == m1) || (a > 2 && m == m2);  // a degenerate element
+    if (quad == 0 && !twice) {
+      __hip_atomic_store(head + 2 * (size_t)m + (r & 1), ((unsigned long long)r << 32) | ne, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      if (ne != kNoElem) next[atomicAdd(nNext, 1)] = m;
     }
   }
+}
+
+// Colour-sorted element q = order[q]: its nodes.
+__global__ __launch_bounds__(256) void k_sorted_ien(int nEl, const int* __restrict__ order,
+                                                    const int4* __restrict__ ien, int4* __restrict__ ienSorted)
+{
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nEl) ienSorted[q] = ien[order[q]];
+}
+
+// Elements per colour (256 bins, LDS first).
+__global__ __launch_bounds__(256) void k_color_hist(int nEl, const int* __restrict__ color, int* __restrict__ hist)
+{
+  __shared__ int h[64 * CW];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  for (int e = blockIdx.x * 256 + threadIdx.x; e < nEl; e += gridDim.x * 256)
+    if (color[e] < 64 * CW) atomicAdd(&h[color[e]], 1);
+  __syncthreads();
+  if (h[threadIdx.x]) atomicAdd(hist + threadIdx.x, h[threadIdx.x]);
 }
 
 __global__ __launch_bounds__(256) void k_iota(int n, int* __restrict__ v)
@@ -440,37 +497,56 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
   const int nNo = L->nNo;
   Scratch S;
   int rc;
-  int *d_err = nullptr, *color = nullptr, *d_cnt = nullptr, *order = nullptr, *ids = nullptr, *colSorted = nullptr;
-  unsigned long long *best = nullptr, *used = nullptr;
+  int *d_err = nullptr, *color = nullptr, *d_cnt = nullptr, *order = nullptr, *ids = nullptr, *colSorted = nullptr,
+      *list[2] = {nullptr, nullptr}, *hist = nullptr;
+  unsigned long long *head = nullptr, *used = nullptr;
   if ((rc = S.get(&d_err, 1))) return rc;
   if ((rc = check_ien(4LL * nEl, d_IEN, nNo, d_err, s, "svg_msh_create_dev"))) return rc;
-  if ((rc = S.get(&color, nEl)) || (rc = S.get(&d_cnt, 2)) || (rc = S.get(&best, nNo)) ||
+  if ((rc = S.get(&color, nEl)) || (rc = S.get(&d_cnt, 4)) || (rc = S.get(&head, (size_t)2 * nNo)) ||
       (rc = S.get(&used, (size_t)CW * nNo)) || (rc = S.get(&order, nEl)) || (rc = S.get(&ids, nEl)) ||
-      (rc = S.get(&colSorted, nEl)))
+      (rc = S.get(&colSorted, nEl)) || (rc = S.get(&list[0], nNo)) || (rc = S.get(&list[1], nNo)) ||
+      (rc = S.get(&hist, 64 * CW)))
     return rc;
   const int4* ien4 = reinterpret_cast<const int4*>(d_IEN);
+  auto* M = new svg_msh();
+  struct Guard {  // a return before the end frees the mesh
+    svg_msh* m;
+    ~Guard() { svg_msh_free(m); }
+  } guard{M};
+  M->lhs = L;
+  M->nEl = nEl;
+  M->nNo = nNo;
+  // the element-order map first: its diagonal slots list each node's elements for the colouring
+  if ((rc = msh_gather_build(M, d_IEN, s))) return rc;
   SVG_HIP(hipMemsetAsync(color, 0xff, sizeof(int) * nEl, s));  // -1: uncoloured
   SVG_HIP(hipMemsetAsync(used, 0, sizeof(unsigned long long) * CW * nNo, s));
-  SVG_HIP(hipMemsetAsync(d_cnt, 0, 2 * sizeof(int), s));     // [0] coloured elements, [1] largest colour
+  SVG_HIP(hipMemsetAsync(d_cnt + 3, 0, sizeof(int), s));  // [0..2] list lengths, [3] largest colour
+  SVG_HIP(hipMemsetAsync(hist, 0, sizeof(int) * 64 * CW, s));
   const unsigned gE = blocks_for(nEl, 256);
-  int h[2] = {0, 0};
-  int rounds = 0;
-  while (h[0] < nEl) {
-    if (++rounds > 100000) return set_error(SVG_ERR_ARG, "svg_msh_create_dev: colouring did not finish");
-    // four rounds per host check: a round after the last element is coloured does nothing
-    for (int r = 0; r < 4; r++) {
-      SVG_HIP(hipMemsetAsync(best, 0, sizeof(unsigned long long) * nNo, s));
-      hipLaunchKernelGGL(k_jp_propose, dim3(gE), dim3(256), 0, s, nEl, ien4, (const int*)color, best);
-      hipLaunchKernelGGL(k_jp_select, dim3(gE), dim3(256), 0, s, nEl, ien4, color,
-                         (const unsigned long long*)best, used, d_cnt, d_cnt + 1, d_err);
+  hipLaunchKernelGGL(k_jp_heads, dim3(blocks_for((size_t)4 * nNo, 256)), dim3(256), 0, s, nNo,
+                     (const int*)L->d_diagPtr, (const int*)M->d_cptr, (const int*)M->d_clist, (const int*)color, head,
+                     list[1], d_cnt);
+  const unsigned gR = std::min(blocks_for((size_t)nNo, 16), 512u);
+  int h[4] = {0, 1, 0, 0};
+  int r = 1;
+  while (h[r % 3] > 0) {
+    if (r > 100000) return set_error(SVG_ERR_ARG, "svg_msh_create_dev: colouring did not finish");
+    // 32 rounds per host check: a round with an empty list does nothing
+    for (int k = 0; k < 32; k++) {
+      r++;
+      hipLaunchKernelGGL(k_jp_round, dim3(gR), dim3(256), 0, s, r, ien4, (const int*)L->d_diagPtr,
+                         (const int*)M->d_cptr, (const int*)M->d_clist, color, head, used,
+                         (const int*)list[(r - 1) & 1], list[r & 1], d_cnt, d_cnt + 3, d_err);
     }
-    SVG_HIP(hipMemcpyAsync(h, d_cnt, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    SVG_HIP(hipGetLastError());
+    SVG_HIP(hipMemcpyAsync(h, d_cnt, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
     SVG_HIP(hipStreamSynchronize(s));
   }
   int herr = 0;
   SVG_HIP(hipMemcpy(&herr, d_err, sizeof(int), hipMemcpyDeviceToHost));
   if (herr & 2) return set_error(SVG_ERR_ARG, "svg_msh_create_dev: more than 256 colours needed");
-  const int nColors = h[1] + 1;
+  const int nColors = h[3] + 1;
+  M->nColors = nColors;
   // colour order: stable radix sort of the element ids by colour
   hipLaunchKernelGGL(k_iota, dim3(gE), dim3(256), 0, s, nEl, ids);
   size_t tb = 0;
@@ -480,50 +556,23 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
   if ((rc = S.get(&tmp, tb))) return rc;
   SVG_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, (const int*)color, colSorted, (const int*)ids, order, nEl, 0,
                                              8, s));
-  std::vector<int> hc(nEl);
-  SVG_HIP(hipMemcpyAsync(hc.data(), colSorted, sizeof(int) * nEl, hipMemcpyDeviceToHost, s));
-  auto* M = new svg_msh();
-  M->lhs = L;
-  M->nEl = nEl;
-  M->nNo = nNo;
-  M->nColors = nColors;
-  M->nElPad = (nEl + 63) & ~63;
+  hipLaunchKernelGGL(k_color_hist, dim3(std::min(gE, 1024u)), dim3(256), 0, s, nEl, (const int*)color, hist);
+  SVG_HIP(hipGetLastError());
+  std::vector<int> hc(64 * CW);
+  SVG_HIP(hipMemcpyAsync(hc.data(), hist, sizeof(int) * hc.size(), hipMemcpyDeviceToHost, s));
   if ((rc = dev_alloc(&M->d_x, (size_t)3 * nNo)) || (rc = dev_alloc(&M->d_ien, (size_t)4 * nEl)) ||
-      (rc = dev_alloc(&M->d_slot, (size_t)16 * M->nElPad)) || (rc = dev_alloc(&M->d_err, 1))) {
-    svg_msh_free(M);
+      (rc = dev_alloc(&M->d_err, 1)))
     return rc;
-  }
-  hipError_t e = hipMemsetAsync(M->d_slot, 0, sizeof(int) * 16 * M->nElPad, s);
-  if (e == hipSuccess) e = hipMemsetAsync(d_err, 0, sizeof(int), s);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_slots, dim3(gE), dim3(256), 0, s, nEl, M->nElPad, (const int*)order, ien4,
-                       (const int*)L->d_rowPtr, (const int*)L->d_colPtr, reinterpret_cast<int4*>(M->d_ien),
-                       M->d_slot, d_err);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipMemcpyAsync(M->d_x, d_x, sizeof(double) * 3 * nNo, hipMemcpyDeviceToDevice, s);
-  if (e == hipSuccess) e = hipMemsetAsync(M->d_err, 0, sizeof(int), s);
-  M->ien.resize((size_t)4 * nEl);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(M->ien.data(), d_IEN, sizeof(int) * 4 * (size_t)nEl, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(&herr, d_err, sizeof(int), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&M->h_err, sizeof(int), hipHostMallocDefault);
-  if (e != hipSuccess) {
-    svg_msh_free(M);
-    return hip_check(e, "svg_msh_create_dev");
-  }
-  if (herr & 4) {
-    svg_msh_free(M);
-    return set_error(SVG_ERR_ARG, "slot_map: pattern does not contain an element pair");
-  }
+  hipLaunchKernelGGL(k_sorted_ien, dim3(gE), dim3(256), 0, s, nEl, (const int*)order, ien4,
+                     reinterpret_cast<int4*>(M->d_ien));
+  SVG_HIP(hipGetLastError());
+  SVG_HIP(hipMemcpyAsync(M->d_x, d_x, sizeof(double) * 3 * nNo, hipMemcpyDeviceToDevice, s));
+  SVG_HIP(hipMemsetAsync(M->d_err, 0, sizeof(int), s));
+  SVG_HIP(hipStreamSynchronize(s));
+  SVG_HIP(hipHostMalloc((void**)&M->h_err, sizeof(int), hipHostMallocDefault));
   M->colorOff.assign(nColors + 1, 0);
-  for (int q = 0; q < nEl; q++) M->colorOff[hc[q] + 1]++;
-  for (int c = 0; c < nColors; c++) M->colorOff[c + 1] += M->colorOff[c];
-  if ((rc = msh_gather_build(M, d_IEN, s))) {
-    svg_msh_free(M);
-    return rc;
-  }
+  for (int c = 0; c < nColors; c++) M->colorOff[c + 1] = M->colorOff[c] + hc[c];
+  guard.m = nullptr;
   *out = M;
   return SVG_OK;
 }
