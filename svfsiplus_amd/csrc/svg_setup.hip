@@ -143,66 +143,79 @@ __global__ __launch_bounds__(256) void k_jp_heads(int nNo, const int* __restrict
 // of its nodes; of the nodes that changed, the first in e's order handles it.
 // The winner takes its colour, and its nodes' new heads (slots of parity r) go
 // to the next list. Lists' lengths rotate through three counters: read
-// (r - 1), written (r), cleared for the next round. What bounds a round is the
-// chain of dependent loads (list, element, heads, masks, colours): about 7 us
-// on any mesh, where the same round over every uncoloured element took 49 us
-// on the 240k-tet pipe (one contended counter above all).
-__global__ __launch_bounds__(256) void k_jp_round(int r, const int4* __restrict__ ien,
-                                                  const int* __restrict__ diagPtr, const int* __restrict__ cptr,
-                                                  const int* __restrict__ clist, int* color,
-                                                  unsigned long long* head, unsigned long long* __restrict__ used,
-                                                  const int* __restrict__ list, int* __restrict__ next,
-                                                  int* __restrict__ cnt, int* __restrict__ maxColor,
-                                                  int* __restrict__ err)
+// (r - 1), written (r), cleared for the next round. The counter is added to
+// once per 64 nodes: one atomic per node on the one address, 5 ns each, took
+// 148 us per round on the 1.2M-tet pipe. What is left is the chain of
+// dependent loads (list, element, heads, masks, colours).
+constexpr int JP_G = 64;  // nodes per workgroup and pass
+
+__global__ __launch_bounds__(16 * JP_G) void k_jp_round(int r, const int4* __restrict__ ien,
+                                                        const int* __restrict__ diagPtr, const int* __restrict__ cptr,
+                                                        const int* __restrict__ clist, int* color,
+                                                        unsigned long long* head,
+                                                        unsigned long long* __restrict__ used,
+                                                        const int* __restrict__ list, int* __restrict__ next,
+                                                        int* __restrict__ cnt, int* __restrict__ maxColor,
+                                                        int* __restrict__ err)
 {
+  __shared__ int push[4 * JP_G], nPush, at;
   const int n = cnt[(r - 1) % 3];
-  int* nNext = cnt + r % 3;
   if (blockIdx.x == 0 && threadIdx.x == 0) cnt[(r + 1) % 3] = 0;
   const int lane = threadIdx.x & 63, g = threadIdx.x >> 4, a = (threadIdx.x >> 2) & 3, quad = threadIdx.x & 3;
   const unsigned long long group = 0xffffull << (lane & 48);
-  // whole groups of 16 lanes leave or go on together
-  for (int q = blockIdx.x * 16 + g; q < n; q += gridDim.x * 16) {
-    const int v = list[q];
-    const unsigned e = (unsigned)head[2 * (size_t)v + ((r - 1) & 1)];
-    if (e == kNoElem) continue;
-    const int4 w = ien[e];
-    const int m = a == 0 ? w.x : a == 1 ? w.y : a == 2 ? w.z : w.w;
-    const unsigned long long hp = head[2 * (size_t)m + ((r - 1) & 1)];
-    const unsigned long long hc =
-        __hip_atomic_load(head + 2 * (size_t)m + (r & 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool changed = (int)(hp >> 32) == r - 1;
-    const bool heads = (int)(hc >> 32) != r && (unsigned)(hp > hc ? hp : hc) == e;
-    const unsigned long long ch = __ballot(changed) & group;
-    if ((__ballot(heads) & group) != group) continue;  // e does not head every node
-    if (__shfl(m, (int)__builtin_ctzll(ch), 64) != v) continue;  // another changed node handles e
-    unsigned long long mk[CW];
+  for (int q0 = blockIdx.x * JP_G; q0 < n; q0 += gridDim.x * JP_G) {
+    if (threadIdx.x == 0) nPush = 0;
+    __syncthreads();
+    // whole groups of 16 lanes take part or do not
+    const int q = q0 + g;
+    const int v = q < n ? list[q] : 0;
+    const unsigned e = q < n ? (unsigned)head[2 * (size_t)v + ((r - 1) & 1)] : kNoElem;
+    if (e != kNoElem) {
+      const int4 w = ien[e];
+      const int m = a == 0 ? w.x : a == 1 ? w.y : a == 2 ? w.z : w.w;
+      const unsigned long long hp = head[2 * (size_t)m + ((r - 1) & 1)];
+      const unsigned long long hc =
+          __hip_atomic_load(head + 2 * (size_t)m + (r & 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool changed = (int)(hp >> 32) == r - 1;
+      const bool heads = (int)(hc >> 32) != r && (unsigned)(hp > hc ? hp : hc) == e;
+      const unsigned long long ch = __ballot(changed) & group;
+      // e heads every node, and v is the changed node that handles it
+      if ((__ballot(heads) & group) == group && __shfl(m, (int)__builtin_ctzll(ch), 64) == v) {
+        unsigned long long mk[CW];
 #pragma unroll
-    for (int k = 0; k < CW; k++) {
-      mk[k] = used[(size_t)CW * m + k];
-      mk[k] |= __shfl_xor(mk[k], 4, 16);
-      mk[k] |= __shfl_xor(mk[k], 8, 16);
-    }
-    int c = -1;
+        for (int k = 0; k < CW; k++) {
+          mk[k] = used[(size_t)CW * m + k];
+          mk[k] |= __shfl_xor(mk[k], 4, 16);
+          mk[k] |= __shfl_xor(mk[k], 8, 16);
+        }
+        int c = -1;
 #pragma unroll
-    for (int k = 0; k < CW; k++)
-      if (c < 0 && ~mk[k]) c = 64 * k + __builtin_ctzll(~mk[k]);
-    if ((threadIdx.x & 15) == 0) {
-      color[e] = c < 0 ? 0x7fffffff : c;  // past 256 colours: reported at the end
-      if (c < 0)
-        atomicOr(err, 2);
-      else if (c > __hip_atomic_load(maxColor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(maxColor, c);
+        for (int k = 0; k < CW; k++)
+          if (c < 0 && ~mk[k]) c = 64 * k + __builtin_ctzll(~mk[k]);
+        if ((threadIdx.x & 15) == 0) {
+          color[e] = c < 0 ? 0x7fffffff : c;  // past 256 colours: reported at the end
+          if (c < 0)
+            atomicOr(err, 2);
+          else if (c > __hip_atomic_load(maxColor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(maxColor, c);
+        }
+        if (quad == 0 && c >= 0) used[(size_t)CW * m + c / 64] |= 1ull << (c % 64);
+        const int s = diagPtr[m];
+        const unsigned ne = jp_scan(clist, cptr[s], cptr[s + 1], color, (int)e, quad);
+        const int m0 = __shfl(m, 0, 16), m1 = __shfl(m, 4, 16), m2 = __shfl(m, 8, 16);
+        const bool twice = (a > 0 && m == m0) || (a > 1 && m == m1) || (a > 2 && m == m2);  // a degenerate element
+        if (quad == 0 && !twice) {
+          __hip_atomic_store(head + 2 * (size_t)m + (r & 1), ((unsigned long long)r << 32) | ne, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+          if (ne != kNoElem) push[atomicAdd(&nPush, 1)] = m;
+        }
+      }
     }
-    if (quad == 0 && c >= 0) used[(size_t)CW * m + c / 64] |= 1ull << (c % 64);
-    const int s = diagPtr[m];
-    const unsigned ne = jp_scan(clist, cptr[s], cptr[s + 1], color, (int)e, quad);
-    const int m0 = __shfl(m, 0, 16), m1 = __shfl(m, 4, 16), m2 = __shfl(m, 8, 16);
-    const bool twice = (a > 0 && m == m0) || (a > 1 && m == m1) || (a > 2 && m == m2);  // a degenerate element
-    if (quad == 0 && !twice) {
-      __hip_atomic_store(head + 2 * (size_t)m + (r & 1), ((unsigned long long)r << 32) | ne, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      if (ne != kNoElem) next[atomicAdd(nNext, 1)] = m;
-    }
+    __syncthreads();
+    if (threadIdx.x == 0 && nPush) at = atomicAdd(cnt + r % 3, nPush);
+    __syncthreads();
+    if ((int)threadIdx.x < nPush) next[at + threadIdx.x] = push[threadIdx.x];
+    __syncthreads();
   }
 }
 
@@ -239,19 +252,33 @@ int bits_for(unsigned long long v)
   return b;
 }
 
-// Device scratch released on every return path.
+// Device scratch released on every return path, cut from blocks of at least
+// `hint` bytes: an allocation and its free cost about 0.1 ms each, so a set-up
+// call whose hint covers its arrays pays for one.
 struct Scratch {
-  std::vector<void*> p;
+  size_t hint, used = 0, cap = 0;
+  std::vector<void*> blocks;
+  explicit Scratch(size_t h) : hint(h) {}
   template <typename T>
   int get(T** out, size_t n)
   {
-    int rc = dev_alloc(out, n);
-    if (rc == SVG_OK) p.push_back((void*)*out);
-    return rc;
+    const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+    if (used + bytes > cap) {
+      unsigned char* b = nullptr;
+      const size_t want = std::max(bytes, hint);
+      int rc = dev_alloc(&b, want);
+      if (rc) return rc;
+      blocks.push_back(b);
+      cap = want;
+      used = 0;
+    }
+    *out = reinterpret_cast<T*>((unsigned char*)blocks.back() + used);
+    used += bytes;
+    return SVG_OK;
   }
   ~Scratch()
   {
-    for (void* q : p) (void)hipFree(q);
+    for (void* q : blocks) (void)hipFree(q);
   }
 };
 
@@ -349,7 +376,7 @@ int msh_gather_build(svg_msh* M, const int* d_IEN, hipStream_t s)
   if (reinterpret_cast<uintptr_t>(d_IEN) & 15)
     return set_error(SVG_ERR_ARG, "element-order assembly: IEN must be 16-byte aligned (read as int4)");
   const long long n = 16LL * nEl;
-  Scratch S;
+  Scratch S(sizeof(int) * 5 * (size_t)n + ((size_t)4 << 20));  // key, sorted, val; the sort's two buffers
   int rc;
   int *key = nullptr, *sorted = nullptr, *val = nullptr, *d_err = nullptr;
   if ((rc = dev_alloc(&M->d_ien0, (size_t)4 * nEl)) || (rc = dev_alloc(&M->d_cptr, (size_t)nnz + 1)) ||
@@ -415,12 +442,12 @@ int svg_lhs_create_dev(int nNo, int nEl, const int* d_IEN, int nFaces, svg_lhs**
     return set_error(SVG_ERR_ARG, "svg_lhs_create_dev: d_IEN must be 16-byte aligned (read as int4)");
   if ((unsigned long long)nNo * (unsigned long long)nNo >= (1ULL << 62))
     return set_error(SVG_ERR_ARG, "svg_lhs_create_dev: nNo too large");
-  Scratch S;
+  const long long K = 16LL * nEl + nNo;
+  Scratch S(sizeof(unsigned long long) * 4 * (size_t)std::min(K, 0x7fffffffLL) + ((size_t)4 << 20));
   int rc;
   int* d_err = nullptr;
   if ((rc = S.get(&d_err, 1))) return rc;
   if ((rc = check_ien(4LL * nEl, d_IEN, nNo, d_err, s, "svg_lhs_create_dev"))) return rc;
-  const long long K = 16LL * nEl + nNo;
   if (K > 0x7fffffffLL) return set_error(SVG_ERR_ARG, "svg_lhs_create_dev: too many node pairs");
   unsigned long long *keys = nullptr, *sorted = nullptr, *uniq = nullptr;
   int* d_nnz = nullptr;
@@ -495,7 +522,8 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
   if (reinterpret_cast<uintptr_t>(d_IEN) & 15)
     return set_error(SVG_ERR_ARG, "svg_msh_create_dev: d_IEN must be 16-byte aligned (read as int4)");
   const int nNo = L->nNo;
-  Scratch S;
+  // per element the colour, order and id arrays and the sort's buffers, per node heads, masks and lists
+  Scratch S(sizeof(int) * 6 * (size_t)nEl + (16 + 8 * CW + 8) * (size_t)nNo + ((size_t)4 << 20));
   int rc;
   int *d_err = nullptr, *color = nullptr, *d_cnt = nullptr, *order = nullptr, *ids = nullptr, *colSorted = nullptr,
       *list[2] = {nullptr, nullptr}, *hist = nullptr;
@@ -526,7 +554,7 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
   hipLaunchKernelGGL(k_jp_heads, dim3(blocks_for((size_t)4 * nNo, 256)), dim3(256), 0, s, nNo,
                      (const int*)L->d_diagPtr, (const int*)M->d_cptr, (const int*)M->d_clist, (const int*)color, head,
                      list[1], d_cnt);
-  const unsigned gR = std::min(blocks_for((size_t)nNo, 16), 512u);
+  const unsigned gR = std::min(blocks_for((size_t)nNo, JP_G), 512u);
   int h[4] = {0, 1, 0, 0};
   int r = 1;
   while (h[r % 3] > 0) {
@@ -534,7 +562,7 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
     // 32 rounds per host check: a round with an empty list does nothing
     for (int k = 0; k < 32; k++) {
       r++;
-      hipLaunchKernelGGL(k_jp_round, dim3(gR), dim3(256), 0, s, r, ien4, (const int*)L->d_diagPtr,
+      hipLaunchKernelGGL(k_jp_round, dim3(gR), dim3(16 * JP_G), 0, s, r, ien4, (const int*)L->d_diagPtr,
                          (const int*)M->d_cptr, (const int*)M->d_clist, color, head, used,
                          (const int*)list[(r - 1) & 1], list[r & 1], d_cnt, d_cnt + 3, d_err);
     }

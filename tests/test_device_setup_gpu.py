@@ -115,3 +115,36 @@ def test_device_setup_rejects_bad_connectivity(torch_cuda):
         DeviceLhs(p, d_ien=d_ien)
     with pytest.raises(RuntimeError, match="IEN entry out of range"):
         W.pattern(p.nNo, ien)
+
+
+@pytest.mark.parametrize("kind", ["pipe", "random"])
+def test_device_colouring_is_the_priority_greedy(torch_cuda, kind):
+    """The device colouring is the sequential greedy one in decreasing element
+    priority (the hash of the element id), element for element: on a pipe, and on
+    random connectivity whose elements repeat nodes and share most of them."""
+    from svfsiplus_amd.newton import DeviceLhs, DeviceMesh, device_arrays
+    rng = np.random.default_rng(4)
+    p = W.make_pipe(8)
+    if kind == "random":
+        ien = rng.integers(0, 90, (700, 4)).astype(np.int32)
+        p = W.Pipe(0, 0, rng.standard_normal((90, 3)), ien, np.zeros(90, np.int32), *W.pattern(90, ien), 0.3, 3.0)
+    d_ien, d_x = device_arrays(p)
+    L = DeviceLhs(p, d_ien=d_ien)
+    M = DeviceMesh(L, p, d_ien=d_ien, d_x=d_x)
+    off, ien = np.empty(M.nColors + 1, np.int32), np.empty((p.nEl, 4), np.int32)
+    _lib.call("svg_msh_colors", M.h, off.ctypes.data)
+    _lib.call("svg_msh_sorted_ien", M.h, ien.ctypes.data)
+    x = np.arange(p.nEl, dtype=np.uint32) * np.uint32(2654435761) + np.uint32(0x9E3779B9)
+    for shift, mul in ((16, 0x85EBCA6B), (13, 0xC2B2AE35)):
+        x = (x ^ (x >> np.uint32(shift))) * np.uint32(mul)
+    x ^= x >> np.uint32(16)
+    used = [set() for _ in range(p.nNo)]
+    color = np.empty(p.nEl, np.int64)
+    for e in np.argsort(-x.astype(np.int64)):
+        taken = set().union(*(used[v] for v in p.IEN[e]))
+        color[e] = next(c for c in range(257) if c not in taken)
+        for v in p.IEN[e]:
+            used[v].add(color[e])
+    assert M.nColors == color.max() + 1
+    assert np.array_equal(np.diff(off), np.bincount(color))
+    assert np.array_equal(ien, p.IEN[np.argsort(color, kind="stable")])
