@@ -3,20 +3,20 @@
 // fluid_3d_c (:1389-1689) and do_assem (lhsa.cpp:97-141), in two kernels:
 //
 //   k_fluid_elem    one element per lane over the whole mesh in one launch:
-//                   geometry, the Gauss-point scalars (tauM, tauC, tauB,
-//                   u.Nx, u'.Nx) and the element residual, stored as one
-//                   640-byte record per element;
-//   k_fluid_gather  one lane per 4x4 block of the pattern: the tangent
-//                   contributions of the elements that share the block's
-//                   node pair, formed from their records and added in
-//                   increasing element order; the lane of a diagonal block
-//                   adds the residual rows of its node the same way.
+//                   geometry, the Gauss-point values (u, u', tauM, tauC, tauB)
+//                   and the element residual, stored as one 512-byte record
+//                   per element;
+//   k_fluid_gather  one lane per element entry (element, a, b) in the order of
+//                   the block slots: the 4x4 tangent block of the entry formed
+//                   from the record, then the entries of each slot added in
+//                   increasing element order through LDS; the entries of a
+//                   diagonal block carry the residual rows of its node.
 //
 // Each block and residual row receives its element contributions in element
 // order, as the reference's element loop adds them, and every operation is
 // rounded separately (no contraction into fused multiply-adds, as in the
 // reference's build), so Val and R equal the reference's bit for bit. No
-// colouring and no atomics: each lane owns the block (row) it writes.
+// colouring and no atomics: each wavefront owns the blocks (rows) it writes.
 //
 // Specialisations, each exact for this element and material (the values
 // dropped are signed zeros, which leave every sum unchanged):
@@ -48,33 +48,30 @@ struct FluidConst {
   double N[4][4];  // N[g][a]
 };
 
-// Element record (kTet4Rec doubles per element, caller's element order), laid
-// out so that it is written in 16-byte pairs as the values are produced:
-//   [0] wl  [1] 0  [2+2g] tauM(g)  [3+2g] tauC(g)  [10+g] tauB(g)  [14..15] 0
-//   node chunk a at 16 + 16 a:
-//     [0..2] Nx(:,a)  [3] 0  [4+2g] uNx(g,a)  [5+2g] upNx(g,a)  [12..15] lR(0..3,a)
-constexpr int kRecNode = 16;
-static_assert(kTet4Rec == 16 + 4 * kRecNode, "element record layout");
-constexpr int kRecTauM = 2, kRecTauB = 10, kRecU = 4, kRecR = 12;
+// Element record (kTet4Rec doubles per element, caller's element order): four
+// 128-byte lines, each written whole and read by the gather in 16-byte pairs.
+//   line 0, at 4 a (a = 0..3):  Nx(0,a), Nx(1,a), Nx(2,a) (a = 3: wl), tauB(g = a)
+//   lines 1, 2, at 16 + 8 g:    u(0..2), u'(0..2), tauM, tauC at Gauss point g
+//   line 3, at 48 + 4 a:        lR(0..3, a)
+// Nx(2,3) is formed again as the element forms it, -Nx(2,0) - Nx(2,1) - Nx(2,2),
+// and u.Nx, u'.Nx from u, u' and Nx with the same operations.
+static_assert(kTet4Rec == 64, "element record layout");
+constexpr int kRecG = 16, kRecR = 48;
 
-__host__ __device__ __forceinline__ void put2(double* __restrict__ p, int k, double x, double y)
-{
-  *reinterpret_cast<double2*>(p + k) = make_double2(x, y);
-}
-
-__host__ __device__ __forceinline__ bool tet4_is_zero(double v)
+__device__ __forceinline__ bool tet4_is_zero(double v)
 {
   double a = fabs(v);
   double nrm = fmax(a, DBL_EPSILON);
   return (a / nrm) < 10.0 * DBL_EPSILON;
 }
 
-// One element: returns 1 (and writes nothing) on a zero Jacobian, else fills
-// its record. xl(3,4) coordinates, al(3,4) acceleration minus body force,
-// yl(4,4) velocity and pressure, as the reference's local arrays.
-__host__ __device__ __forceinline__ int tet4_element(const double (&xl)[3][4], const double (&al)[3][4],
-                                                     const double (&yl)[4][4], const FluidConst& C,
-                                                     double* __restrict__ rec)
+// One element: returns 1 on a zero Jacobian (its record is then of no use),
+// else 0. xl(3,4) coordinates, al(3,4) acceleration minus body force, yl(4,4)
+// velocity and pressure, as the reference's local arrays; put(line, v) stores
+// a line of the record.
+template <typename Put>
+__device__ __forceinline__ int tet4_element(const double (&xl)[3][4], const double (&al)[3][4],
+                                            const double (&yl)[4][4], const FluidConst& C, Put put)
 {
 #pragma clang fp contract(off)
   // ---- gnn, nn.cpp:503-540 (TET4 parent gradients are 0/1/-1: xXi = x_j - x_3)
@@ -86,7 +83,7 @@ __host__ __device__ __forceinline__ int tet4_element(const double (&xl)[3][4], c
   const double Jac = xXi[0][0] * xXi[1][1] * xXi[2][2] + xXi[0][1] * xXi[1][2] * xXi[2][0] +
                      xXi[0][2] * xXi[1][0] * xXi[2][1] - xXi[0][0] * xXi[1][2] * xXi[2][1] -
                      xXi[0][1] * xXi[1][0] * xXi[2][2] - xXi[0][2] * xXi[1][1] * xXi[2][0];
-  if (tet4_is_zero(Jac)) return 1;
+  const int bad = tet4_is_zero(Jac) ? 1 : 0;
   double xiX[3][3];
   xiX[0][0] = (xXi[1][1] * xXi[2][2] - xXi[1][2] * xXi[2][1]) / Jac;
   xiX[0][1] = (xXi[2][1] * xXi[0][2] - xXi[2][2] * xXi[0][1]) / Jac;
@@ -156,16 +153,7 @@ __host__ __device__ __forceinline__ int tet4_element(const double (&xl)[3][4], c
 #pragma unroll
     for (int a = 0; a < 4; a++) lR[i][a] = 0.0;
 
-  put2(rec, 14, 0.0, 0.0);
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    double* A = rec + 16 + kRecNode * a;
-    put2(A, 0, Nx[0][a], Nx[1][a]);
-    put2(A, 2, Nx[2][a], 0.0);
-  }
-
-  double gUpNx[4][4];
-  double tauB_prev = 0.0;
+  double gUpNx[4][4], tauBg[4], line[16];
 #pragma unroll
   for (int g = 0; g < 4; g++) {
     const double* N = C.N[g];
@@ -224,21 +212,21 @@ __host__ __device__ __forceinline__ int tet4_element(const double (&xl)[3][4], c
         lR[i][a] = lR[i][a] + wr * N[a] * rV3[i] + w * (Nx[0][a] * rM[0][i] + Nx[1][a] * rM[1][i] + Nx[2][a] * rM[2][i]);
       }
       gUpNx[g][a] = up[0] * Nx[0][a] + up[1] * Nx[1][a] + up[2] * Nx[2][a];
-      put2(rec + 16 + kRecNode * a, kRecU + 2 * g, u[0] * Nx[0][a] + u[1] * Nx[1][a] + u[2] * Nx[2][a],
-           gUpNx[g][a]);
     }
     // Brinkman term (fluid.cpp:2132-2138)
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
       for (int i = 0; i < 3; i++) lR[i][a] = lR[i][a] + muK * w * N[a] * (u[i] + up[i]);
-    if (g == 0)
-      put2(rec, 0, wl, 0.0);
-    put2(rec, kRecTauM + 2 * g, tauM, tauC);
-    if (g & 1)
-      put2(rec, kRecTauB + g - 1, tauB_prev, tauB);
-    else
-      tauB_prev = tauB;
+    tauBg[g] = tauB;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      line[8 * (g & 1) + i] = u[i];
+      line[8 * (g & 1) + 3 + i] = up[i];
+    }
+    line[8 * (g & 1) + 6] = tauM;
+    line[8 * (g & 1) + 7] = tauC;
+    if (g & 1) put(1 + g / 2, line);
   }
   // Continuity residual (fluid_3d_c, fluid.cpp:1655-1658), Gauss points in order.
 #pragma unroll
@@ -246,41 +234,67 @@ __host__ __device__ __forceinline__ int tet4_element(const double (&xl)[3][4], c
 #pragma unroll
     for (int a = 0; a < 4; a++) lR[3][a] = lR[3][a] + w * (C.N[g][a] * divU - gUpNx[g][a]);
 #pragma unroll
+  for (int a = 0; a < 4; a++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) line[4 * a + i] = lR[i][a];
+  put(3, line);
+#pragma unroll
   for (int a = 0; a < 4; a++) {
-    double* A = rec + 16 + kRecNode * a;
-    put2(A, kRecR, lR[0][a], lR[1][a]);
-    put2(A, kRecR + 2, lR[2][a], lR[3][a]);
+    line[4 * a + 0] = Nx[0][a];
+    line[4 * a + 1] = Nx[1][a];
+    line[4 * a + 2] = a < 3 ? Nx[2][a] : wl;
+    line[4 * a + 3] = tauBg[a];
   }
-  return 0;
+  put(0, line);
+  return bad;
 }
 
-// The 4x4 tangent block (a, b) of one element from its record: E the element
-// part, A and B the node chunks of a and b, Na/Nb the shape functions of a and
-// b at the four Gauss points; acc(4i+j) as lK(4i+j, a, b), summed over g in
-// order (fluid.cpp:2058-2130 momentum and pressure columns, 1662-1688
-// continuity rows).
-__host__ __device__ __forceinline__ void tet4_block(const double* __restrict__ E, const double* __restrict__ A,
-                                                    const double* __restrict__ B, const double (&Na)[4],
-                                                    const double (&Nb)[4], const FluidConst& C, double (&acc)[16])
+// A staged record in LDS (GA_RS 16-byte units): lines 0..2 as in memory, but
+// with Nx(2,3) in its place in line 0 and wl after line 2.
+constexpr int GA_RS = 25;  // 24 + 1: rows read by different lanes fall on different banks
+constexpr int GA_WL = 48;  // wl (in doubles)
+
+// The 4x4 tangent block (a, b) of one element from its staged record: acc(4i+j)
+// as lK(4i+j, a, b), summed over g in order (fluid.cpp:2058-2130 momentum and
+// pressure columns, 1662-1688 continuity rows). Na and Nb hold the shape
+// functions of a and b at the Gauss points. The loop over g is kept rolled,
+// the next point's values loaded ahead: unrolled, the four points' values and
+// their hoisted products take registers that leave two wavefronts per SIMD.
+__device__ __forceinline__ void tet4_block(const double2* __restrict__ rec, int a, int b, const double* Na,
+                                           const double* Nb, const FluidConst& C, double (&acc)[16])
 {
 #pragma clang fp contract(off)
   const double rho = C.rho, mu = C.mu, muK = mu * C.K;
   const double rho_amd = rho * C.amd;
-  const double wl = E[0];
-  const double Nxa[3] = {A[0], A[1], A[2]}, Nxb[3] = {B[0], B[1], B[2]};
+  const double* recd = reinterpret_cast<const double*>(rec);
+  const double2 la = rec[2 * a], lb = rec[2 * b];
+  const double wl = recd[GA_WL];
+  double2 q0 = rec[kRecG / 2], q1 = rec[kRecG / 2 + 1], q2 = rec[kRecG / 2 + 2], q3 = rec[kRecG / 2 + 3];
+  double qB = recd[3];
+  const double Nxa[3] = {la.x, la.y, recd[4 * a + 2]}, Nxb[3] = {lb.x, lb.y, recd[4 * b + 2]};
   const double NxNx = Nxa[0] * Nxb[0] + Nxa[1] * Nxb[1] + Nxa[2] * Nxb[2];
 #pragma unroll
   for (int k = 0; k < 16; k++) acc[k] = 0.0;
-#pragma unroll
+#pragma unroll 1
   for (int g = 0; g < 4; g++) {
-    const double uNxa = A[kRecU + 2 * g], uNxb = B[kRecU + 2 * g];
-    const double upNxa = A[kRecU + 2 * g + 1], upNxb = B[kRecU + 2 * g + 1];
-    const double tauM = E[kRecTauM + 2 * g], tauC = E[kRecTauM + 2 * g + 1], tauB = E[kRecTauB + g];
+    const double u0 = q0.x, u1 = q0.y, u2 = q1.x, p0 = q1.y, p1 = q2.x, p2 = q2.y;
+    const double tauM = q3.x, tauC = q3.y, tauB = qB;
+    const double Nag = Na[g], Nbg = Nb[g];
+    {
+      const double2* nx = rec + kRecG / 2 + 4 * min(g + 1, 3);
+      q0 = nx[0];
+      q1 = nx[1];
+      q2 = nx[2];
+      q3 = nx[3];
+      qB = recd[4 * min(g + 1, 3) + 3];
+    }
+    const double uNxa = u0 * Nxa[0] + u1 * Nxa[1] + u2 * Nxa[2], uNxb = u0 * Nxb[0] + u1 * Nxb[1] + u2 * Nxb[2];
+    const double upNxa = p0 * Nxa[0] + p1 * Nxa[1] + p2 * Nxa[2], upNxb = p0 * Nxb[0] + p1 * Nxb[1] + p2 * Nxb[2];
     const double uaNxa = uNxa + upNxa;
-    const double T1ub = -rho * uNxb - muK * Nb[g];  // updu(i,i,b)
+    const double T1ub = -rho * uNxb - muK * Nbg;  // updu(i,i,b)
     const double rtu = rho * tauM * uaNxa;
     // momentum, fluid.cpp:2058-2113
-    const double T1 = mu * NxNx + rho_amd * Nb[g] * (Na[g] + rho * tauM * uaNxa) + rho * Na[g] * (uNxb + upNxb) +
+    const double T1 = mu * NxNx + rho_amd * Nbg * (Nag + rho * tauM * uaNxa) + rho * Nag * (uNxb + upNxb) +
                       tauB * upNxa * upNxb;
 #pragma unroll
     for (int i = 0; i < 3; i++)
@@ -289,7 +303,7 @@ __host__ __device__ __forceinline__ void tet4_block(const double* __restrict__ E
         if (i == j) {
           const double T2 = (mu + tauC) * (Nxa[i] * Nxb[i]) - rtu * T1ub;
           acc[4 * i + j] = acc[4 * i + j] + wl * (T2 + T1);
-          acc[4 * i + j] = acc[4 * i + j] + muK * wl * Nb[g] * Na[g];
+          acc[4 * i + j] = acc[4 * i + j] + muK * wl * Nbg * Nag;
         } else {
           const double T2 = mu * (Nxa[j] * Nxb[i]) + tauC * (Nxa[i] * Nxb[j]);
           acc[4 * i + j] = acc[4 * i + j] + wl * T2;
@@ -297,20 +311,20 @@ __host__ __device__ __forceinline__ void tet4_block(const double* __restrict__ E
       }
     // pressure columns, fluid.cpp:2117-2130
 #pragma unroll
-    for (int i = 0; i < 3; i++) acc[4 * i + 3] = acc[4 * i + 3] - wl * (Nxa[i] * Nb[g] - Nxb[i] * rtu);
+    for (int i = 0; i < 3; i++) acc[4 * i + 3] = acc[4 * i + 3] - wl * (Nxa[i] * Nbg - Nxb[i] * rtu);
     // continuity rows, fluid.cpp:1662-1688
-    const double T1c = rho_amd * Nb[g];
+    const double T1c = rho_amd * Nbg;
 #pragma unroll
     for (int j = 0; j < 3; j++) {
       const double T2 = Nxa[j] * (T1ub - T1c);
-      acc[12 + j] = acc[12 + j] + wl * (Na[g] * Nxb[j] - tauM * T2);
+      acc[12 + j] = acc[12 + j] + wl * (Nag * Nxb[j] - tauM * T2);
     }
     acc[15] = acc[15] + wl * tauM * NxNx;
   }
 }
 
 // Gathers an element's local arrays (construct_fluid, fluid.cpp:575-598).
-__host__ __device__ __forceinline__ void tet4_gather(const int (&nd)[4], const double* __restrict__ X,
+__device__ __forceinline__ void tet4_gather(const int (&nd)[4], const double* __restrict__ X,
                                                     const double* __restrict__ Ag, const double* __restrict__ Yg,
                                                     const double* __restrict__ Bf, double (&xl)[3][4],
                                                     double (&al)[3][4], double (&yl)[4][4])
@@ -330,104 +344,249 @@ __host__ __device__ __forceinline__ void tet4_gather(const int (&nd)[4], const d
   }
 }
 
-__global__ __launch_bounds__(256) void k_fluid_elem(int nEl, const int4* __restrict__ ien,
-                                                    const double* __restrict__ X, const double* __restrict__ Ag,
-                                                    const double* __restrict__ Yg, const double* __restrict__ Bf,
-                                                    FluidConst C, double* __restrict__ rec, int* __restrict__ err)
+// One wavefront per 64 elements. A record leaves line by line through LDS, so
+// that each 16-byte store instruction writes eight whole 128-byte lines: stored
+// straight from the lanes, every store touched 64 lines and half of the lines
+// went to memory twice (1.63 GB written for 0.75 GB of records, 596 us on the
+// 1.2M-tet pipe; 155 us and 0.60 GB for 0.60 GB as here).
+constexpr int ELEM_LS = 9;  // LDS row stride of a line in 16-byte units (128 + 16: no bank conflicts)
+
+__global__ __launch_bounds__(64) void k_fluid_elem(int nEl, const int4* __restrict__ ien,
+                                                   const double* __restrict__ X, const double* __restrict__ Ag,
+                                                   const double* __restrict__ Yg, const double* __restrict__ Bf,
+                                                   FluidConst C, double* __restrict__ rec, int* __restrict__ err,
+                                                   volatile int* __restrict__ bad)
 {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nEl) return;
+  __shared__ double2 ls[64 * ELEM_LS];
+  const int t = threadIdx.x, e0 = blockIdx.x * 64, e = min(e0 + t, nEl - 1);
   const int4 v = ien[e];
   const int nd[4] = {v.x, v.y, v.z, v.w};
   double xl[3][4], al[3][4], yl[4][4];
   tet4_gather(nd, X, Ag, Yg, Bf, xl, al, yl);
-  if (tet4_element(xl, al, yl, C, rec + (size_t)kTet4Rec * e)) atomicMin(err, e);
-}
-
-__device__ __forceinline__ double sel4(const double (&v)[4], int a)
-{
-  return a == 0 ? v[0] : a == 1 ? v[1] : a == 2 ? v[2] : v[3];
-}
-
-// One lane per block slot s: Val(:, s) += the tangent blocks of its element
-// entries in element order; the lane of a diagonal block also adds the
-// residual rows of its node, R(:, i) += lR(:, a), in the same order.
-__global__ __launch_bounds__(256) void k_fluid_gather(int nnz, const int* __restrict__ sorder,
-                                                      const int* __restrict__ cptr, const int* __restrict__ clist,
-                                                      const int4* __restrict__ ien, const double* __restrict__ rec,
-                                                      FluidConst C, double* __restrict__ R, double* __restrict__ Val)
-{
-#pragma clang fp contract(off)
-  // each XCD walks one contiguous band of the lane order (its L2 keeps the
-  // element records of the band's rows)
-  const int bx = xcd_block(blockIdx.x, gridDim.x);
-  if (bx < 0) return;
-  const int t = bx * blockDim.x + threadIdx.x;
-  if (t >= nnz) return;
-  const int s = sorder[t];
-  const int c0 = cptr[s], c1 = cptr[s + 1];
-  if (c0 == c1) return;
-  double v[16];
-  double2* vp = reinterpret_cast<double2*>(Val + 16 * (size_t)s);
+  double2* out = reinterpret_cast<double2*>(rec) + (size_t)(kTet4Rec / 2) * e0;
+  const int rows = min(64, nEl - e0);
+  auto put = [&](int line, const double (&w)[16]) {
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const double2 t = vp[k];
-    v[2 * k] = t.x;
-    v[2 * k + 1] = t.y;
-  }
-  double r[4] = {0.0, 0.0, 0.0, 0.0};
-  int node = -1;
-  for (int c = c0; c < c1; c++) {
-    const int code = clist[c];
-    const int e = code >> 4, a = (code >> 2) & 3, b = code & 3;
-    const double* Er = rec + (size_t)kTet4Rec * e;
-    double E[14], A[16], B[12];
-#pragma unroll
-    for (int k = 0; k < 7; k++) {
-      const double2 t = reinterpret_cast<const double2*>(Er)[k];
-      E[2 * k] = t.x;
-      E[2 * k + 1] = t.y;
-    }
+    for (int k = 0; k < 8; k++) ls[t * ELEM_LS + k] = make_double2(w[2 * k], w[2 * k + 1]);
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      const double2 u = reinterpret_cast<const double2*>(Er + 16 + kRecNode * a)[k];
-      A[2 * k] = u.x;
-      A[2 * k + 1] = u.y;
+      const int q = 64 * k + t, r = q >> 3, c = q & 7;
+      if (r < rows) out[(size_t)(kTet4Rec / 2) * r + 8 * line + c] = ls[r * ELEM_LS + c];
     }
-#pragma unroll
-    for (int k = 0; k < 6; k++) {
-      const double2 u = reinterpret_cast<const double2*>(Er + 16 + kRecNode * b)[k];
-      B[2 * k] = u.x;
-      B[2 * k + 1] = u.y;
-    }
-    double Na[4], Nb[4];
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const double Ng[4] = {C.N[g][0], C.N[g][1], C.N[g][2], C.N[g][3]};
-      Na[g] = sel4(Ng, a);
-      Nb[g] = sel4(Ng, b);
-    }
-    double acc[16];
-    tet4_block(E, A, B, Na, Nb, C, acc);
-#pragma unroll
-    for (int k = 0; k < 16; k++) v[k] = v[k] + acc[k];
-    if (a == b) {
-      if (node < 0) {
-        const int4 nv = ien[e];
-        node = a == 0 ? nv.x : a == 1 ? nv.y : a == 2 ? nv.z : nv.w;
-        const double4 t = reinterpret_cast<const double4*>(R)[node];
-        r[0] = t.x;
-        r[1] = t.y;
-        r[2] = t.z;
-        r[3] = t.w;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; i++) r[i] = r[i] + A[kRecR + i];
-    }
+    __syncthreads();
+  };
+  if (tet4_element(xl, al, yl, C, put)) {
+    atomicMin(err, e);
+    *bad = 1;
+    __threadfence_system();
   }
+}
+
+// One lane per element entry in slot order, one wavefront per chunk: whole
+// slots [chunk[w], chunk[w+1]) with at most 64 entries between them (a slot of
+// more entries is a chunk of its own). The records of the chunk's elements
+// (uniq, at most kUniq of them, about 28) are staged in LDS by whole lines: a
+// lane reading its record from memory is an L1 access per lane and load, 2400
+// per wavefront, and those bounded the kernel (1557 us on the 1.2M-tet pipe).
+// A chunk with more elements (uniqN 0) goes kUniq entries at a time, each
+// entry's element staged as it comes. The lanes' blocks then replace the
+// records in LDS, and each of the chunk's slot values is summed over the
+// slot's entries in element order, 16 lanes per slot: Val is read and written
+// once, as whole lines, past the caches that keep the records (non-temporal).
+// Work per lane is the same everywhere; one lane per slot, as before, looped
+// over 1 to 24 and more entries, which needed lanes ordered by entry count to
+// balance and then re-read every record 6.5 times from memory (1207 us on the
+// 1.2M-tet pipe, 89 us of latency on the 15k-tet one; as here 1031 and 21 us,
+// FP64 issue, LDS and the load latency of three wavefronts per SIMD each
+// taking about half of the time).
+constexpr int GA_LS = 20;  // LDS row stride of an entry (doubles): 16 block values, 4 residual rows
+constexpr int GA_LDS = kUniq * GA_RS > 64 * GA_LS / 2 ? kUniq * GA_RS : 64 * GA_LS / 2;
+constexpr int GA_T = 3;    // slot values per lane loaded ahead of the blocks (12 slots; a chunk has about 10)
+
+// v + the entries q0 <= q < q1 of LDS column l, in order.
+__device__ __forceinline__ double slot_sum(double v, const double* l, int q0, int q1)
+{
+#pragma clang fp contract(off)
+  int q = q0;
+  for (; q + 4 <= q1; q += 4) {
+    const double x0 = l[q * GA_LS], x1 = l[(q + 1) * GA_LS], x2 = l[(q + 2) * GA_LS], x3 = l[(q + 3) * GA_LS];
+    v = v + x0;
+    v = v + x1;
+    v = v + x2;
+    v = v + x3;
+  }
+  for (; q < q1; q++) v = v + l[q * GA_LS];
+  return v;
+}
+
+__device__ __forceinline__ void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(256, 3) void k_fluid_gather(int nChunk, const int2* __restrict__ chunk,
+                                                         const int* __restrict__ cptr, const int* __restrict__ clist,
+                                                         const unsigned short* __restrict__ lcode,
+                                                         const int* __restrict__ uniq,
+                                                         const unsigned char* __restrict__ uniqN,
+                                                         const int* __restrict__ colPtr,
+                                                         const double* __restrict__ rec, FluidConst C,
+                                                         double* __restrict__ R, double* __restrict__ Val)
+{
+#pragma clang fp contract(off)
+  __shared__ double2 lds2[4][GA_LDS];
+  __shared__ double Nt[4][4];  // Nt[a][g]
+  __shared__ int segs[4][65];
+  // each XCD walks one contiguous band of the slots (its L2 keeps the element
+  // records of the band's rows)
+  const int bx = xcd_block(blockIdx.x, gridDim.x);
+  if (bx < 0) return;
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, w = 4 * bx + wv;
+  if (threadIdx.x < 16) Nt[threadIdx.x & 3][threadIdx.x >> 2] = C.N[threadIdx.x >> 2][threadIdx.x & 3];
+  __syncthreads();
+  if (w >= nChunk) return;
+  // a wavefront's time is its chain of dependent loads, so each step issues
+  // all it can: chunk and element list; then the slots' bounds, columns and
+  // values, the entries and the records; then the residual rows
+  const int2 w0 = chunk[w], w1 = chunk[w + 1];
+  const int nu = uniqN[w];
+  int uid = uniq[(size_t)kUniq * w + (lane & (kUniq - 1))];
+  const int s0 = w0.x, ns = w1.x - s0, c0 = w0.y, c1 = w1.y, step = nu ? 64 : kUniq;
+  int* seg = segs[wv];
+  const int sg = cptr[s0 + min(lane, ns)];
+  const int col = colPtr[s0 + min(lane >> 2, ns - 1)];
+  double v[GA_T];
 #pragma unroll
-  for (int k = 0; k < 8; k++) vp[k] = make_double2(v[2 * k], v[2 * k + 1]);
-  if (node >= 0) reinterpret_cast<double4*>(R)[node] = make_double4(r[0], r[1], r[2], r[3]);
+  for (int p = 0; p < GA_T; p++)
+    if (lane + 64 * p < 16 * ns) v[p] = __builtin_nontemporal_load(Val + 16 * (size_t)s0 + lane + 64 * p);
+  int node = -1;
+  double r = 0.0;
+  double2* L2 = lds2[wv];
+  const double* L = reinterpret_cast<const double*>(L2);
+  const double2* rec2 = reinterpret_cast<const double2*>(rec);
+  for (int base = c0; base < c1; base += step) {
+    const int c = base + lane, cend = min(c1, base + step);
+    // the elements of this pass and each entry's place among them
+    int code = 0, n = nu;
+    if (nu) {
+      if (c < cend) code = lcode[c];
+    } else {
+      n = cend - base;
+      if (c < cend) {
+        code = clist[c];
+        uid = code >> 4;
+        code = (lane << 4) | (code & 15);
+      }
+    }
+    // the records, eight lanes per line: lanes 8 j.. take the three lines of
+    // element 8 p + j (past the last: the last again)
+    static_assert(kUniq == 32, "four elements per group of eight lanes");
+    const int el = lane >> 3;
+    const double2* src0 = rec2 + (size_t)(kTet4Rec / 2) * __shfl(uid, min(el, n - 1), 64) + (lane & 7);
+    const double2* src1 = rec2 + (size_t)(kTet4Rec / 2) * __shfl(uid, min(el + 8, n - 1), 64) + (lane & 7);
+    const double2* src2 = rec2 + (size_t)(kTet4Rec / 2) * __shfl(uid, min(el + 16, n - 1), 64) + (lane & 7);
+    const double2* src3 = rec2 + (size_t)(kTet4Rec / 2) * __shfl(uid, min(el + 24, n - 1), 64) + (lane & 7);
+    const double2 x00 = src0[0], x01 = src0[8], x02 = src0[16];
+    const double2 x10 = src1[0], x11 = src1[8], x12 = src1[16];
+    const double2 x20 = src2[0], x21 = src2[8], x22 = src2[16];
+    const double2 x30 = src3[0], x31 = src3[8], x32 = src3[16];
+    if (base == c0) {
+      if (lane <= ns) seg[lane] = sg;
+      if (lane == 0 && ns == 64) seg[64] = c1;
+      wave_lds_sync();
+    }
+    // a diagonal entry's residual rows straight from its record, and (lane
+    // (slot k, row i)) the diagonal slots' sums, the node being the column
+    const int a = (code >> 2) & 3, b = code & 3;
+    const int e = __shfl(uid, code >> 4, 64);
+    double2 r0, r1;
+    const bool diag = c < cend && a == b;
+    if (diag) {
+      r0 = rec2[(size_t)(kTet4Rec / 2) * e + kRecR / 2 + 2 * a];
+      r1 = rec2[(size_t)(kTet4Rec / 2) * e + kRecR / 2 + 2 * a + 1];
+    }
+    // the entries of slot k in this pass
+    auto part = [&](int k, int& q0, int& q1) {
+      q0 = max(seg[k], base) - base;
+      q1 = min(seg[k + 1], cend) - base;
+    };
+    int q0, q1;
+    part(min(lane >> 2, ns - 1), q0, q1);
+    const int k0 = __shfl(code, q0 & 63, 64);  // the slot's first entry
+    if (node < 0 && lane < 4 * ns && q0 < q1 && ((k0 >> 2) & 3) == (k0 & 3)) {
+      node = col;
+      r = R[4 * (size_t)node + (lane & 3)];
+    }
+    {
+      double2* dst = L2 + GA_RS * el + (lane & 7);
+      dst[0] = x00;
+      dst[8] = x01;
+      dst[16] = x02;
+      dst[8 * GA_RS] = x10;
+      dst[8 * GA_RS + 8] = x11;
+      dst[8 * GA_RS + 16] = x12;
+      dst[16 * GA_RS] = x20;
+      dst[16 * GA_RS + 8] = x21;
+      dst[16 * GA_RS + 16] = x22;
+      dst[24 * GA_RS] = x30;
+      dst[24 * GA_RS + 8] = x31;
+      dst[24 * GA_RS + 16] = x32;
+    }
+    wave_lds_sync();
+    if (lane < n) {
+      double* d = reinterpret_cast<double*>(L2 + GA_RS * lane);
+      d[GA_WL] = d[14];
+      d[14] = -d[2] - d[6] - d[10];
+    }
+    wave_lds_sync();
+    double acc[16];
+    tet4_block(L2 + GA_RS * (code >> 4), a, b, Nt[a], Nt[b], C, acc);  // (a lane without an entry: unused)
+    wave_lds_sync();
+    {
+      double2* row = L2 + lane * (GA_LS / 2);
+#pragma unroll
+      for (int k = 0; k < 8; k++) row[k] = make_double2(acc[2 * k], acc[2 * k + 1]);
+      if (diag) {
+        row[8] = r0;
+        row[9] = r1;
+      }
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int p = 0; p < GA_T; p++) {
+      const int t = lane + 64 * p;
+      if (t < 16 * ns) {
+        part(t >> 4, q0, q1);
+        v[p] = slot_sum(v[p], L + (t & 15), q0, q1);
+      }
+    }
+    for (int t = lane + 64 * GA_T; t < 16 * ns; t += 64) {
+      part(t >> 4, q0, q1);
+      double* vp = Val + 16 * (size_t)s0 + t;
+      if (q0 < q1) *vp = slot_sum(*vp, L + (t & 15), q0, q1);
+    }
+    if (node >= 0) {
+      part(lane >> 2, q0, q1);
+      r = slot_sum(r, L + 16 + (lane & 3), q0, q1);
+    }
+    for (int t = lane + 64; t < 4 * ((ns + 15) & ~15); t += 64) {
+      const int k = min(t >> 2, ns - 1);
+      part(k, q0, q1);
+      const int kk = __shfl(code, q0 & 63, 64);
+      if (t >= 4 * ns || q0 >= q1 || ((kk >> 2) & 3) != (kk & 3)) continue;
+      double* rp = R + 4 * (size_t)colPtr[s0 + k] + (t & 3);
+      *rp = slot_sum(*rp, L + 16 + (t & 3), q0, q1);
+    }
+    wave_lds_sync();
+  }
+  if (c0 == c1) return;
+#pragma unroll
+  for (int p = 0; p < GA_T; p++)
+    if (lane + 64 * p < 16 * ns) __builtin_nontemporal_store(v[p], Val + 16 * (size_t)s0 + lane + 64 * p);
+  if (node >= 0) R[4 * (size_t)node + (lane & 3)] = r;
 }
 
 __global__ void k_set_int(int* p, int v) { *p = v; }
@@ -564,28 +723,47 @@ int construct_fluid_enqueue(svg_msh* M, const svg_fluid_params* p, const double*
     C.N[g][2] = xi[g][2];
     C.N[g][3] = 1.0 - xi[g][0] - xi[g][1] - xi[g][2];
   }
-  launch("set_int", k_set_int, dim3(1), dim3(1), 0, s, M->d_err, INT_MAX);
   const svg_lhs* L = M->lhs;
-  launch("fluid_elem", k_fluid_elem, dim3(blocks_for(M->nEl, 256)), dim3(256), 0, s, M->nEl,
-         reinterpret_cast<const int4*>(M->d_ien0), (const double*)M->d_x, Ag, Yg, Bf, C, M->d_rec, M->d_err);
-  // a zero Jacobian leaves its record unwritten; the gather still runs and
+  launch("fluid_elem", k_fluid_elem, dim3(blocks_for(M->nEl, 64)), dim3(64), 0, s, M->nEl,
+         reinterpret_cast<const int4*>(M->d_ien0), (const double*)M->d_x, Ag, Yg, Bf, C, M->d_rec, M->d_err,
+         (volatile int*)M->d_bad);
+  // a zero Jacobian leaves a record of infinities; the gather still runs and
   // construct_fluid_check reports the element (Val and R are then undefined,
   // as the reference stops with an exception)
-  launch("fluid_gather", k_fluid_gather, dim3((blocks_for(L->nnz, 256) + 7) & ~7u), dim3(256), 0, s, L->nnz,
-         (const int*)M->d_sorder, (const int*)M->d_cptr, (const int*)M->d_clist, reinterpret_cast<const int4*>(M->d_ien0),
+  launch("fluid_gather", k_fluid_gather, dim3((blocks_for(M->nChunk, 4) + 7) & ~7u), dim3(256), 0, s, M->nChunk,
+         (const int2*)M->d_chunk, (const int*)M->d_cptr, (const int*)M->d_clist, (const unsigned short*)M->d_lcode,
+         (const int*)M->d_uniq, (const unsigned char*)M->d_uniqN, (const int*)L->d_colPtr,
          (const double*)M->d_rec, C, R, Val);
   SVG_HIP(hipGetLastError());
   return SVG_OK;
 }
 
+// The flag is in mapped host memory: without an error the check costs the
+// synchronisation alone.
 int construct_fluid_check(svg_msh* M, hipStream_t s)
 {
-  SVG_HIP(hipMemcpyAsync(M->h_err, M->d_err, sizeof(int), hipMemcpyDeviceToHost, s));
   SVG_HIP(hipStreamSynchronize(s));
-  if (*M->h_err != INT_MAX) {
-    return set_error(SVG_ERR_JACOBIAN,
-                     "[construct_fluid] Jacobian for element " + std::to_string(*M->h_err) + " is < 0.");
-  }
+  if (!*(volatile int*)M->h_bad) return SVG_OK;
+  int e = 0;
+  SVG_HIP(hipMemcpyAsync(&e, M->d_err, sizeof(int), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, M->d_err, INT_MAX);
+  SVG_HIP(hipGetLastError());
+  SVG_HIP(hipStreamSynchronize(s));
+  *M->h_bad = 0;
+  return set_error(SVG_ERR_JACOBIAN, "[construct_fluid] Jacobian for element " + std::to_string(e) + " is < 0.");
+}
+
+// The zero-Jacobian flag of a mesh: the lowest such element (INT_MAX: none)
+// and the mapped host word that says there is one.
+int construct_fluid_flag(svg_msh* M)
+{
+  int rc = dev_alloc(&M->d_err, 1);
+  if (rc) return rc;
+  const int none = INT_MAX;
+  SVG_HIP(hipMemcpy(M->d_err, &none, sizeof(int), hipMemcpyHostToDevice));
+  SVG_HIP(hipHostMalloc((void**)&M->h_bad, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+  *M->h_bad = 0;
+  SVG_HIP(hipHostGetDevicePointer((void**)&M->d_bad, M->h_bad, 0));
   return SVG_OK;
 }
 

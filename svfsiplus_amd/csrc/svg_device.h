@@ -226,6 +226,7 @@ unsigned long long lpc_generation(const svg_lpc* N);
 int construct_fluid_enqueue(svg_msh* M, const svg_fluid_params* p, const double* Ag, const double* Yg,
                             const double* Bf, double* R, double* Val, hipStream_t s);
 int construct_fluid_check(svg_msh* M, hipStream_t s);
+int construct_fluid_flag(svg_msh* M);  // allocates the flag of a new mesh
 
 }  // namespace svg
 
@@ -300,22 +301,29 @@ struct svg_msh {
   std::vector<int> colorOff;   // nColors+1 offsets into the colour-sorted order
   double* d_x = nullptr;       // (3,nNo)
   int* d_ien = nullptr;        // (4, nEl) in colour-sorted order (int4 per element)
-  int* d_err = nullptr;        // zero-Jacobian flag (element index + 1)
-  int* h_err = nullptr;        // pinned mirror
+  int* d_err = nullptr;        // lowest element with a zero Jacobian (INT_MAX: none)
+  int* h_bad = nullptr;        // mapped host word: nonzero when d_err was written
+  int* d_bad = nullptr;        // device view of h_bad
   // Element-order assembly (construct_fluid): per block slot s of the pattern,
   // the element pairs that add to it, clist[cptr[s] .. cptr[s+1]) = e*16 + 4a + b
   // in increasing element order e, and the per-element record the gather reads.
   int* d_ien0 = nullptr;       // (4, nEl) in the caller's element order (int4 per element)
   int* d_cptr = nullptr;       // nnz + 1
   int* d_clist = nullptr;      // 16 nEl
-  int* d_sorder = nullptr;     // the nnz slots ordered by their entry count (the gather's lane order)
+  int nChunk = 0;              // the gather's wavefronts: chunk w takes slots [chunk[w].x, chunk[w+1].x)
+  int2* d_chunk = nullptr;     // nChunk + 1: first slot, its first entry
+  int* d_uniq = nullptr;       // kUniq per chunk: the elements of its entries, each once
+  unsigned char* d_uniqN = nullptr;   // their number (0: more than kUniq, uniq unused)
+  unsigned short* d_lcode = nullptr;  // per entry of clist: 16 (place in uniq) + 4 a + b
   double* d_rec = nullptr;     // kTet4Rec * nEl
 };
 
 // Doubles per element in the element-order assembly's record.
-constexpr int kTet4Rec = 80;
-// Builds d_ien0, d_cptr, d_clist and d_rec from the caller-order IEN on the
-// device (d_IEN: 4 nEl ints, 16-byte aligned); synchronises s.
+constexpr int kTet4Rec = 64;
+// Most elements whose records a wavefront of the gather stages at once.
+constexpr int kUniq = 32;
+// Builds d_ien0, d_cptr, d_clist, d_chunk and d_rec from the caller-order IEN
+// on the device (d_IEN: 4 nEl ints, 16-byte aligned); synchronises s.
 namespace svg {
 int msh_gather_build(svg_msh* M, const int* d_IEN, hipStream_t s);
 }

@@ -467,14 +467,12 @@ int svg_msh_create(const svg_lhs* L, int nEl, const int* IEN, int nNo, const dou
     for (int a = 0; a < 4; a++) ien[4 * (size_t)q + a] = IEN[4 * (size_t)e + a];
   }
   if ((rc = dev_alloc(&M->d_x, (size_t)3 * nNo)) || (rc = dev_alloc(&M->d_ien, (size_t)4 * nEl)) ||
-      (rc = dev_alloc(&M->d_err, 1))) {
+      (rc = construct_fluid_flag(M))) {
     svg_msh_free(M);
     return rc;
   }
   hipError_t e = hipMemcpy(M->d_x, x, sizeof(double) * 3 * nNo, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(M->d_ien, ien.data(), sizeof(int) * ien.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(M->d_err, 0, sizeof(int));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&M->h_err, sizeof(int), hipHostMallocDefault);
   if (e != hipSuccess) {
     svg_msh_free(M);
     return hip_check(e, "svg_msh_create: upload");
@@ -505,9 +503,12 @@ int svg_msh_free(svg_msh* M)
   dev_free(M->d_ien0);
   dev_free(M->d_cptr);
   dev_free(M->d_clist);
-  dev_free(M->d_sorder);
+  dev_free(M->d_chunk);
+  dev_free(M->d_uniq);
+  dev_free(M->d_uniqN);
+  dev_free(M->d_lcode);
   dev_free(M->d_rec);
-  if (M->h_err) (void)hipHostFree(M->h_err);
+  if (M->h_bad) (void)hipHostFree(M->h_bad);
   delete M;
   return SVG_OK;
 }

@@ -313,26 +313,68 @@ __global__ __launch_bounds__(256) void k_contrib_keys(int nEl, const int4* __res
   val[k] = (int)k;
 }
 
-// key[s] = (window of slot s's row) * 256 + its entry count (clamped to 255),
-// val[s] = s: the gather's lanes walk windows of kGatherRows rows in order and,
-// inside a window, the slots by entry count.
-constexpr int kGatherRows = 1024;
-__global__ __launch_bounds__(256) void k_slot_count(int nnz, const int* __restrict__ cptr,
-                                                    const int* __restrict__ clist, const int4* __restrict__ ien,
-                                                    int* __restrict__ key, int* __restrict__ val)
+// The gather's chunks (whole slots, at most 64 of them and 64 entries, a slot
+// of more entries alone), packed greedily along each window of kGatherRows
+// rows, one lane per window: FILL = false counts a window's chunks, true
+// writes their first slots from off[window] on. 16 rows (about 1440 entries)
+// leave half a chunk of 23 unfilled at a window's end.
+constexpr int kGatherRows = 16;
+template <bool FILL>
+__global__ __launch_bounds__(64) void k_chunks(int nWin, int nNo, int nnz, const int* __restrict__ rowPtr,
+                                               const int* __restrict__ cptr, int* __restrict__ off,
+                                               int2* __restrict__ chunk)
 {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nnz) return;
-  const int c0 = cptr[s], n = cptr[s + 1] - c0;
-  int row = 0;
-  if (n > 0) {
-    const int code = clist[c0];
-    const int4 v = ien[code >> 4];
-    const int a = (code >> 2) & 3;
-    row = a == 0 ? v.x : a == 1 ? v.y : a == 2 ? v.z : v.w;
+  const int w = blockIdx.x * 64 + threadIdx.x;
+  if (w >= nWin) return;
+  const int s1 = rowPtr[min(nNo, (w + 1) * kGatherRows)];
+  int n = FILL ? off[w] : 0;
+  int first = rowPtr[w * kGatherRows], c0 = cptr[first];
+  if (FILL && first < s1) chunk[n] = make_int2(first, c0);
+  const int open = first < s1 ? 1 : 0;
+  for (int s = first; s < s1; s += 8) {
+    int end[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) end[q] = cptr[min(s + q, s1 - 1) + 1];
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (s + q < s1 && s + q > first && (end[q] - c0 > 64 || s + q - first >= 64)) {
+        // slot s + q opens the next chunk
+        n++;
+        first = s + q;
+        c0 = q > 0 ? end[q - 1] : cptr[s];
+        if (FILL) chunk[n] = make_int2(first, c0);
+      }
   }
-  key[s] = (row / kGatherRows) * 256 + min(n, 255);
-  val[s] = s;
+  if (!FILL) off[w] = n + open;
+  if (FILL && w == nWin - 1) chunk[n + open] = make_int2(nnz, cptr[nnz]);
+}
+
+// The elements of each chunk's entries, each once in the order they first
+// appear, and every entry's place among them; one wavefront per chunk.
+__global__ __launch_bounds__(256) void k_chunk_uniq(int nChunk, const int2* __restrict__ chunk,
+                                                    const int* __restrict__ clist, int* __restrict__ uniq,
+                                                    unsigned char* __restrict__ uniqN,
+                                                    unsigned short* __restrict__ lcode)
+{
+  const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (w >= nChunk) return;
+  const int c0 = chunk[w].y, n = chunk[w + 1].y - c0;
+  const int code = lane < n ? clist[c0 + lane] : -1, e = code >> 4;
+  int first = -1;
+  for (int j = 0; j < min(n, 64); j++)
+    if (__shfl(e, j, 64) == e && first < 0) first = j;
+  const unsigned long long heads = __ballot(first == lane);
+  const int u = __popcll(heads);
+  if (n <= 64 && u <= kUniq) {
+    const int at = __popcll(heads & ((1ull << max(first, 0)) - 1));
+    if (first == lane) uniq[(size_t)kUniq * w + at] = e;
+    if (lane < n) lcode[c0 + lane] = (unsigned short)((at << 4) | (code & 15));
+    if (lane >= u && lane < kUniq) uniq[(size_t)kUniq * w + lane] = 0;
+    if (lane == 0) uniqN[w] = (unsigned char)u;
+  } else {
+    if (lane < kUniq) uniq[(size_t)kUniq * w + lane] = 0;
+    if (lane == 0) uniqN[w] = 0;
+  }
 }
 
 // cptr[s] = first position of slot s in the sorted keys (lower bound), s in [0, nnz].
@@ -402,24 +444,31 @@ int msh_gather_build(svg_msh* M, const int* d_IEN, hipStream_t s)
   hipLaunchKernelGGL(k_contrib_ptr, dim3(blocks_for((size_t)nnz + 1, 256)), dim3(256), 0, s, nnz, n,
                      (const int*)sorted, M->d_cptr);
   SVG_HIP(hipGetLastError());
-  // The gather's lane order: windows of rows in order and, inside a window,
-  // slots sorted (stably) by their entry count, so that the lanes of a
-  // wavefront loop over equally many entries (diagonal blocks have about four
-  // times the entries of the others) while the element records a window
-  // reads stay few enough for one XCD's L2.
-  if ((rc = dev_alloc(&M->d_sorder, (size_t)nnz))) return rc;
-  hipLaunchKernelGGL(k_slot_count, dim3(blocks_for((size_t)nnz, 256)), dim3(256), 0, s, nnz,
-                     (const int*)M->d_cptr, (const int*)M->d_clist, reinterpret_cast<const int4*>(M->d_ien0), key,
-                     val);
+  const int nWin = (L->nNo + kGatherRows - 1) / kGatherRows;
+  int *cnt = nullptr, *off = nullptr;
+  if ((rc = S.get(&cnt, (size_t)nWin + 1)) || (rc = S.get(&off, (size_t)nWin + 1))) return rc;
+  SVG_HIP(hipMemsetAsync(cnt + nWin, 0, sizeof(int), s));
+  hipLaunchKernelGGL(k_chunks<false>, dim3(blocks_for(nWin, 64)), dim3(64), 0, s, nWin, L->nNo, nnz,
+                     (const int*)L->d_rowPtr, (const int*)M->d_cptr, cnt, (int2*)nullptr);
   SVG_HIP(hipGetLastError());
-  const int endBit2 = bits_for((unsigned long long)(L->nNo / kGatherRows) * 256 + 255);
   size_t tb2 = 0;
-  SVG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb2, (const int*)key, sorted, (const int*)val, M->d_sorder,
-                                             nnz, 0, endBit2, s));
-  unsigned char* tmp2 = tmp;
-  if (tb2 > tb && (rc = S.get(&tmp2, tb2))) return rc;
-  SVG_HIP(hipcub::DeviceRadixSort::SortPairs(tmp2, tb2, (const int*)key, sorted, (const int*)val, M->d_sorder, nnz,
-                                             0, endBit2, s));
+  SVG_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb2, (const int*)cnt, off, nWin + 1, s));
+  unsigned char* tmp2 = nullptr;
+  if ((rc = S.get(&tmp2, tb2))) return rc;
+  SVG_HIP(hipcub::DeviceScan::ExclusiveSum(tmp2, tb2, (const int*)cnt, off, nWin + 1, s));
+  SVG_HIP(hipMemcpyAsync(&M->nChunk, off + nWin, sizeof(int), hipMemcpyDeviceToHost, s));
+  SVG_HIP(hipStreamSynchronize(s));
+  if ((rc = dev_alloc(&M->d_chunk, (size_t)M->nChunk + 1))) return rc;
+  hipLaunchKernelGGL(k_chunks<true>, dim3(blocks_for(nWin, 64)), dim3(64), 0, s, nWin, L->nNo, nnz,
+                     (const int*)L->d_rowPtr, (const int*)M->d_cptr, off, M->d_chunk);
+  SVG_HIP(hipGetLastError());
+  if ((rc = dev_alloc(&M->d_uniq, (size_t)kUniq * M->nChunk)) || (rc = dev_alloc(&M->d_uniqN, (size_t)M->nChunk)) ||
+      (rc = dev_alloc(&M->d_lcode, (size_t)n)))
+    return rc;
+  hipLaunchKernelGGL(k_chunk_uniq, dim3(blocks_for(M->nChunk, 4)), dim3(256), 0, s, M->nChunk,
+                     (const int2*)M->d_chunk, (const int*)M->d_clist, M->d_uniq, M->d_uniqN,
+                     M->d_lcode);
+  SVG_HIP(hipGetLastError());
   int herr = 0;
   SVG_HIP(hipMemcpyAsync(&herr, d_err, sizeof(int), hipMemcpyDeviceToHost, s));
   SVG_HIP(hipStreamSynchronize(s));
@@ -589,15 +638,13 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
   std::vector<int> hc(64 * CW);
   SVG_HIP(hipMemcpyAsync(hc.data(), hist, sizeof(int) * hc.size(), hipMemcpyDeviceToHost, s));
   if ((rc = dev_alloc(&M->d_x, (size_t)3 * nNo)) || (rc = dev_alloc(&M->d_ien, (size_t)4 * nEl)) ||
-      (rc = dev_alloc(&M->d_err, 1)))
+      (rc = construct_fluid_flag(M)))
     return rc;
   hipLaunchKernelGGL(k_sorted_ien, dim3(gE), dim3(256), 0, s, nEl, (const int*)order, ien4,
                      reinterpret_cast<int4*>(M->d_ien));
   SVG_HIP(hipGetLastError());
   SVG_HIP(hipMemcpyAsync(M->d_x, d_x, sizeof(double) * 3 * nNo, hipMemcpyDeviceToDevice, s));
-  SVG_HIP(hipMemsetAsync(M->d_err, 0, sizeof(int), s));
   SVG_HIP(hipStreamSynchronize(s));
-  SVG_HIP(hipHostMalloc((void**)&M->h_err, sizeof(int), hipHostMallocDefault));
   M->colorOff.assign(nColors + 1, 0);
   for (int c = 0; c < nColors; c++) M->colorOff[c + 1] = M->colorOff[c] + hc[c];
   guard.m = nullptr;

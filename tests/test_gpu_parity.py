@@ -145,6 +145,56 @@ def test_construct_fluid(torch_cuda, phys, n):
     assert np.array_equal(R1, R0) and np.array_equal(V1, V0)
 
 
+def _fan(m):
+    """Two cones of m tets each around the axis c - top, c - bottom: the slots of
+    the axis nodes have m and 2 m entries."""
+    t = np.arange(m) * (2.0 * np.pi / m)
+    x = np.concatenate([[[0, 0, 0], [0, 0, 1.1], [0.1, 0, -0.9]], np.stack([np.cos(t), np.sin(t), 0.1 * np.sin(5 * t)], 1)])
+    i, j = 3 + np.arange(m), 3 + (np.arange(m) + 1) % m
+    z = np.zeros(m, int)
+    ien = np.concatenate([np.stack([z, i, j, z + 1], 1), np.stack([z + 2, i, j, z], 1)])[np.random.default_rng(m).permutation(2 * m)]
+    return W.Pipe(0, 0, x, ien.astype(np.int32), np.zeros(len(x), np.int32), *W.pattern(len(x), ien), 1.0, 2.0)
+
+
+def _shuffled(n):
+    """The pipe with its nodes and elements in no order."""
+    p, rng = W.make_pipe(n), np.random.default_rng(n)
+    to = rng.permutation(p.nNo)
+    x = np.empty_like(p.x)
+    x[to] = p.x
+    ien = to[p.IEN][rng.permutation(p.nEl)].astype(np.int32)
+    return W.Pipe(n, 5 * n, x, ien, p.flags, *W.pattern(p.nNo, ien), p.radius, p.length)
+
+
+@pytest.mark.parametrize("mesh", ["one_tet", "shuffled6", "fan9", "fan31", "fan33", "fan64", "fan65", "fan120"])
+def test_construct_fluid_irregular(torch_cuda, phys, mesh):
+    """Meshes at the gather's limits: block slots of 1 to 240 entries (a wavefront
+    takes 64 entries, of up to 32 elements staged at once), rows whose elements
+    are in no order, sums onto R and Val that are not zero."""
+    from svfsiplus_amd.newton import DeviceLhs, DeviceMesh, construct_fluid, device_arrays
+    torch = torch_cuda
+    if mesh == "one_tet":
+        ien = np.array([[0, 1, 2, 3]], np.int32)
+        p = W.Pipe(0, 0, np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1.0]]), ien, np.zeros(4, np.int32),
+                   *W.pattern(4, ien), 1.0, 1.0)
+    else:
+        p = _shuffled(int(mesh[8:])) if mesh.startswith("shuffled") else _fan(int(mesh[3:]))
+    rng = np.random.default_rng(5)
+    Ag, Yg = rng.standard_normal((2, p.nNo, 4))
+    R0, V0 = oracle.construct_fluid(p, phys, Ag, Yg)
+    for dev in (False, True):
+        ien, x = device_arrays(p) if dev else (None, None)
+        L = DeviceLhs(p, faces=[], d_ien=ien)
+        M = DeviceMesh(L, p, d_ien=ien, d_x=x)
+        dR, dV = _dev(torch, np.zeros_like(R0)), _dev(torch, np.zeros_like(V0))
+        construct_fluid(M, phys, _dev(torch, Ag), _dev(torch, Yg), dR, dV)
+        assert np.array_equal(dR.cpu().numpy(), R0) and np.array_equal(dV.cpu().numpy(), V0), (mesh, dev)
+        # added to what is there, entry by entry: twice the same call, doubled to rounding
+        construct_fluid(M, phys, _dev(torch, Ag), _dev(torch, Yg), dR, dV)
+        for got, one in ((dR, R0), (dV, V0)):
+            assert np.abs(got.cpu().numpy() - 2 * one).max() <= 1e-12 * np.abs(one).max()
+
+
 @pytest.mark.parametrize("n", [4, 8])
 def test_gmres_solve(torch_cuda, phys, n):
     """gmres_v on the device: bitwise equal to the oracle run with the device's
