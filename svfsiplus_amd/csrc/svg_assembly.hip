@@ -32,6 +32,7 @@
 // Per-entry summation over Gauss points keeps the reference order g = 0..3.
 #include "svg_device.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 #include <cmath>
@@ -398,7 +399,7 @@ __global__ __launch_bounds__(64) void k_fluid_elem(int nEl, const int4* __restri
 // Work per lane is the same everywhere; one lane per slot, as before, looped
 // over 1 to 24 and more entries, which needed lanes ordered by entry count to
 // balance and then re-read every record 6.5 times from memory (1207 us on the
-// 1.2M-tet pipe, 89 us of latency on the 15k-tet one; as here 1031 and 21 us,
+// 1.2M-tet pipe, 89 us of latency on the 15k-tet one; as here 1035 and 20 us,
 // FP64 issue, LDS and the load latency of three wavefronts per SIMD each
 // taking about half of the time).
 constexpr int GA_LS = 20;  // LDS row stride of an entry (doubles): 16 block values, 4 residual rows
@@ -591,26 +592,27 @@ __global__ __launch_bounds__(256, 3) void k_fluid_gather(int nChunk, const int2*
 
 __global__ void k_set_int(int* p, int v) { *p = v; }
 
-// Neumann-face assembly of the fluid equation on TRI3 faces, one face element
-// per lane, launched per face colour: b_assem_neu_bc (eq_assem.cpp:58-172)
-// with gnnb's outward area normal (nn.cpp:552-760) and b_fluid
-// (fluid.cpp:46-133, fixed mesh): R(i,a) -= w N_a (h n_i + udn u_i),
-// Val(4i+i, a b) -= wl N_a N_b udn, udn = beta rho (u.n - |u.n|)/2.
+// Neumann-face assembly of the fluid equation on TRI3 faces: b_assem_neu_bc
+// (eq_assem.cpp:58-172) with gnnb's outward area normal (nn.cpp:552-760) and
+// b_fluid (fluid.cpp:46-133, fixed mesh): R(i,a) -= w N_a (h n_i + udn u_i),
+// Val(4i+i, a b) -= wl N_a N_b udn, udn = beta rho (u.n - |u.n|)/2. One
+// lane per block slot and per node of the face: it forms the terms of its
+// face elements itself and adds them in colour order (an element is formed by
+// its 12 lanes; at a face's size that is cheaper than a launch, and nothing is
+// kept between calls). One launch per face colour, as before, cost 5 to 12 us
+// of latency for each of 8 colours.
 struct FaceConst {
   double rho, beta, af, gam, dt;
   double N[3][3];         // N[g][a] at the three TRI3 Gauss points
 };
 
-__global__ __launch_bounds__(128) void k_b_fluid_tri3(int q0, int qn, const int4* __restrict__ ien,
-                                                      const int* __restrict__ slot, int nFePad,
-                                                      const double* __restrict__ x, const double* __restrict__ hg,
-                                                      const double* __restrict__ Yg, FaceConst C,
-                                                      double* __restrict__ R, double* __restrict__ Val)
+// The residual terms lR(i, a) of a face element (nd: its nodes, then the
+// parent's interior node), wl and udn at the Gauss points.
+__device__ __forceinline__ void face_terms(const int4& nd, const double* __restrict__ x, const double* __restrict__ hg,
+                                           const double* __restrict__ Yg, const FaceConst& C, double (&lR)[3][3],
+                                           double& wl, double (&udng)[3])
 {
 #pragma clang fp contract(off)
-  const int q = q0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= q0 + qn) return;
-  const int4 nd = ien[q];
   const int id[3] = {nd.x, nd.y, nd.z};
   double xl[3][3], yl[3][3], hl[3];
   for (int a = 0; a < 3; a++) {
@@ -638,9 +640,9 @@ __global__ __launch_bounds__(128) void k_b_fluid_tri3(int q0, int qn, const int4
   const double Jac = sqrt(nn);
   for (int i = 0; i < 3; i++) n[i] = n[i] / Jac;
   const double w = (1.0 / 6.0) * Jac;
-  const double wl = w * C.af * C.gam * C.dt;
-  double lR[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-  double lK[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+  wl = w * C.af * C.gam * C.dt;
+  for (int i = 0; i < 3; i++)
+    for (int a = 0; a < 3; a++) lR[i][a] = 0.0;
   for (int g = 0; g < 3; g++) {
     const double* N = C.N[g];
     double h = 0.0, y[3] = {0.0, 0.0, 0.0};
@@ -653,20 +655,53 @@ __global__ __launch_bounds__(128) void k_b_fluid_tri3(int q0, int qn, const int4
     udn = 0.50 * C.beta * C.rho * (udn - fabs(udn));
     double hc[3];
     for (int i = 0; i < 3; i++) hc[i] = h * n[i] + udn * y[i];
-    for (int a = 0; a < 3; a++) {
+    for (int a = 0; a < 3; a++)
       for (int i = 0; i < 3; i++) lR[i][a] = lR[i][a] - w * N[a] * hc[i];
-      for (int b = 0; b < 3; b++) lK[a][b] = lK[a][b] - wl * N[a] * N[b] * udn;
-    }
+    udng[g] = udn;
   }
-  for (int a = 0; a < 3; a++) {
-    double* r = R + 4 * (size_t)id[a];
-    for (int i = 0; i < 3; i++) r[i] = r[i] + lR[i][a];
-    for (int b = 0; b < 3; b++) {
-      double* v = Val + 16 * (size_t)slot[(size_t)(3 * a + b) * nFePad + q];
-      v[0] = v[0] + lK[a][b];
-      v[5] = v[5] + lK[a][b];
-      v[10] = v[10] + lK[a][b];
+}
+
+// Lane t < nSlot: Val's block slot[t] gets the terms of its entries (9 q + 3 a
+// + b, in colour order); the others: node[k]'s rows of R those of (3 q + a).
+__global__ __launch_bounds__(64) void k_b_fluid(int nSlot, const int* __restrict__ slot, const int* __restrict__ sptr,
+                                                const int* __restrict__ sent, int nNode, const int* __restrict__ node,
+                                                const int* __restrict__ nptr, const int* __restrict__ nent,
+                                                const int4* __restrict__ ien, const double* __restrict__ x,
+                                                const double* __restrict__ hg, const double* __restrict__ Yg,
+                                                FaceConst C, double* __restrict__ R, double* __restrict__ Val)
+{
+#pragma clang fp contract(off)
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  double lR[3][3], wl, udn[3];
+  if (t < nSlot) {
+    double* v = Val + 16 * (size_t)slot[t];
+    double v0 = v[0], v1 = v[5], v2 = v[10];
+    for (int k = sptr[t]; k < sptr[t + 1]; k++) {
+      const int q = sent[k] / 9, ab = sent[k] - 9 * q, a = ab / 3, b = ab - 3 * a;
+      face_terms(ien[q], x, hg, Yg, C, lR, wl, udn);
+      double lK = 0.0;
+      for (int g = 0; g < 3; g++) lK = lK - wl * C.N[g][a] * C.N[g][b] * udn[g];
+      v0 = v0 + lK;
+      v1 = v1 + lK;
+      v2 = v2 + lK;
     }
+    v[0] = v0;
+    v[5] = v1;
+    v[10] = v2;
+  } else if (t - nSlot < nNode) {
+    const int k = t - nSlot;
+    double* r = R + 4 * (size_t)node[k];
+    double s0 = r[0], s1 = r[1], s2 = r[2];
+    for (int c = nptr[k]; c < nptr[k + 1]; c++) {
+      const int q = nent[c] / 3, a = nent[c] - 3 * q;
+      face_terms(ien[q], x, hg, Yg, C, lR, wl, udn);
+      s0 = s0 + (a == 0 ? lR[0][0] : a == 1 ? lR[0][1] : lR[0][2]);
+      s1 = s1 + (a == 0 ? lR[1][0] : a == 1 ? lR[1][1] : lR[1][2]);
+      s2 = s2 + (a == 0 ? lR[2][0] : a == 1 ? lR[2][1] : lR[2][2]);
+    }
+    r[0] = s0;
+    r[1] = s1;
+    r[2] = s2;
   }
 }
 
@@ -821,25 +856,51 @@ extern "C" int svg_face_create(const svg_msh* M, int nFe, const int* faceIEN, co
   auto* Fa = new svg_face();
   Fa->msh = M;
   Fa->nFe = nFe;
-  Fa->nColors = nColors;
-  Fa->colorOff = off;
-  Fa->nFePad = (nFe + 63) & ~63;
-  std::vector<int> ie((size_t)4 * nFe), sl((size_t)9 * Fa->nFePad, 0);
-  for (int q = 0; q < nFe; q++) {
-    const int e = order[q];
-    for (int a = 0; a < 4; a++) ie[4 * (size_t)q + a] = ien4[4 * (size_t)e + a];
-    for (int p = 0; p < 9; p++) sl[(size_t)p * Fa->nFePad + q] = slots[9 * (size_t)e + p];
+  std::vector<int> ie((size_t)4 * nFe);
+  for (int q = 0; q < nFe; q++)
+    for (int a = 0; a < 4; a++) ie[4 * (size_t)q + a] = ien4[4 * (size_t)order[q] + a];
+  // the entries of each block slot and of each node, in colour order
+  auto group = [&](int per, auto key, std::vector<int>& ids, std::vector<int>& ptr, std::vector<int>& ent) {
+    std::vector<std::pair<int, int>> kv((size_t)per * nFe);
+    for (int q = 0; q < nFe; q++)
+      for (int p = 0; p < per; p++) kv[(size_t)per * q + p] = {key(q, p), per * q + p};
+    std::sort(kv.begin(), kv.end());
+    for (size_t k = 0; k < kv.size(); k++) {
+      if (k == 0 || kv[k].first != kv[k - 1].first) {
+        ids.push_back(kv[k].first);
+        ptr.push_back((int)k);
+      }
+      ent.push_back(kv[k].second);
+    }
+    ptr.push_back((int)kv.size());
+  };
+  std::vector<int> sid, sptr, sent, nid, nptr, nent;
+  group(9, [&](int q, int p) { return slots[9 * (size_t)order[q] + p]; }, sid, sptr, sent);
+  group(3, [&](int q, int p) { return ie[4 * (size_t)q + p]; }, nid, nptr, nent);
+  Fa->nSlot = (int)sid.size();
+  Fa->nNode = (int)nid.size();
+  // one upload: the connectivity, then the two groups' lists
+  std::vector<int> all(ie);
+  int at[6], k = 0;
+  for (const auto* v : {&sid, &sptr, &sent, &nid, &nptr, &nent}) {
+    at[k++] = (int)all.size();
+    all.insert(all.end(), v->begin(), v->end());
   }
-  if ((rc = dev_alloc(&Fa->d_ien, ie.size())) || (rc = dev_alloc(&Fa->d_slot, sl.size()))) {
+  if ((rc = dev_alloc(&Fa->d_ien, all.size()))) {
     svg_face_free(Fa);
     return rc;
   }
-  hipError_t e = hipMemcpy(Fa->d_ien, ie.data(), sizeof(int) * ie.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(Fa->d_slot, sl.data(), sizeof(int) * sl.size(), hipMemcpyHostToDevice);
+  hipError_t e = hipMemcpy(Fa->d_ien, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     svg_face_free(Fa);
     return hip_check(e, "svg_face_create: upload");
   }
+  Fa->d_slot = Fa->d_ien + at[0];
+  Fa->d_sptr = Fa->d_ien + at[1];
+  Fa->d_sent = Fa->d_ien + at[2];
+  Fa->d_node = Fa->d_ien + at[3];
+  Fa->d_nptr = Fa->d_ien + at[4];
+  Fa->d_nent = Fa->d_ien + at[5];
   *out = Fa;
   return SVG_OK;
 }
@@ -848,7 +909,6 @@ extern "C" int svg_face_free(svg_face* Fa)
 {
   if (!Fa) return SVG_OK;
   dev_free(Fa->d_ien);
-  dev_free(Fa->d_slot);
   delete Fa;
   return SVG_OK;
 }
@@ -873,13 +933,9 @@ extern "C" int svg_b_assem_neu_bc(svg_face* Fa, const svg_fluid_params* p, doubl
     C.N[g][2] = 1.0 - xi[g][0] - xi[g][1];
   }
   const svg_msh* M = Fa->msh;
-  for (int c = 0; c < Fa->nColors; c++) {
-    const int q0 = Fa->colorOff[c], qn = Fa->colorOff[c + 1] - q0;
-    if (qn <= 0) continue;
-    launch("b_fluid", k_b_fluid_tri3, dim3(blocks_for(qn, 128)), dim3(128), 0, s, q0, qn,
-           reinterpret_cast<const int4*>(Fa->d_ien), (const int*)Fa->d_slot, Fa->nFePad, (const double*)M->d_x, hg, Yg,
-           C, R, Val);
-  }
+  launch("b_fluid", k_b_fluid, dim3(blocks_for((size_t)Fa->nSlot + Fa->nNode, 64)), dim3(64), 0, s, Fa->nSlot,
+         Fa->d_slot, Fa->d_sptr, Fa->d_sent, Fa->nNode, Fa->d_node, Fa->d_nptr, Fa->d_nent,
+         reinterpret_cast<const int4*>(Fa->d_ien), (const double*)M->d_x, hg, Yg, C, R, Val);
   SVG_HIP(hipGetLastError());
   return SVG_OK;
 }

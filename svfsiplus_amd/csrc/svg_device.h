@@ -328,12 +328,12 @@ namespace svg {
 int msh_gather_build(svg_msh* M, const int* d_IEN, hipStream_t s);
 }
 
-// A TRI3 Neumann face of a fluid mesh (faceType: IEN, gE), colour-sorted.
+// A TRI3 Neumann face of a fluid mesh (faceType: IEN, gE), colour-sorted. The
+// lists group the face elements' entries by block slot and by node.
 struct svg_face {
   const svg_msh* msh = nullptr;
-  int nFe = 0, nColors = 0;
-  std::vector<int> colorOff;
-  int* d_ien = nullptr;    // (4, nFe): the 3 face nodes and the parent element's interior node
-  int* d_slot = nullptr;   // 9 slots per face element, SoA: slot[p*nFePad + e]
-  int nFePad = 0;
+  int nFe = 0, nSlot = 0, nNode = 0;
+  int* d_ien = nullptr;    // (4, nFe): the 3 face nodes and the parent element's interior node; then the lists
+  const int *d_slot = nullptr, *d_sptr = nullptr, *d_sent = nullptr;  // slots; entries 9 q + 3 a + b per slot
+  const int *d_node = nullptr, *d_nptr = nullptr, *d_nent = nullptr;  // nodes; entries 3 q + a per node
 };
