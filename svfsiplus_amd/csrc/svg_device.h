@@ -64,12 +64,59 @@ __device__ __forceinline__ int xcd_block(int b, int nb)
   return r < nb ? r : -1;
 }
 
+// Lane l's partner value v[l ^ O] (O = 32, 16, 8, 4, 2, 1) by register moves
+// within the vector unit: half-wave and half-row swaps, then DPP. A shuffle
+// through the LDS crossbar takes about 130 cycles a level, these about 30.
+template <int O>
+__device__ __forceinline__ unsigned lane_xor(unsigned v)
+{
+  if constexpr (O == 32 || O == 16) {
+    // one result holds the partner's value for the low, the other for the high lanes
+    const bool high = (__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) & O) != 0;
+    if constexpr (O == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      return high ? r[0] : r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+      return high ? r[0] : r[1];
+    }
+  } else if constexpr (O == 8) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);  // row_ror:8
+  } else if constexpr (O == 4) {
+    const int up = __builtin_amdgcn_update_dpp(0, (int)v, 0x104, 0xF, 0x5, false);    // row_shl:4, lanes 0-3 and 8-11
+    return (unsigned)__builtin_amdgcn_update_dpp(up, (int)v, 0x114, 0xF, 0xA, false);  // row_shr:4, the others
+  } else {
+    constexpr int perm = O == 2 ? 0x4E : 0xB1;  // quad_perm [2,3,0,1], [1,0,3,2]
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, perm, 0xF, 0xF, false);
+  }
+}
+
+template <int O>
+__device__ __forceinline__ double lane_xor(double v)
+{
+  const unsigned long long u = __double_as_longlong(v);
+  const unsigned long long lo = lane_xor<O>((unsigned)u), hi = lane_xor<O>((unsigned)(u >> 32));
+  return __longlong_as_double((long long)(lo | (hi << 32)));
+}
+
+// Fixed butterfly over the 64 lanes of a wavefront (all of them active).
 __device__ __forceinline__ double wave_sum(double v)
 {
-  // Fixed butterfly over the 64 lanes of a wavefront.
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v += lane_xor<32>(v);
+  v += lane_xor<16>(v);
+  v += lane_xor<8>(v);
+  v += lane_xor<4>(v);
+  v += lane_xor<2>(v);
+  v += lane_xor<1>(v);
   return v;
+}
+
+// G sums at once (independent chains, which the scheduler interleaves).
+template <int G>
+__device__ __forceinline__ void wave_sums(double (&v)[G])
+{
+#pragma unroll
+  for (int q = 0; q < G; q++) v[q] = wave_sum(v[q]);
 }
 
 template <typename T>

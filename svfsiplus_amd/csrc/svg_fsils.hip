@@ -458,10 +458,7 @@ __device__ __forceinline__ void span_dots(const TWv* __restrict__ w, const T* __
         acc[q] = acc[q] + v * wr[r];
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-      for (int q = 0; q < G; q++) acc[q] += __shfl_xor(acc[q], o, 64);  // wave_sum's butterfly
+    wave_sums<G>(acc);
     if (lane == 0) {
 #pragma unroll
       for (int q = 0; q < G; q++) lds[wv * mc + j + q] = acc[q];
