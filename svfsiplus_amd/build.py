@@ -21,7 +21,7 @@ CSRC = PKG / "csrc"
 LIB = PKG / "libsvgpu.so"
 
 HIP_SOURCES = ["svg_runtime.hip", "svg_fsils.hip", "svg_assembly.hip", "svg_lpc.hip", "svg_setup.hip",
-               "svg_coarse.hip"]
+               "svg_coarse.hip", "svg_small.hip"]
 CPP_SOURCES = ["host_setup.cpp"]
 HOST_DIR = PKG / "host"
 HOST_SOURCES = ["svg_fsils.cpp"]            # C++ host API (into the library)

@@ -218,6 +218,10 @@ struct NsWork {
   double* h_dots = nullptr;
   double* partial = nullptr;
   int partialCap = 0;
+  // the Schur CG as one launch (cg_small): rows of a workgroup (0 not looked at, -1 does not fit), its most blocks
+  int smallRows = 0, smallCap = 0;
+  double* cgEx = nullptr;   // its exchanged vectors (8 nNo)
+  int* ctr = nullptr;       // its barrier
 };
 
 // Two-level (aggregation coarse level + block Jacobi) preconditioner of an lhs.
@@ -255,6 +259,7 @@ int coarse_num_aggregates(const svg_lhs* L);
 unsigned long long coarse_generation(const svg_lhs* L);  // changes when the level is rebuilt
 
 // Shared between the translation units.
+int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol, hipStream_t s, int* ran);
 void krylov_free(KrylovWork& k);   // every buffer, pinned mirror and event of a Krylov workspace
 int lhs_ensure_trans(svg_lhs* L);  // block-transpose map (pattern must be symmetric)
 int lpc_prepare_dev(svg_lhs* L, const double* Val, hipStream_t s);

@@ -1958,8 +1958,8 @@ static int gmres_dev(const Op& A, KrylovWork& k, svg_subls* ls, const double* R,
   return SVG_OK;
 }
 
-// cgrad::schur (cgrad.cpp:50-160) on P in place: P <- (L - D G)^-1 P.
-static int schur_dev(svg_lhs* L, svg_subls* ls, double* Pio, hipStream_t s)
+// The Schur CG as four launches an iteration; the result in w.cgX and w.h_cg.
+static int schur_launches(svg_lhs* L, const svg_subls* ls, double* Pio, hipStream_t s)
 {
   auto& w = L->ns;
   const bool coupled = has_coupled(L);
@@ -1967,8 +1967,6 @@ static int schur_dev(svg_lhs* L, svg_subls* ls, double* Pio, hipStream_t s)
   const int nb = (int)blocks_for(nNo, RED_SPAN);
   double* part1 = w.partial;
   double* part2 = w.partial + nb;
-  auto t0 = std::chrono::steady_clock::now();
-  ls->suc = 0;
   launch("cg_init", k_cg_init, dim3(nb), dim3(RED_BS), 0, s, nNo, (const double*)Pio, w.cgX, w.cgP, part1);
   launch("cg_start", k_cg_start, dim3(1), dim3(RED_BS), 0, s, (const double*)part1, nb, w.cg, ls->absTol,
          ls->relTol);
@@ -2001,8 +1999,28 @@ static int schur_dev(svg_lhs* L, svg_subls* ls, double* Pio, hipStream_t s)
   }
   SVG_HIP(hipGetLastError());
   SVG_HIP(hipMemcpyAsync(w.h_cg, w.cg, sizeof(CgState), hipMemcpyDeviceToHost, s));
-  SVG_HIP(hipMemcpyAsync(Pio, w.cgX, sizeof(double) * nNo, hipMemcpyDeviceToDevice, s));
   SVG_HIP(hipStreamSynchronize(s));
+  return SVG_OK;
+}
+
+// cgrad::schur (cgrad.cpp:50-160) on P in place: P <- (L - D G)^-1 P.
+static int schur_dev(svg_lhs* L, svg_subls* ls, double* Pio, hipStream_t s)
+{
+  auto& w = L->ns;
+  const bool coupled = has_coupled(L);
+  const int nNo = L->nNo;
+  auto t0 = std::chrono::steady_clock::now();
+  ls->suc = 0;
+  int ran = 0;
+  if (!coupled) {
+    int rc = cg_small(L, Pio, ls->mItr, ls->absTol, ls->relTol, s, &ran);
+    if (rc) return rc;
+  }
+  if (!ran) {
+    int rc = schur_launches(L, ls, Pio, s);
+    if (rc) return rc;
+  }
+  SVG_HIP(hipMemcpyAsync(Pio, w.cgX, sizeof(double) * nNo, hipMemcpyDeviceToDevice, s));
   const CgState& c = *w.h_cg;
   ls->iNorm = c.iNorm;
   ls->suc = c.suc;

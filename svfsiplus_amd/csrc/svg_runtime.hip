@@ -429,8 +429,9 @@ int svg_lhs_free(svg_lhs* L)
   }
   auto& w = L->ns;
   for (double* p : {w.mK, w.mG, w.mD, w.mL, w.Gt, w.Rm, w.Rmi, w.Rc, w.Rci, w.U, w.MU, w.P, w.MP, w.cgX, w.cgP,
-                    w.cgSP, w.cgGP, w.cgGP0, w.coef, w.dots, w.partial})
+                    w.cgSP, w.cgGP, w.cgGP0, w.coef, w.dots, w.partial, w.cgEx})
     if (p) (void)hipFree(p);
+  if (w.ctr) (void)hipFree(w.ctr);
   if (w.cg) (void)hipFree(w.cg);
   if (w.h_cg) (void)hipHostFree(w.h_cg);
   if (w.h_dots) (void)hipHostFree(w.h_dots);

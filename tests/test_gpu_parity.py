@@ -400,6 +400,29 @@ def test_coupled_ns_solver(torch_cuda):
     assert rel <= 1e-2
 
 
+@pytest.mark.parametrize("n,nz", [(2, 3), (4, 7), (12, 30), (16, 40)])
+def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz):
+    """The NS solver where its Schur CG runs as one launch: less than one
+    workgroup's rows, a ragged last one, 6 and 12 reduction spans (four are
+    summed at a time); bit for bit the device-order oracle, counts and all."""
+    from svfsiplus_amd.newton import DeviceLhs, fsils_solve
+    import ctypes as C
+    torch = torch_cuda
+    p = W.make_pipe(n, nz=nz)
+    Ag, Yg = _state(p, phys, seed=n)
+    R, V = oracle.construct_fluid(p, phys, Ag, Yg)
+    ols = oracle.ls_create(oracle.LS_NS, absTol=1e-30, maxItr=2)
+    ls = _lib.Ls()
+    C.memmove(C.byref(ls), C.byref(ols), C.sizeof(ls))
+    dR, dV = _dev(torch, R), _dev(torch, V)
+    fsils_solve(DeviceLhs(p), ls, 4, dR, dV)
+    with oracle.device_order():
+        x0, _, ols = oracle.fsils_solve(p, ols, R, V)
+    assert (ls.RI.itr, ls.GM.itr, ls.CG.itr, ls.CG.suc) == (ols.RI.itr, ols.GM.itr, ols.CG.itr, ols.CG.suc)
+    assert (ls.RI.fNorm, ls.CG.fNorm, ls.CG.iNorm) == (ols.RI.fNorm, ols.CG.fNorm, ols.CG.iNorm)
+    assert np.array_equal(dR.cpu().numpy(), x0)
+
+
 @pytest.mark.parametrize("name", ["pipe_n2", "pipe_n4"])
 def test_ns_solver_against_reference_golden(torch_cuda, name):
     """Bipartitioned NS solver (ns_solver.cpp) on the device against the reference's record."""
