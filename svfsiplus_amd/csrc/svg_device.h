@@ -200,6 +200,11 @@ struct KrylovWork {
   float* w32 = nullptr;       // mixed precision, two-level preconditioner: the FP32 SpMV's output A z_i
   double* r2 = nullptr;       // two-level with the network as smoother: its input B (u - A P zc)
   double* scal = nullptr;     // scratch scalars for standalone dots
+  // restart cycles in one launch (gmres_small): most blocks of a workgroup (0 not looked at, -1 does not
+  // fit) and most columns they touch
+  int smallCap = 0, smallCapU = 0;
+  double* small = nullptr;    // its partial sums, exchanged vectors and solution coefficients
+  int* ctr = nullptr;         // its barrier
 };
 
 // Workspace of the bipartitioned NS solver (ns_solver.cpp:167-499).
@@ -259,6 +264,8 @@ int coarse_num_aggregates(const svg_lhs* L);
 unsigned long long coarse_generation(const svg_lhs* L);  // changes when the level is rebuilt
 
 // Shared between the translation units.
+bool gmres_small_fits(svg_lhs* L, int sD);
+int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double* R, hipStream_t s, int* ran);
 int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol, hipStream_t s, int* ran);
 void krylov_free(KrylovWork& k);   // every buffer, pinned mirror and event of a Krylov workspace
 int lhs_ensure_trans(svg_lhs* L);  // block-transpose map (pattern must be symmetric)

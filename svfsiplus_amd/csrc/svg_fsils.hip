@@ -1292,6 +1292,9 @@ void krylov_free(KrylovWork& k)
   dev_free(k.z32);
   dev_free(k.w32);
   dev_free(k.r2);
+  dev_free(k.small);
+  dev_free(k.ctr);
+  k.smallCap = 0;
   if (k.h_st) (void)hipHostFree(k.h_st);
   k.h_st = nullptr;
   if (k.h_done) {
@@ -1675,7 +1678,9 @@ static int gmres_v_dev(svg_lhs* L, svg_subls* ls, int dof, const double* Val, do
   if (rc) return rc;
   const int n = k.n, sD = ls->sD;
   const Op A{L, Val, 4};
-  if (L->spmvVariant < 0 && (rc = svg_spmv_tune(L, Val, nullptr, s))) return rc;
+  // a small system's cycles run in one launch each few of them, with no SpMV launch to tune
+  const bool small = !has_coupled(L) && gmres_small_fits(L, sD);
+  if (!small && L->spmvVariant < 0 && (rc = svg_spmv_tune(L, Val, nullptr, s))) return rc;
   auto t0 = std::chrono::steady_clock::now();
   FinArgs fa{};
   fa.sD = sD;
@@ -1698,7 +1703,22 @@ static int gmres_v_dev(svg_lhs* L, svg_subls* ls, int dof, const double* Val, do
   svg_fill(k.X, (size_t)n, 0.0, s);
   const unsigned nbv = blocks_for(n, 256);
   double dB = ls->fNorm;
-  for (int l = 0; l < ls->mItr; l++) {
+  int ran = 0;
+  if (small && ls->mItr > 0) {
+    if ((rc = gmres_small(L, ls, Val, R, s, &ran))) return rc;
+    if (ran) {
+      if (k.h_st->divzero) return set_error(SVG_ERR_ARG, "Array Divide by zero.");
+      dB = k.h_st->fStart;
+      ls->itr = k.h_st->itr;
+      ls->fNorm = k.h_st->fNorm;
+      ls->suc = k.h_st->suc;
+    } else {
+      // from the start again, launch by launch
+      svg_fill(k.X, (size_t)n, 0.0, s);
+      if ((rc = dot_device(n, R, R, 0, 1, k.partial, k.scal, k.st, fa, k.h, k.cs, k.sn, k.err, k.coef, s))) return rc;
+    }
+  }
+  for (int l = 0; !ran && l < ls->mItr; l++) {
     dB = ls->fNorm;
     *k.h_done = 0;
     op_apply(A, k.X, k.u, R, nullptr, s);  // u0 = R - A X

@@ -61,6 +61,13 @@ __device__ __forceinline__ bool grid_sync(int* ctr, int& target, int* ok)
   return *ok != 0;
 }
 
+// Orders a wavefront's LDS accesses across its lanes.
+__device__ __forceinline__ void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Sum over n entries in the order of the per-launch reductions: spans of 1024,
 // lane t of 256 adds its entries t, t + 256, .. of the span in order, butterflies,
 // the four wavefront sums in order, then the spans (lane b, b + 64, .. in order
@@ -309,6 +316,353 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
   }
 }
 
+// ----------------------------------------------------------- GMRES ---------
+// gmres_v's restart cycles (gmres.cpp:529-612) on the 4x4 system, as run_cycle
+// enqueues them: residual, Arnoldi steps, back substitution and X, up to
+// `cycles` restarts in a launch. Workgroup 4 b + s owns, of the reduction span
+// b (1024 entries), the entries 256 r + 64 s + l (r < 4, l < 64): one
+// wavefront's share of the span's sums, so a step's dots follow its product
+// without a barrier between them. Its blocks of the matrix and the list of the
+// columns they touch stay in LDS; its part of the Krylov basis is read by no
+// other workgroup and stays in the caches. Two barriers a step:
+//   1  u_i of the listed columns (exchanged), w = A u_i, the share's dots with
+//      u_0 .. u_i and w                                   -> part
+//   2  every workgroup finishes the dots, the norm and the coefficients itself;
+//      u_{i+1}                                            -> ex (double buffered)
+// the Givens rotations and the stop test run beside the update. On the 15k-tet
+// pipe (52 workgroups) a step takes 16 us, as four launches 35 us.
+constexpr int GM_BS = 256, GM_MAX = 256;
+constexpr int GM_BLK_B = 16 * 8 + 2, GM_COL_B = 4 + 32;  // LDS bytes per block and per listed column
+
+struct GmSmall {
+  int nNo, sD, cap, capU, cycles;
+  const int *rowPtr, *colPtr;
+  const double *K, *R;
+  double *X, *u, *ex, *part, *h, *y;
+  size_t ld;
+  GmState* st;
+  int* ctr;
+};
+
+__global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
+{
+#pragma clang fp contract(off)
+  extern __shared__ double lds[];
+  __shared__ double sh[4][GM_MAX];  // sums, h column, cosines, sines; the set-up's bitmap first
+  __shared__ double wl[4][64];      // the workgroup's entries of w, [r][l]
+  __shared__ double sc[4];          // scale, err_i, err_{i+1}
+  __shared__ int okf, stopf, wsum[4];
+  double *sums = sh[0], *lh = sh[1], *lcs = sh[2], *lsn = sh[3];
+  unsigned *bits = reinterpret_cast<unsigned*>(sh[0]), *before = reinterpret_cast<unsigned*>(sh[1]);  // 512 words each
+  double* val = lds;                                                     // [capU][4]
+  double* K = lds + 4 * (size_t)A.capU;                                  // [cap][16]
+  int* list = reinterpret_cast<int*>(K + 16 * (size_t)A.cap);            // [capU]
+  unsigned short* loc = reinterpret_cast<unsigned short*>(list + A.capU);  // [cap]
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int b = blockIdx.x >> 2, s = blockIdx.x & 3, n = 4 * A.nNo, nblk = (n + 1023) >> 10;
+  const int k = 1024 * b + 256 * wv + 64 * s + lane;  // this lane's entry, r = its wavefront
+  const bool own = k < n;
+  const int row = min(k >> 2, A.nNo - 1), ci = k & 3;
+  // the rows of share r: 16 from first(r)
+  auto first = [&](int r) { return min(A.nNo, 256 * b + 64 * r + 16 * s); };
+  int off = 0, j0 = 0;  // this wavefront's blocks in LDS and in the matrix
+  for (int r = 0; r <= wv; r++) {
+    j0 = A.rowPtr[first(r)];
+    if (r < wv) off += A.rowPtr[min(A.nNo, first(r) + 16)] - j0;
+  }
+  const int nb = A.rowPtr[min(A.nNo, first(wv) + 16)] - j0;
+  for (int q = t; q < 512; q += GM_BS) bits[q] = 0;
+  __syncthreads();
+  for (int q = lane; q < 8 * nb; q += 64)
+    reinterpret_cast<double2*>(K + 16 * (size_t)off)[q] = reinterpret_cast<const double2*>(A.K + 16 * (size_t)j0)[q];
+  for (int q = lane; q < nb; q += 64) {
+    const int c = A.colPtr[j0 + q];
+    atomicOr(&bits[c >> 5], 1u << (c & 31));
+  }
+  __syncthreads();
+  {
+    int n2[2], m = 0;
+#pragma unroll
+    for (int q = 0; q < 2; q++) n2[q] = __popc(bits[2 * t + q]), m += n2[q];
+    int inc = m;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += v;
+    }
+    if (lane == 63) wsum[wv] = inc;
+    __syncthreads();
+    int at = inc - m;
+    for (int q = 0; q < wv; q++) at += wsum[q];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      before[2 * t + q] = at;
+      for (unsigned w = bits[2 * t + q], e = at; w; w &= w - 1, e++) list[e] = 32 * (2 * t + q) + __builtin_ctz(w);
+      at += n2[q];
+    }
+  }
+  __syncthreads();
+  const int nu = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+  for (int q = lane; q < nb; q += 64) {
+    const int c = A.colPtr[j0 + q];
+    loc[off + q] = (unsigned short)(before[c >> 5] + __popc(bits[c >> 5] & ((1u << (c & 31)) - 1u)));
+  }
+  const int ja = own ? A.rowPtr[row] - j0 + off : 0, jb = own ? A.rowPtr[row + 1] - j0 + off : 0;
+  __syncthreads();
+
+  const AgentBuf bex0(A.ex, sizeof(double) * n), bex1(A.ex + n, sizeof(double) * n);
+  const AgentBuf bpart(A.part, sizeof(double) * 4 * nblk * (A.sD + 1));
+  // A v for the exchanged vector v of buffer p: this lane's entry
+  auto product = [&](int p) {
+    for (int q = t; q < 2 * nu; q += GM_BS) {
+      const int byte = 32 * list[q >> 1] + 16 * (q & 1);
+      reinterpret_cast<double2*>(val)[q] = p ? bex1.ld2(byte) : bex0.ld2(byte);
+    }
+    __syncthreads();
+    double acc = 0.0;
+#pragma unroll 4
+    for (int j = ja; j < jb; j++) {
+      const double2* kp = reinterpret_cast<const double2*>(K + 16 * (size_t)j + 4 * ci);
+      const double2* up = reinterpret_cast<const double2*>(val + 4 * (size_t)loc[j]);
+      const double2 k0 = kp[0], k1 = kp[1], u0 = up[0], u1 = up[1];
+      double x = acc + k0.x * u0.x;
+      x = x + k0.y * u0.y;
+      x = x + k1.x * u1.x;
+      acc = x + k1.y * u1.y;
+    }
+    return acc;
+  };
+  // the share's sums of column j over its wavefront's lanes -> part
+  auto put_part = [&](int j, double v) {
+    if (lane == 0) st_agent(A.part + (size_t)4 * nblk * j + 4 * b + s, v);
+  };
+  // the finished sum of column j: lane b adds the span's four shares in order
+  auto finish = [&](const double2& x, const double2& y) {
+    double v = x.x;
+    v = v + x.y;
+    v = v + y.x;
+    v = v + y.y;
+    return wave_sum(lane < nblk ? v : 0.0);
+  };
+  const double eps = A.st->eps;
+  int itr = A.st->itr, suc = 0, divzero = 0, last_i = 0, target = 0, cyc = 0;
+  double fNorm = A.st->fNorm, fPrev = fNorm;
+  const double rhs = own ? A.R[k] : 0.0;
+  double x = own ? A.X[k] : 0.0;
+  bool ok = true;
+  for (; cyc < A.cycles; cyc++) {
+    fPrev = fNorm;
+    // u_0 = (R - A X) / |R - A X|
+    if (own) st_agent(A.ex + k, x);
+    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    double v = rhs - product(0);
+    wl[wv][lane] = own ? v : 0.0;
+    __syncthreads();
+    if (wv == 0) {
+      double a = 0.0;
+#pragma unroll
+      for (int r = 0; r < 4; r++) a = a + wl[r][lane] * wl[r][lane];
+      put_part(0, wave_sum(a));
+    }
+    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    {
+      const int c = 32 * min(lane, nblk - 1);
+      const double e0 = sqrt(finish(bpart.ld2(c), bpart.ld2(c + 16)));
+      itr++;
+      if (e0 == 0.0) {
+        divzero = 1;
+        break;
+      }
+      v = v / e0;
+      if (t == 0) sc[1] = e0;
+    }
+    if (own) {
+      A.u[k] = v;
+      st_agent(A.ex + n + k, v);
+    }
+    if (t == 0) stopf = 0;
+    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    int i = 0;
+    for (;; i++) {
+      const double w = product((i & 1) ^ 1);
+      wl[wv][lane] = own ? w : 0.0;
+      __syncthreads();
+      {
+        // columns wv, wv + 4, .. of u_0 .. u_i, w: the four shares' entries in order
+        double wr[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) wr[r] = wl[r][lane];
+        const int kb = 1024 * b + 64 * s + lane;
+        for (int c = wv; c <= i; c += 16) {
+          double ub[4][4], a[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              ub[q][r] = A.u[(size_t)min(c + 4 * q, i) * A.ld + min(kb + 256 * r, n - 1)];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            a[q] = 0.0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) a[q] = a[q] + (kb + 256 * r < n ? ub[q][r] : 0.0) * wr[r];
+          }
+          wave_sums<4>(a);
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            if (c + 4 * q <= i) put_part(c + 4 * q, a[q]);
+        }
+        if (((i + 1) & 3) == wv) {
+          double a = 0.0;
+#pragma unroll
+          for (int r = 0; r < 4; r++) a = a + wr[r] * wr[r];
+          put_part(i + 1, wave_sum(a));
+        }
+      }
+      if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+      for (int c = wv; c <= i + 1; c += 16) {
+        double2 p0[4], p1[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int byte = 8 * (4 * nblk * min(c + 4 * q, i + 1) + 4 * min(lane, nblk - 1));
+          p0[q] = bpart.ld2(byte);
+          p1[q] = bpart.ld2(byte + 16);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const double f = finish(p0[q], p1[q]);
+          if (lane == 0 && c + 4 * q <= i + 1) sums[c + 4 * q] = f;
+        }
+      }
+      __syncthreads();
+      if (t < 64) {
+        // h(i+1, i) by the Pythagorean norm, 1 / h(i+1, i) (gmres.cpp:556-566)
+        double hh = sums[i + 1];
+#pragma unroll 8
+        for (int j = 0; j <= i; j++) hh = hh - sums[j] * sums[j];
+        hh = sqrt(fabs(hh));
+        if (t == 0) {
+          lh[i + 1] = hh;
+          sc[0] = 1.0 / hh;
+        }
+      }
+      __syncthreads();
+      if (wv == 3) {
+        // Givens rotations and the stop test (gmres.cpp:568-592), beside the update
+        if (lane == 0) {
+          const double hh = lh[i + 1];
+          double cur = sums[0];
+          for (int j = 0; j < i; j++) {
+            const double nx = sums[j + 1];
+            const double tmp = lcs[j] * cur + lsn[j] * nx;
+            cur = -lsn[j] * cur + lcs[j] * nx;
+            lh[j] = tmp;
+          }
+          const double tmp = sqrt(cur * cur + hh * hh);
+          const double c = cur / tmp, sv = hh / tmp;
+          lcs[i] = c;
+          lsn[i] = sv;
+          lh[i] = tmp;
+          const double ei = sc[1], e1 = -sv * ei;
+          sc[1] = e1;
+          sc[2] = c * ei;
+          stopf = fabs(e1) < eps ? 1 : 0;
+        }
+      }
+      {
+        double z = w;
+        for (int jq = 0; jq <= i; jq += 8) {
+          double q8[8];
+#pragma unroll
+          for (int q = 0; q < 8; q++) q8[q] = A.u[(size_t)min(jq + q, i) * A.ld + min(k, n - 1)];
+#pragma unroll
+          for (int q = 0; q < 8; q++)
+            if (jq + q <= i) z = z + (-sums[jq + q]) * q8[q];
+        }
+        z = sc[0] * z;
+        if (own) {
+          if (i + 1 < A.sD) A.u[(size_t)(i + 1) * A.ld + k] = z;
+          st_agent(A.ex + (size_t)(i & 1) * n + k, z);
+        }
+      }
+      ok = grid_sync(A.ctr, target, &okf);
+      itr++;
+      if (blockIdx.x == 0) {
+        // column i of the triangle and err(i), for the back substitution
+        for (int j = t; j <= i; j += GM_BS) A.h[(size_t)(A.sD + 1) * i + j] = lh[j];
+        if (t == 0) {
+          A.y[i] = sc[2];
+          A.y[i + 1] = sc[1];
+        }
+      }
+      if (!ok || stopf || i + 1 == A.sD) break;
+    }
+    if (!ok) break;
+    last_i = i;
+    suc = stopf;
+    fNorm = fabs(sc[1]);
+    __syncthreads();
+    // back substitution (gmres.cpp:595-608) by workgroup 0: a row's products by a
+    // wavefront (the next row's entries loaded ahead), their sum in order
+    double *y = lcs, *pr = lsn;
+    if (blockIdx.x == 0 && wv == 0) {
+      auto tri = [&](int j, int c) { return A.h[(size_t)(A.sD + 1) * min(c, last_i) + j]; };
+      double h0 = tri(last_i, lane), h1 = tri(last_i, lane + 64), h2 = tri(last_i, lane + 128),
+             h3 = tri(last_i, lane + 192);
+      for (int j = lane; j <= last_i; j += 64) y[j] = A.y[j];
+      wave_sync();
+      for (int j = last_i; j >= 0; j--) {
+        auto put = [&](int c, double hv) {
+          if (c >= j && c <= last_i) pr[c] = c > j ? hv * y[c] : hv;
+        };
+        put(lane, h0);
+        put(lane + 64, h1);
+        put(lane + 128, h2);
+        put(lane + 192, h3);
+        const int nx = max(j - 1, 0);
+        h0 = tri(nx, lane);
+        if (last_i >= 64) h1 = tri(nx, lane + 64), h2 = tri(nx, lane + 128), h3 = tri(nx, lane + 192);
+        wave_sync();
+        double a = y[j];
+#pragma unroll 8
+        for (int c = j + 1; c <= last_i; c++) a = a - pr[c];
+        a = a / pr[j];
+        wave_sync();
+        if (lane == 0) y[j] = a;
+        wave_sync();
+      }
+      for (int j = lane; j <= last_i; j += 64) st_agent(A.y + GM_MAX + j, y[j]);
+    }
+    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    for (int j = t; j <= last_i; j += GM_BS) sums[j] = ld_agent(A.y + GM_MAX + j);
+    __syncthreads();
+    for (int jq = 0; jq <= last_i; jq += 8) {
+      double q8[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) q8[q] = A.u[(size_t)min(jq + q, last_i) * A.ld + min(k, n - 1)];
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (jq + q <= last_i) x = x + sums[jq + q] * q8[q];
+    }
+    __syncthreads();
+    if (suc) {
+      cyc++;
+      break;
+    }
+  }
+  if (own) A.X[k] = x;
+  if (t == 0) {
+    if (!ok) __hip_atomic_store(&A.st->pad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (blockIdx.x == 0) {
+      A.st->itr = itr;
+      A.st->suc = suc;
+      A.st->divzero = divzero;
+      A.st->last_i = last_i;
+      A.st->cyc = cyc;
+      A.st->fNorm = fNorm;
+      A.st->fStart = fPrev;
+    }
+  }
+}
+
 int num_cus(int* n)
 {
   int dev = 0;
@@ -383,6 +737,93 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
   SVG_HIP(hipMemcpyAsync(w.h_cg, w.cg, sizeof(CgState), hipMemcpyDeviceToHost, s));
   SVG_HIP(hipStreamSynchronize(s));
   *ran = w.h_cg->pad ? 0 : 1;
+  return SVG_OK;
+}
+
+// Restart cycles of gmres_v for the system (Val, R) with X = 0 in L->kw.X and
+// the initial state in L->kw.st, in launches of up to GM_CYCLES cycles: *ran = 0
+// when the system does not fit (a workgroup per compute unit, its blocks in LDS)
+// or the workgroups did not meet, else the state after the last cycle is in
+// L->kw.h_st, fStart the residual norm before it (synchronises).
+constexpr int GM_CYCLES = 16;
+constexpr int GM_LDS = 149 * 1024;  // of 160 KB, 10 KB are the kernel's own arrays
+
+bool gmres_small_fits(svg_lhs* L, int sD)
+{
+  auto& k = L->kw;
+  if (k.smallCap == 0) {
+    k.smallCap = -1;
+    const int nNo = L->nNo, nblk = (4 * nNo + 1023) / 1024;
+    int cus = 0, cap = 0, capU = 0;
+    if (num_cus(&cus) != SVG_OK || 4 * nblk > cus || nblk > 64) return false;
+    std::vector<int> seen(nNo, -1);
+    for (int w = 0; w < 4 * nblk; w++) {
+      int nb = 0, nu = 0;
+      for (int r = 0; r < 4; r++) {
+        const int a = std::min(nNo, 256 * (w / 4) + 64 * r + 16 * (w % 4)), e = std::min(nNo, a + 16);
+        nb += L->rowPtr[e] - L->rowPtr[a];
+        for (int j = L->rowPtr[a]; j < L->rowPtr[e]; j++)
+          if (seen[L->colPtr[j]] != w) seen[L->colPtr[j]] = w, nu++;
+      }
+      cap = std::max(cap, nb);
+      capU = std::max(capU, nu);
+    }
+    if ((size_t)GM_BLK_B * cap + (size_t)GM_COL_B * capU > GM_LDS) return false;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gmres_small), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            GM_LDS) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    k.smallCap = cap;
+    k.smallCapU = capU;
+  }
+  return k.smallCap > 0 && sD < GM_MAX - 1;
+}
+
+int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double* R, hipStream_t s, int* ran)
+{
+  auto& k = L->kw;
+  *ran = 0;
+  const int n = k.n, nblk = (n + 1023) / 1024;
+  const size_t nPart = (size_t)4 * nblk * (k.sD + 1);
+  int rc;
+  if (!k.small && (rc = dev_alloc(&k.small, nPart + 2 * (size_t)n + 2 * GM_MAX))) return rc;
+  if (!k.ctr && (rc = dev_alloc(&k.ctr, 1))) return rc;
+  GmSmall A{};
+  A.nNo = L->nNo;
+  A.sD = ls->sD;
+  A.cap = k.smallCap;
+  A.capU = k.smallCapU;
+  A.rowPtr = L->d_rowPtr;
+  A.colPtr = L->d_colPtr;
+  A.K = Val;
+  A.R = R;
+  A.X = k.X;
+  A.u = k.u;
+  A.part = k.small;
+  A.ex = k.small + nPart;
+  A.y = A.ex + 2 * (size_t)n;
+  A.h = k.h;
+  A.ld = k.ld;
+  A.st = k.st;
+  A.ctr = k.ctr;
+  const unsigned bytes = (unsigned)(GM_BLK_B * A.cap + GM_COL_B * A.capU);
+  for (int done = 0; done < ls->mItr;) {
+    A.cycles = std::min(GM_CYCLES, ls->mItr - done);
+    hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, k.ctr, &k.st->pad);
+    void* args[] = {&A};
+    if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_gmres_small), dim3(4 * nblk), dim3(GM_BS), args,
+                                   bytes, s) != hipSuccess) {
+      (void)hipGetLastError();  // not launched: the per-launch path
+      return SVG_OK;
+    }
+    SVG_HIP(hipMemcpyAsync(k.h_st, k.st, sizeof(GmState), hipMemcpyDeviceToHost, s));
+    SVG_HIP(hipStreamSynchronize(s));
+    if (k.h_st->pad) return SVG_OK;
+    done += A.cycles;
+    if (k.h_st->suc || k.h_st->divzero) break;
+  }
+  *ran = 1;
   return SVG_OK;
 }
 

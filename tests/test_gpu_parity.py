@@ -226,6 +226,33 @@ def test_gmres_solve(torch_cuda, phys, n):
     assert rel <= 10 * tol
 
 
+@pytest.mark.parametrize("n,nz,sD,cycles", [(2, 3, 50, 1000), (4, 9, 1, 40), (4, 20, 250, 1000), (6, 11, 100, 3),
+                                            (10, 24, 50, 1000), (12, 61, 50, 20)])
+def test_gmres_one_launch_cycles(torch_cuda, phys, n, nz, sD, cycles):
+    """gmres_v where a launch runs whole restart cycles: one workgroup group to 41
+    of them, Krylov dimensions 1 to 250 (the back substitution's rows take 64
+    columns a load), more restarts than one launch runs, stops before and at the
+    limit: bit for bit the device-order oracle."""
+    from svfsiplus_amd.newton import DeviceLhs, fsils_solve, ls_create
+    torch = torch_cuda
+    p = W.make_pipe(n, nz=nz)
+    Ag, Yg = _state(p, phys, seed=n)
+    R, V = oracle.construct_fluid(p, phys, Ag, Yg)
+    with oracle.device_order():
+        x0, _, ols = oracle.fsils_solve(
+            p, oracle.ls_create(oracle.LS_GMRES, relTol=1e-6, absTol=1e-30, maxItr=cycles, dimKry=sD), R, V)
+    ls = ls_create(_lib.LS_GMRES, relTol=1e-6, absTol=1e-30, maxItr=cycles, dimKry=sD)
+    dR, dV = _dev(torch, R), _dev(torch, V)
+    L = DeviceLhs(p)
+    for _ in range(2):  # the second solve finds the workspaces of the first
+        dR.copy_(torch.from_numpy(R))
+        dV.copy_(torch.from_numpy(V))
+        fsils_solve(L, ls, 4, dR, dV)
+        assert (ls.RI.itr, ls.RI.suc, ls.RI.iNorm, ls.RI.fNorm) == (ols.RI.itr, ols.RI.suc, ols.RI.iNorm, ols.RI.fNorm)
+        assert abs(ls.RI.dB - ols.RI.dB) <= 1e-12 * abs(ols.RI.dB)
+        assert np.array_equal(dR.cpu().numpy(), x0)
+
+
 def test_newton_time_step(torch_cuda, phys):
     """Three Newton iterations (pici, construct_fluid, fsils_solve, picc) against the oracle:
     identical linear iteration counts and residual norms to the device-order oracle (assembly
