@@ -329,9 +329,13 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
 //      u_0 .. u_i and w                                   -> part
 //   2  every workgroup finishes the dots, the norm and the coefficients itself;
 //      u_{i+1}                                            -> ex (double buffered)
-// the Givens rotations and the stop test run beside the update. On the 15k-tet
-// pipe (52 workgroups) a step takes 16 us, as four launches 35 us.
-constexpr int GM_BS = 256, GM_MAX = 256;
+// the Givens rotations and the stop test run beside the update, on a wavefront
+// of their own, and the first GM_PF columns of the basis are on their way while
+// the product is formed (for the dots) and over barrier 1 (for the update): 24
+// is what the registers hold, 28 spill. On the 15k-tet pipe (52 workgroups) a
+// step takes 15.3 us; 16 without either, 35 as four launches.
+constexpr int GM_BS = 320, GM_MAX = 256;  // four wavefronts of entries, one for the rotations
+constexpr int GM_PF = 24;
 constexpr int GM_BLK_B = 16 * 8 + 2, GM_COL_B = 4 + 32;  // LDS bytes per block and per listed column
 
 struct GmSmall {
@@ -358,19 +362,19 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
   double* K = lds + 4 * (size_t)A.capU;                                  // [cap][16]
   int* list = reinterpret_cast<int*>(K + 16 * (size_t)A.cap);            // [capU]
   unsigned short* loc = reinterpret_cast<unsigned short*>(list + A.capU);  // [cap]
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int b = blockIdx.x >> 2, s = blockIdx.x & 3, n = 4 * A.nNo, nblk = (n + 1023) >> 10;
   const int k = 1024 * b + 256 * wv + 64 * s + lane;  // this lane's entry, r = its wavefront
-  const bool own = k < n;
+  const bool own = wv < 4 && k < n;
   const int row = min(k >> 2, A.nNo - 1), ci = k & 3;
   // the rows of share r: 16 from first(r)
   auto first = [&](int r) { return min(A.nNo, 256 * b + 64 * r + 16 * s); };
   int off = 0, j0 = 0;  // this wavefront's blocks in LDS and in the matrix
-  for (int r = 0; r <= wv; r++) {
+  for (int r = 0; r <= wv && r < 4; r++) {
     j0 = A.rowPtr[first(r)];
     if (r < wv) off += A.rowPtr[min(A.nNo, first(r) + 16)] - j0;
   }
-  const int nb = A.rowPtr[min(A.nNo, first(wv) + 16)] - j0;
+  const int nb = wv < 4 ? A.rowPtr[min(A.nNo, first(wv) + 16)] - j0 : 0;
   for (int q = t; q < 512; q += GM_BS) bits[q] = 0;
   __syncthreads();
   for (int q = lane; q < 8 * nb; q += 64)
@@ -383,18 +387,18 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
   {
     int n2[2], m = 0;
 #pragma unroll
-    for (int q = 0; q < 2; q++) n2[q] = __popc(bits[2 * t + q]), m += n2[q];
+    for (int q = 0; q < 2; q++) n2[q] = wv < 4 ? __popc(bits[2 * t + q]) : 0, m += n2[q];
     int inc = m;
     for (int o = 1; o < 64; o <<= 1) {
       const int v = __shfl_up(inc, o, 64);
       if (lane >= o) inc += v;
     }
-    if (lane == 63) wsum[wv] = inc;
+    if (lane == 63 && wv < 4) wsum[wv] = inc;
     __syncthreads();
     int at = inc - m;
     for (int q = 0; q < wv; q++) at += wsum[q];
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
+    for (int q = 0; q < 2 && wv < 4; q++) {
       before[2 * t + q] = at;
       for (unsigned w = bits[2 * t + q], e = at; w; w &= w - 1, e++) list[e] = 32 * (2 * t + q) + __builtin_ctz(w);
       at += n2[q];
@@ -455,7 +459,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
     if (own) st_agent(A.ex + k, x);
     if (!(ok = grid_sync(A.ctr, target, &okf))) break;
     double v = rhs - product(0);
-    wl[wv][lane] = own ? v : 0.0;
+    if (wv < 4) wl[wv][lane] = own ? v : 0.0;
     __syncthreads();
     if (wv == 0) {
       double a = 0.0;
@@ -483,42 +487,57 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
     if (!(ok = grid_sync(A.ctr, target, &okf))) break;
     int i = 0;
     for (;; i++) {
+      // the share's entries of u_0 .. u_i for the dots, column wv + 4 q, on their
+      // way while the product is formed
+      const int kb = 1024 * b + 64 * s + lane;
+      double pu[GM_PF / 4][4];
+#pragma unroll
+      for (int q = 0; q < GM_PF / 4; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          pu[q][r] = 0.0;
+          if (wv < 4 && wv + 4 * q <= i) pu[q][r] = A.u[(size_t)(wv + 4 * q) * A.ld + min(kb + 256 * r, n - 1)];
+        }
       const double w = product((i & 1) ^ 1);
-      wl[wv][lane] = own ? w : 0.0;
+      if (wv < 4) wl[wv][lane] = own ? w : 0.0;
       __syncthreads();
-      {
-        // columns wv, wv + 4, .. of u_0 .. u_i, w: the four shares' entries in order
+      if (wv < 4) {
         double wr[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) wr[r] = wl[r][lane];
-        const int kb = 1024 * b + 64 * s + lane;
-        for (int c = wv; c <= i; c += 16) {
-          double ub[4][4], a[4];
+        // one column: the four spans' rows in order, then the butterfly
+        auto dot = [&](double u0, double u1, double u2, double u3) {
+          double a = 0.0 + (kb < n ? u0 : 0.0) * wr[0];
+          a = a + (kb + 256 < n ? u1 : 0.0) * wr[1];
+          a = a + (kb + 512 < n ? u2 : 0.0) * wr[2];
+          a = a + (kb + 768 < n ? u3 : 0.0) * wr[3];
+          return wave_sum(a);
+        };
+#pragma unroll
+        for (int q = 0; q < GM_PF / 4; q++)
+          if (wv + 4 * q <= i) put_part(wv + 4 * q, dot(pu[q][0], pu[q][1], pu[q][2], pu[q][3]));
+        for (int c = GM_PF + wv; c <= i; c += 16) {
+          double ub[4][4];
 #pragma unroll
           for (int q = 0; q < 4; q++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
               ub[q][r] = A.u[(size_t)min(c + 4 * q, i) * A.ld + min(kb + 256 * r, n - 1)];
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            a[q] = 0.0;
-#pragma unroll
-            for (int r = 0; r < 4; r++) a[q] = a[q] + (kb + 256 * r < n ? ub[q][r] : 0.0) * wr[r];
-          }
-          wave_sums<4>(a);
-#pragma unroll
           for (int q = 0; q < 4; q++)
-            if (c + 4 * q <= i) put_part(c + 4 * q, a[q]);
+            if (c + 4 * q <= i) put_part(c + 4 * q, dot(ub[q][0], ub[q][1], ub[q][2], ub[q][3]));
         }
-        if (((i + 1) & 3) == wv) {
-          double a = 0.0;
+        if (((i + 1) & 3) == wv) put_part(i + 1, dot(wr[0], wr[1], wr[2], wr[3]));
+      }
+      // this lane's entries for the update, on their way over the barrier
+      double pv[GM_PF];
 #pragma unroll
-          for (int r = 0; r < 4; r++) a = a + wr[r] * wr[r];
-          put_part(i + 1, wave_sum(a));
-        }
+      for (int q = 0; q < GM_PF; q++) {
+        pv[q] = 0.0;
+        if (wv < 4 && q <= i) pv[q] = A.u[(size_t)q * A.ld + min(k, n - 1)];
       }
       if (!(ok = grid_sync(A.ctr, target, &okf))) break;
-      for (int c = wv; c <= i + 1; c += 16) {
+      for (int c = wv; wv < 4 && c <= i + 1; c += 16) {
         double2 p0[4], p1[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -545,7 +564,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
         }
       }
       __syncthreads();
-      if (wv == 3) {
+      if (wv == 4) {
         // Givens rotations and the stop test (gmres.cpp:568-592), beside the update
         if (lane == 0) {
           const double hh = lh[i + 1];
@@ -567,9 +586,12 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
           stopf = fabs(e1) < eps ? 1 : 0;
         }
       }
-      {
+      if (wv < 4) {
         double z = w;
-        for (int jq = 0; jq <= i; jq += 8) {
+#pragma unroll
+        for (int q = 0; q < GM_PF; q++)
+          if (q <= i) z = z + (-sums[q]) * pv[q];
+        for (int jq = GM_PF; jq <= i; jq += 8) {
           double q8[8];
 #pragma unroll
           for (int q = 0; q < 8; q++) q8[q] = A.u[(size_t)min(jq + q, i) * A.ld + min(k, n - 1)];
