@@ -413,44 +413,59 @@ __global__ __launch_bounds__(256) void k_cl_ac(int nSeg, const int* __restrict__
 // No pivoting: the matrix is definite (every pivot a leading principal minor's
 // ratio, nonzero); a zero or non-finite pivot raises *flag.
 
+// The entry of lane p (uniform).
+__device__ __forceinline__ double lane_value(double v, int p)
+{
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, p), hi = __builtin_amdgcn_readlane((int)(b >> 32), p);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
 // The pivot block by unpivoted Gauss-Jordan in registers: lane (w, i) of the
-// 256 holds row i, columns 16w..16w+15 (v); step p publishes row p and column
-// p through LDS, double buffered by the step's parity (a thread writing step
-// p + 1's buffer has passed step p's barrier, so every thread has read that
-// buffer at step p - 1), one barrier per step. Block column K of the
-// elimination: a zero or non-finite pivot raises *flag.
-__device__ __forceinline__ void gj_pivot_regs(double (&v)[16], int K, double (&rowb)[2][GJB],
-                                              double (&colb)[2][GJB], int* __restrict__ flag)
+// 256 holds row i, columns 16w..16w+15 (v). Row p is each wavefront's own lane
+// p, column p goes through LDS, double buffered by the step's parity (a thread
+// writing step p + 1's buffer has passed step p's barrier, so every thread has
+// read that buffer at step p - 1), one barrier per step. A serial chain of 64
+// steps on one workgroup: the steps run as a loop over the wavefronts' 16
+// columns, whose code is fetched once (the update of a 3328-column block that
+// carries it 54.6 -> 49.6 us, with all 64 steps unrolled and row p through LDS
+// too before). Block column K of the elimination: a zero or non-finite pivot
+// raises *flag.
+__device__ __forceinline__ void gj_pivot_regs(double (&v)[16], int K, double (&colb)[2][GJB],
+                                              int* __restrict__ flag)
 {
   static_assert(GJB == 64, "gj_pivot_regs: one row per lane");
-  const int t = threadIdx.x, i = t & 63, w = t >> 6, j0 = 16 * w;
+  const int i = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll 1
+  for (int pw = 0; pw < 4; pw++) {
 #pragma unroll
-  for (int p = 0; p < GJB; p++) {
-    const int buf = p & 1;
-    if (i == p) {
+    for (int pq = 0; pq < 16; pq++) {
+      const int p = 16 * pw + pq, buf = pq & 1;
+      if (w == pw) colb[buf][i] = v[pq];
+      __syncthreads();
+      const double pv = colb[buf][p], sip = colb[buf][i];
+      // 1 / pv: the hardware reciprocal refined by two Newton steps (a shorter
+      // dependent chain than the correctly rounded division; this is the
+      // elimination's critical path)
+      double inv = __builtin_amdgcn_rcp(pv);
+      inv = fma(inv, fma(-pv, inv, 1.0), inv);
+      inv = fma(inv, fma(-pv, inv, 1.0), inv);
+      // the general entry, then column p (one wavefront, a fixed register) and
+      // row p (one lane) overwritten: no per-entry selects
+      double r[16];
 #pragma unroll
-      for (int jj = 0; jj < 16; jj++) rowb[buf][j0 + jj] = v[jj];
+      for (int jj = 0; jj < 16; jj++) {
+        r[jj] = lane_value(v[jj], p) * inv;
+        v[jj] = v[jj] - sip * r[jj];
+      }
+      if (w == pw) v[pq] = -sip * inv;
+      if (i == p) {
+#pragma unroll
+        for (int jj = 0; jj < 16; jj++) v[jj] = r[jj];
+        if (w == pw) v[pq] = inv;
+      }
+      if (threadIdx.x == 0 && !(fabs(pv) > 0.0 && isfinite(pv))) *flag = 1 + K * GJB + p;
     }
-    if (w == p / 16) colb[buf][i] = v[p % 16];
-    __syncthreads();
-    const double pv = rowb[buf][p];
-    // 1 / pv: the hardware reciprocal refined by two Newton steps (a shorter
-    // dependent chain than the correctly rounded division; this is the
-    // elimination's critical path)
-    double inv = __builtin_amdgcn_rcp(pv);
-    inv = fma(inv, fma(-pv, inv, 1.0), inv);
-    inv = fma(inv, fma(-pv, inv, 1.0), inv);
-    const double sip = colb[buf][i];
-    // the general entry, then column p (one wavefront, a fixed register) and
-    // row p (one lane) overwritten: no per-entry selects
-#pragma unroll
-    for (int jj = 0; jj < 16; jj++) v[jj] = v[jj] - sip * (rowb[buf][j0 + jj] * inv);
-    if (w == p / 16) v[p % 16] = -sip * inv;
-    if (i == p) {
-#pragma unroll
-      for (int jj = 0; jj < 16; jj++) v[jj] = (j0 + jj == p) ? inv : rowb[buf][j0 + jj] * inv;
-    }
-    if (t == 0 && !(fabs(pv) > 0.0 && isfinite(pv))) *flag = 1 + K * GJB + p;
   }
 }
 
@@ -466,7 +481,7 @@ __global__ __launch_bounds__(256) void k_gj_pivot(const double* __restrict__ A0,
                                                   const long long* __restrict__ blkOff, int K,
                                                   double* __restrict__ piv0, int* __restrict__ flag)
 {
-  __shared__ double rowb[2][GJB], colb[2][GJB];
+  __shared__ double colb[2][GJB];
   const int b = blockIdx.z, N = blkN[b];
   if (K >= N / GJB) return;
   const double* A = A0 + blkOff[b] + (size_t)K * GJB * N + (size_t)K * GJB;
@@ -475,7 +490,7 @@ __global__ __launch_bounds__(256) void k_gj_pivot(const double* __restrict__ A0,
   double v[16];
 #pragma unroll
   for (int jj = 0; jj < 16; jj++) v[jj] = A[(size_t)i * N + j0 + jj];
-  gj_pivot_regs(v, K, rowb, colb, flag);
+  gj_pivot_regs(v, K, colb, flag);
 #pragma unroll
   for (int jj = 0; jj < 16; jj++) piv[i * GJB + j0 + jj] = v[jj];
 }
@@ -554,7 +569,7 @@ __global__ __launch_bounds__(256) void k_gj_update(double* __restrict__ A0, cons
                                                    const double* __restrict__ cp0, int* __restrict__ flag)
 {
   __shared__ double T[GJB][GJB + 1];
-  __shared__ double rowb[2][GJB], colb[2][GJB];
+  __shared__ double colb[2][GJB];
   const int b = blockIdx.z, N = blkN[b], nb = N / GJB;
   if (K >= nb || (int)blockIdx.x >= nb || (int)blockIdx.y >= nb) return;
   double* A = A0 + blkOff[b];
@@ -596,7 +611,7 @@ __global__ __launch_bounds__(256) void k_gj_update(double* __restrict__ A0, cons
   double vr[16];
 #pragma unroll
   for (int jj = 0; jj < 16; jj++) vr[jj] = T[i][j0 + jj];
-  gj_pivot_regs(vr, K + 1, rowb, colb, flag);
+  gj_pivot_regs(vr, K + 1, colb, flag);
   double* pn = gj_piv_slot(piv0, b, K + 1);
 #pragma unroll
   for (int jj = 0; jj < 16; jj++) pn[i * GJB + j0 + jj] = vr[jj];
