@@ -545,7 +545,7 @@ constexpr int FIN_BS = 1024;  // finaliser: one workgroup of 16 wavefronts
 struct FinLds {
   double sums[MAXM];
   double lh[MAXM], lcs[MAXM], lsn[MAXM];
-  double pre_err, pre_eps;
+  double pre_err, pre_eps, hh, cur;
   int pre_itr;
 };
 
@@ -565,32 +565,48 @@ __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restr
   double& pre_err = S.pre_err;
   double& pre_eps = S.pre_eps;
   int& pre_itr = S.pre_itr;
-  if (A.mode == FIN_ARNOLDI && st->done) return;
+  // a finished cycle is left at the first barrier: the flag's load overlaps the sums'
+  const int done = A.mode == FIN_ARNOLDI ? st->done : 0;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   if (A.mode == FIN_ARNOLDI) {
     if (t == 64) pre_err = err[A.i];
     if (t == 128) pre_eps = st->eps;
     if (t == 192) pre_itr = st->itr;
   }
-  for (int j = wv; j < m; j += FIN_BS / 64) {
-    const double* pj = partial + (size_t)j * pstride;
-    double acc = 0.0;
-    // the lane's partials b = lane, lane + 64, ... added in order; loaded 16
-    // at a time (indices clamped, clamped values unused) so that the loads
-    // overlap instead of costing one memory latency each
-    for (int b0 = 0; b0 < nblk; b0 += 16 * 64) {
-      double v[16];
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int b = b0 + lane + 64 * q;
-        v[q] = pj[b < nblk ? b : nblk - 1];
+  constexpr int W = FIN_BS / 64;
+  if (nblk <= 64) {
+    // one partial a lane: a wavefront's columns two at a time
+    for (int j = wv; j < m; j += 2 * W) {
+      const int b = min(lane, nblk - 1), k = min(j + W, m - 1);
+      const double x = partial[(size_t)j * pstride + b], y = partial[(size_t)k * pstride + b];
+      double acc[2] = {lane < nblk ? 0.0 + x : 0.0, lane < nblk ? 0.0 + y : 0.0};
+      wave_sums<2>(acc);
+      if (lane == 0) {
+        sums[j] = acc[0];
+        if (j + W < m) sums[j + W] = acc[1];
       }
-#pragma unroll
-      for (int q = 0; q < 16; q++)
-        if (b0 + lane + 64 * q < nblk) acc = acc + v[q];
     }
-    acc = wave_sum(acc);
-    if (lane == 0) sums[j] = acc;
+  } else {
+    for (int j = wv; j < m; j += W) {
+      const double* pj = partial + (size_t)j * pstride;
+      double acc = 0.0;
+      // the lane's partials b = lane, lane + 64, ... added in order; loaded 16
+      // at a time (indices clamped, clamped values unused) so that the loads
+      // overlap instead of costing one memory latency each
+      for (int b0 = 0; b0 < nblk; b0 += 16 * 64) {
+        double v[16];
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+          const int b = b0 + lane + 64 * q;
+          v[q] = pj[b < nblk ? b : nblk - 1];
+        }
+#pragma unroll
+        for (int q = 0; q < 16; q++)
+          if (b0 + lane + 64 * q < nblk) acc = acc + v[q];
+      }
+      acc = wave_sum(acc);
+      if (lane == 0) sums[j] = acc;
+    }
   }
   if (A.mode == FIN_ARNOLDI) {
     for (int j = t; j < A.i; j += FIN_BS) {
@@ -599,6 +615,7 @@ __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restr
     }
   }
   __syncthreads();
+  if (done) return;
   if (A.mode == FIN_DOT) {
     if (t == 0) out[0] = sums[0];
     return;
@@ -667,26 +684,38 @@ __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restr
     }
     return;
   }
-  // FIN_ARNOLDI: serial part on LDS by one lane, then parallel stores
+  // FIN_ARNOLDI: two serial chains, on a wavefront each: the Pythagorean norm
+  // and the earlier columns' rotations (their running entry in a register)
   const int i = A.i, ldh = A.sD + 1;
   if (t == 0) {
-    for (int j = 0; j <= i + 1; j++) lh[j] = sums[j];
-    double hh = lh[i + 1];
-    for (int j = 0; j <= i; j++) hh = hh - lh[j] * lh[j];
+    double hh = sums[i + 1];
+#pragma unroll 8
+    for (int j = 0; j <= i; j++) hh = hh - sums[j] * sums[j];
     hh = sqrt(fabs(hh));
-    lh[i + 1] = hh;
+    S.hh = hh;
     st->scale = 1.0 / hh;
-    for (int j = 0; j <= i - 1; j++) {
-      double tmp = lcs[j] * lh[j] + lsn[j] * lh[j + 1];
-      lh[j + 1] = -lsn[j] * lh[j] + lcs[j] * lh[j + 1];
-      lh[j] = tmp;
+  } else if (t == 64) {
+    double cur = sums[0];
+#pragma unroll 8
+    for (int j = 0; j < i; j++) {
+      const double nx = sums[j + 1];
+      lh[j] = lcs[j] * cur + lsn[j] * nx;
+      cur = -lsn[j] * cur + lcs[j] * nx;
     }
-    double tmp = sqrt(lh[i] * lh[i] + lh[i + 1] * lh[i + 1]);
-    double c = lh[i] / tmp, sv = lh[i + 1] / tmp;
+    S.cur = cur;
+  }
+  __syncthreads();
+  double* hc = h + (size_t)ldh * i;
+  for (int j = t; j < i; j += FIN_BS) hc[j] = lh[j];
+  for (int j = t; j <= i; j += FIN_BS) coef[j] = sums[j];
+  if (t == 0) {
+    const double hh = S.hh, hi = S.cur;
+    double tmp = sqrt(hi * hi + hh * hh);
+    double c = hi / tmp, sv = hh / tmp;
     cs[i] = c;
     sn[i] = sv;
-    lh[i] = tmp;
-    lh[i + 1] = 0.0;
+    hc[i] = tmp;
+    hc[i + 1] = 0.0;
     double ei = pre_err;
     double e1 = -sv * ei;
     err[i + 1] = e1;
@@ -717,10 +746,6 @@ __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restr
       }
     }
   }
-  __syncthreads();
-  double* hc = h + (size_t)ldh * i;
-  for (int j = t; j <= i + 1; j += FIN_BS) hc[j] = lh[j];
-  for (int j = t; j <= i; j += FIN_BS) coef[j] = sums[j];
 }
 
 __global__ __launch_bounds__(FIN_BS) void k_fin(FinArgs A, const double* __restrict__ partial, int nblk, int m,
