@@ -488,26 +488,52 @@ __device__ __forceinline__ void span_dots(const TWv* __restrict__ w, const T* __
 
 constexpr int MDOT_CB_G = 4;  // FP32 basis columns per load batch (4: 24.1 us, 8: 25.1 us on the 1.2M-tet pipe)
 
-// Dots of w against m vectors base + j*ld (j < m), pass 1: each workgroup
-// sums its 1024-element span (256 lanes x 4 elements at stride 256, in order),
-// butterflies inside each wavefront and adds the 4 wavefront sums in order;
+// Columns a workgroup of the dots' first pass takes. With few spans a workgroup
+// a span leaves compute units waiting on one column batch's latency after the
+// other: the columns are split over up to `wgs` workgroups in all, eight columns
+// at least each (w is read again by each of them). 230 spans, FP32 basis: 10.4
+// -> 6.9 us a step; 810 spans: FP32 19.3 -> 18.7 us with two, FP64 (twice the
+// bytes in flight) 31.7 -> 33.5, so it is split only below 512 spans.
+constexpr int DOT_WGS_F32 = 2048, DOT_WGS_F64 = 1024;
+static int dot_cols(int nblk, int mc, int wgs)
+{
+  const int split = std::max(1, std::min((mc + 7) / 8, wgs / std::max(nblk, 1)));
+  return (mc + split - 1) / split;
+}
+
+// Dots of w against m vectors base + j*ld (j < m) and, with self, w.w as column
+// m, pass 1: workgroup (b, y) takes the columns [y cols, (y + 1) cols) of span
+// b (1024 elements [k0, kend)): 256 lanes x 4 elements at stride 256, in order,
+// butterflies inside each wavefront, the 4 wavefront sums added in order;
 // partial[j*nblk + b].
-__global__ __launch_bounds__(RED_BS) void k_mdot(int n, const double* __restrict__ w, const double* __restrict__ base,
-                                                 size_t ld, int m, double* __restrict__ partial,
-                                                 const int* __restrict__ skip)
+template <int G, typename T, typename TWv>
+__device__ __forceinline__ void mdot_body(const TWv* __restrict__ w, const T* __restrict__ base, size_t ld, int m,
+                                          bool self, int cols, size_t k0, size_t kend, double* __restrict__ partial,
+                                          int nblk, double* lds)
 {
 #pragma clang fp contract(off)
-  extern __shared__ double lds[];  // [RED_NW waves][m]
-  if (skip && *skip) return;
-  const int t = threadIdx.x;
-  const int nblk = gridDim.x;
-  span_dots<1>(w, base, ld, m, false, (size_t)blockIdx.x * RED_SPAN + t, (size_t)n, lds, m);
+  const int t = threadIdx.x, j0 = blockIdx.y * cols, mc = min(m + (self ? 1 : 0) - j0, cols);
+  const bool own = self && j0 + mc == m + 1;  // column m is this workgroup's last
+  span_dots<G>(w, base + (size_t)j0 * ld, ld, own ? mc - 1 : mc, own, k0 + t, kend, lds, mc);
   __syncthreads();
-  for (int j = t; j < m; j += RED_BS) {
+  for (int j = t; j < mc; j += RED_BS) {
     double v = lds[j];
-    for (int q = 1; q < RED_NW; q++) v = v + lds[q * m + j];
-    partial[(size_t)j * nblk + blockIdx.x] = v;
+    for (int q = 1; q < RED_NW; q++) v = v + lds[q * mc + j];
+    partial[(size_t)(j0 + j) * nblk + blockIdx.x] = v;
   }
+}
+
+__global__ __launch_bounds__(RED_BS) void k_mdot(int n, const double* __restrict__ w, const double* __restrict__ base,
+                                                 size_t ld, int m, int cols, double* __restrict__ partial,
+                                                 const int* __restrict__ skip)
+{
+  extern __shared__ double lds[];  // [RED_NW waves][cols]
+  if (skip && *skip) return;
+  const size_t k0 = (size_t)blockIdx.x * RED_SPAN;
+  if (gridDim.y > 1)
+    mdot_body<4>(w, base, ld, m, false, cols, k0, (size_t)n, partial, gridDim.x, lds);
+  else
+    mdot_body<1>(w, base, ld, m, false, cols, k0, (size_t)n, partial, gridDim.x, lds);
 }
 
 // The mixed-precision solve keeps its Krylov basis in FP32 (a compressed
@@ -515,21 +541,12 @@ __global__ __launch_bounds__(RED_BS) void k_mdot(int n, const double* __restrict
 // base + j*ld, then w.w as column m, in k_mdot's order; partial[j*nblk + b].
 template <typename TWv>
 __global__ __launch_bounds__(RED_BS) void k_mdot_cb(int n, const TWv* __restrict__ w, const float* __restrict__ base,
-                                                    size_t ld, int m, double* __restrict__ partial,
+                                                    size_t ld, int m, int cols, double* __restrict__ partial,
                                                     const int* __restrict__ skip)
 {
-#pragma clang fp contract(off)
-  extern __shared__ double lds[];  // [RED_NW waves][m + 1]
+  extern __shared__ double lds[];  // [RED_NW waves][cols]
   if (skip && *skip) return;
-  const int t = threadIdx.x;
-  const int nblk = gridDim.x, mc = m + 1;
-  span_dots<MDOT_CB_G>(w, base, ld, m, true, (size_t)blockIdx.x * RED_SPAN + t, (size_t)n, lds, mc);
-  __syncthreads();
-  for (int j = t; j < mc; j += RED_BS) {
-    double v = lds[j];
-    for (int q = 1; q < RED_NW; q++) v = v + lds[q * mc + j];
-    partial[(size_t)j * nblk + blockIdx.x] = v;
-  }
+  mdot_body<MDOT_CB_G>(w, base, ld, m, true, cols, (size_t)blockIdx.x * RED_SPAN, (size_t)n, partial, gridDim.x, lds);
 }
 
 constexpr int FIN_BS = 1024;  // finaliser: one workgroup of 16 wavefronts
@@ -1409,8 +1426,9 @@ static int dot_device(int n, const double* w, const double* base, size_t ld, int
   if (m > MAXM) return set_error(SVG_ERR_ARG, "reduction: too many sums");
   const int* skip = (fa.mode == FIN_ARNOLDI) ? &st->done : nullptr;
   // algorithmic bytes: w and the m - 1 basis vectors read, the partials written; the finaliser reads them
-  launch_b("mdot", 8.0 * n * m + 8.0 * m * nblk, k_mdot, dim3(nblk), dim3(RED_BS), (size_t)RED_NW * m * sizeof(double),
-           s, n, w, base, ld, m, partial, skip);
+  const int cols = dot_cols(nblk, m, DOT_WGS_F64);
+  launch_b("mdot", 8.0 * n * m + 8.0 * m * nblk, k_mdot, dim3(nblk, (m + cols - 1) / cols), dim3(RED_BS),
+           (size_t)RED_NW * cols * sizeof(double), s, n, w, base, ld, m, cols, partial, skip);
   launch_b("mdot_fin", 8.0 * m * nblk, k_fin, dim3(1), dim3(FIN_BS), 0, s, fa, (const double*)partial, nblk, m, st,
            h, cs, sn, err, coef, out, (volatile int*)host_done);
   return SVG_OK;
@@ -1425,10 +1443,11 @@ static int dot_device_cb(int n, const TWv* w, const float* base, size_t ld, int 
   int nblk = (n + RED_SPAN - 1) / RED_SPAN;
   if (nblk < 1) nblk = 1;
   if (m + 1 > MAXM) return set_error(SVG_ERR_ARG, "reduction: too many sums");
+  const int cols = dot_cols(nblk, m + 1, DOT_WGS_F32);
   // algorithmic bytes: w (FP64 or FP32) and the m FP32 basis vectors read, the partials written
-  launch_b("mdot_cb", (double)sizeof(TWv) * n + 4.0 * n * m + 8.0 * (m + 1) * nblk, k_mdot_cb<TWv>, dim3(nblk),
-           dim3(RED_BS), (size_t)RED_NW * (m + 1) * sizeof(double), s, n, w, base, ld, m, k.partial,
-           (const int*)&k.st->done);
+  launch_b("mdot_cb", (double)sizeof(TWv) * n + 4.0 * n * m + 8.0 * (m + 1) * nblk, k_mdot_cb<TWv>,
+           dim3(nblk, m / cols + 1), dim3(RED_BS), (size_t)RED_NW * cols * sizeof(double), s, n, w, base, ld, m, cols,
+           k.partial, (const int*)&k.st->done);
   launch_b("mdot_fin", 8.0 * (m + 1) * nblk, k_fin, dim3(1), dim3(FIN_BS), 0, s, fa, (const double*)k.partial, nblk,
            m + 1, k.st, k.h, k.cs, k.sn, k.err, k.coef, k.scal, (volatile int*)k.d_done);
   return SVG_OK;
@@ -2429,48 +2448,33 @@ static int precond_diag_dev(svg_lhs* L, int dof, double* Val, double* R, double*
 __global__ __launch_bounds__(RED_BS) void k_bmdot(const int* __restrict__ spanStart, const int* __restrict__ spanEnd,
                                                   const int* __restrict__ spanSys, int nsp,
                                                   const double* __restrict__ w, const double* __restrict__ base,
-                                                  size_t ld, int m, double* __restrict__ partial,
+                                                  size_t ld, int m, int cols, double* __restrict__ partial,
                                                   const GmState* __restrict__ st, int check)
 {
-#pragma clang fp contract(off)
-  extern __shared__ double lds[];  // [RED_NW waves][m]
+  extern __shared__ double lds[];  // [RED_NW waves][cols]
   const int b = blockIdx.x;
   if (check) {  // 1: skip systems that stopped iterating; 2: also those done in this cycle
     const GmState& S = st[spanSys[b]];
     if (!S.act || (check == 2 && S.done)) return;
   }
-  const int t = threadIdx.x;
-  span_dots<1>(w, base, ld, m, false, (size_t)spanStart[b] + t, (size_t)spanEnd[b], lds, m);
-  __syncthreads();
-  for (int j = t; j < m; j += RED_BS) {
-    double v = lds[j];
-    for (int q = 1; q < RED_NW; q++) v = v + lds[q * m + j];
-    partial[(size_t)j * nsp + b] = v;
-  }
+  if (gridDim.y > 1)
+    mdot_body<4>(w, base, ld, m, false, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
+  else
+    mdot_body<1>(w, base, ld, m, false, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
 }
 
 // k_mdot_cb per span of the batched solve (FP32 basis, then w.w as column m).
 __global__ __launch_bounds__(RED_BS) void k_bmdot_cb(const int* __restrict__ spanStart,
                                                      const int* __restrict__ spanEnd, const int* __restrict__ spanSys,
                                                      int nsp, const double* __restrict__ w,
-                                                     const float* __restrict__ base, size_t ld, int m,
+                                                     const float* __restrict__ base, size_t ld, int m, int cols,
                                                      double* __restrict__ partial, const GmState* __restrict__ st)
 {
-#pragma clang fp contract(off)
-  extern __shared__ double lds[];  // [RED_NW waves][m + 1]
-  const int b = blockIdx.x, mc = m + 1;
-  {
-    const GmState& S = st[spanSys[b]];
-    if (!S.act || S.done) return;
-  }
-  const int t = threadIdx.x;
-  span_dots<MDOT_CB_G>(w, base, ld, m, true, (size_t)spanStart[b] + t, (size_t)spanEnd[b], lds, mc);
-  __syncthreads();
-  for (int j = t; j < mc; j += RED_BS) {
-    double v = lds[j];
-    for (int q = 1; q < RED_NW; q++) v = v + lds[q * mc + j];
-    partial[(size_t)j * nsp + b] = v;
-  }
+  extern __shared__ double lds[];  // [RED_NW waves][cols]
+  const int b = blockIdx.x;
+  const GmState& S = st[spanSys[b]];
+  if (!S.act || S.done) return;
+  mdot_body<MDOT_CB_G>(w, base, ld, m, true, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
 }
 
 // The FP32 SpMV of the batched solve: rows of systems that converged or
@@ -2506,14 +2510,27 @@ __global__ __launch_bounds__(256) void k_bgs_update(int n, double* __restrict__ 
   const double* c = coef + (size_t)sy * (sD + 2);
   double* w = u + (size_t)(i + 1) * ld;
   double v = w[k];
-  for (int j = 0; j <= i; j++) v = v + (-c[j]) * u[(size_t)j * ld + k];
+  // eight vectors' loads (and the system's coefficients) issued before their updates
+  for (int j0 = 0; j0 <= i; j0 += 8) {
+    double b[8], cj[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int j = min(j0 + q, i);
+      b[q] = u[(size_t)j * ld + k];
+      cj[q] = c[j];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (j0 + q <= i) v = v + (-cj[q]) * b[q];
+  }
   v = S.scale * v;
   w[k] = v;
   if (u32) u32[k] = (float)v;
   if (z) z[k] = v;  // flexible solve: the next step is one the network does not precondition
 }
 
-// k_gs_update_cb per system of the batched solve (each node's 4 rows belong to one system).
+// k_gs_update_cb per system of the batched solve (each node's 4 rows belong to
+// one system), eight vectors' loads ahead of their updates.
 __global__ __launch_bounds__(256) void k_bgs_update_cb(int n, double* __restrict__ w, float* __restrict__ v32,
                                                        size_t ld, int i, int sD, const double* __restrict__ coef,
                                                        const GmState* __restrict__ st,
@@ -2527,11 +2544,21 @@ __global__ __launch_bounds__(256) void k_bgs_update_cb(int n, double* __restrict
   if (!S.act || S.done) return;
   const double* c = coef + (size_t)sy * (sD + 2);
   double2 v = *reinterpret_cast<const double2*>(w + k);
-  for (int j = 0; j <= i; j++) {
-    const float2 b = *reinterpret_cast<const float2*>(v32 + (size_t)j * ld + k);
-    const double cj = -c[j];
-    v.x = v.x + cj * (double)b.x;
-    v.y = v.y + cj * (double)b.y;
+  for (int j0 = 0; j0 <= i; j0 += 8) {
+    float2 b[8];
+    double cj[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int j = min(j0 + q, i);
+      b[q] = *reinterpret_cast<const float2*>(v32 + (size_t)j * ld + k);
+      cj[q] = -c[j];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (j0 + q <= i) {
+        v.x = v.x + cj[q] * (double)b[q].x;
+        v.y = v.y + cj[q] * (double)b[q].y;
+      }
   }
   v.x = S.scale * v.x;
   v.y = S.scale * v.y;
@@ -2666,9 +2693,10 @@ static void batch_graph_free(svg_batch* B)
 
 static void batch_mdot(svg_batch* B, const double* w, const double* base, size_t ld, int m, int check, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_bmdot, dim3(B->nsp), dim3(RED_BS), (size_t)RED_NW * m * sizeof(double), s,
-                     (const int*)B->d_spanStart, (const int*)B->d_spanEnd, (const int*)B->d_spanSys, B->nsp, w, base,
-                     ld, m, B->partial, (const GmState*)B->st, check);
+  const int cols = dot_cols(B->nsp, m, DOT_WGS_F64);
+  hipLaunchKernelGGL(k_bmdot, dim3(B->nsp, (m + cols - 1) / cols), dim3(RED_BS),
+                     (size_t)RED_NW * cols * sizeof(double), s, (const int*)B->d_spanStart, (const int*)B->d_spanEnd,
+                     (const int*)B->d_spanSys, B->nsp, w, base, ld, m, cols, B->partial, (const GmState*)B->st, check);
 }
 
 static void batch_fin(svg_batch* B, const FinArgs& fa, int m, hipStream_t s)
@@ -2777,9 +2805,11 @@ static int batch_cycle(svg_batch* B, const double* Val, const double* R, const B
              tl ? (const float*)(B->z32 + B->ld * i)
                 : (netStep(i) ? (const float*)B->u32 : (const float*)(B->v32 + B->ld * i)),
              un, nullptr, s, "bspmv32", (const int*)B->d_sysOfNode, (const GmState*)B->st);
-      hipLaunchKernelGGL(k_bmdot_cb, dim3(B->nsp), dim3(RED_BS), (size_t)RED_NW * (i + 2) * sizeof(double), s,
-                         (const int*)B->d_spanStart, (const int*)B->d_spanEnd, (const int*)B->d_spanSys, B->nsp,
-                         (const double*)un, (const float*)B->v32, B->ld, i + 1, B->partial, (const GmState*)B->st);
+      const int cols = dot_cols(B->nsp, i + 2, DOT_WGS_F32);
+      hipLaunchKernelGGL(k_bmdot_cb, dim3(B->nsp, (i + 1) / cols + 1), dim3(RED_BS),
+                         (size_t)RED_NW * cols * sizeof(double), s, (const int*)B->d_spanStart,
+                         (const int*)B->d_spanEnd, (const int*)B->d_spanSys, B->nsp, (const double*)un,
+                         (const float*)B->v32, B->ld, i + 1, cols, B->partial, (const GmState*)B->st);
       batch_fin(B, fa, i + 2, s);
       hipLaunchKernelGGL(k_bgs_update_cb, dim3(nbv2), dim3(256), 0, s, n, un, B->v32, B->ld, i, sD,
                          (const double*)B->coef, (const GmState*)B->st, (const int*)B->d_sysOfNode,

@@ -253,6 +253,26 @@ def test_gmres_one_launch_cycles(torch_cuda, phys, n, nz, sD, cycles):
         assert np.array_equal(dR.cpu().numpy(), x0)
 
 
+@pytest.mark.parametrize("n,nz,sD", [(16, 60, 50), (24, 125, 27), (28, 125, 18)])
+def test_gmres_split_dots(torch_cuda, phys, n, nz, sD):
+    """gmres_v where the dots' columns are split over workgroups (69 spans: up to
+    seven ways, 308: up to three, 414: up to two), every number of columns up to
+    the Krylov dimension: bit for bit the device-order oracle."""
+    from svfsiplus_amd.newton import DeviceLhs, fsils_solve, ls_create
+    torch = torch_cuda
+    p = W.make_pipe(n, nz=nz)
+    Ag, Yg = _state(p, phys, seed=n)
+    R, V = oracle.construct_fluid(p, phys, Ag, Yg)
+    with oracle.device_order():
+        x0, _, ols = oracle.fsils_solve(
+            p, oracle.ls_create(oracle.LS_GMRES, relTol=1e-9, absTol=1e-30, maxItr=1, dimKry=sD), R, V)
+    ls = ls_create(_lib.LS_GMRES, relTol=1e-9, absTol=1e-30, maxItr=1, dimKry=sD)
+    dR, dV = _dev(torch, R), _dev(torch, V)
+    fsils_solve(DeviceLhs(p), ls, 4, dR, dV)
+    assert (ls.RI.itr, ls.RI.suc, ls.RI.iNorm, ls.RI.fNorm) == (ols.RI.itr, ols.RI.suc, ols.RI.iNorm, ols.RI.fNorm)
+    assert np.array_equal(dR.cpu().numpy(), x0)
+
+
 def test_newton_time_step(torch_cuda, phys):
     """Three Newton iterations (pici, construct_fluid, fsils_solve, picc) against the oracle:
     identical linear iteration counts and residual norms to the device-order oracle (assembly
