@@ -245,13 +245,13 @@ int coarse_check(const svg_lhs* L, hipStream_t s);
 // z = M(v) in FP64 (z64) and/or FP32 (z32); skip: kernels return at once when *skip.
 void coarse_apply_dev(const svg_lhs* L, const float* v, double* z64, float* z32, const int* skip, hipStream_t s);
 void coarse_apply_dev(const svg_lhs* L, const double* v, double* z64, float* z32, const int* skip, hipStream_t s);
-// The batched solve's form (one coarse block per system): the systems that do
-// not iterate in the cycle (per st and sysOfNode) are skipped, and the
-// systems that fell back to the diagonal preconditioner get z = v.
-void coarse_apply_batch_dev(const svg_lhs* L, const float* v, double* z64, float* z32, const GmState* st,
-                            const int* sysOfNode, hipStream_t s);
-void coarse_apply_batch_dev(const svg_lhs* L, const double* v, double* z64, float* z32, const GmState* st,
-                            const int* sysOfNode, hipStream_t s);
+// The batched solve's form (one coarse block per system of B): the systems
+// that do not iterate in the cycle are skipped, and the systems that fell back
+// to the diagonal preconditioner get z = v.
+void coarse_apply_batch_dev(const svg_lhs* L, const float* v, double* z64, float* z32, const svg_batch* B,
+                            hipStream_t s);
+void coarse_apply_batch_dev(const svg_lhs* L, const double* v, double* z64, float* z32, const svg_batch* B,
+                            hipStream_t s);
 // With another smoother: r2 = v - A P zc (FP64; the coarse solution zc is kept),
 // then, after the smoother wrote z from r2, z(3, i) += zc(agg(i)).
 void coarse_residual_dev(const svg_lhs* L, const float* v, double* r2, const int* skip, hipStream_t s);
@@ -334,6 +334,7 @@ struct svg_batch {
   std::vector<int> nodeOff;               // nsys + 1
   int *d_sysOfNode = nullptr, *d_spanStart = nullptr, *d_spanEnd = nullptr, *d_spanSys = nullptr;
   int* d_sysSpanOff = nullptr;            // nsys + 1
+  int maxSysSpans = 0;                    // the largest system's
   double *u = nullptr, *X = nullptr, *h = nullptr, *cs = nullptr, *sn = nullptr, *err = nullptr, *coef = nullptr,
          *y = nullptr, *partial = nullptr;
   svg::GmState* st = nullptr;

@@ -566,6 +566,99 @@ struct FinLds {
   int pre_itr;
 };
 
+// The sums of m columns of up to 64 partials (column j's at partial[j *
+// pstride + b]): one partial a lane, a wavefront's columns two at a time.
+template <int W>
+__device__ __forceinline__ void fin_sums64(const double* __restrict__ partial, size_t pstride, int nblk, int m,
+                                           double* __restrict__ sums)
+{
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int j = wv; j < m; j += 2 * W) {
+    const int b = min(lane, nblk - 1), k = min(j + W, m - 1);
+    const double x = partial[(size_t)j * pstride + b], y = partial[(size_t)k * pstride + b];
+    double acc[2] = {lane < nblk ? 0.0 + x : 0.0, lane < nblk ? 0.0 + y : 0.0};
+    wave_sums<2>(acc);
+    if (lane == 0) {
+      sums[j] = acc[0];
+      if (j + W < m) sums[j + W] = acc[1];
+    }
+  }
+}
+
+// The Pythagorean norm h(i+1, i) (gmres.cpp:556-566), a serial chain.
+__device__ __forceinline__ double arnoldi_norm(int i, const double* __restrict__ sums)
+{
+#pragma clang fp contract(off)
+  double hh = sums[i + 1];
+#pragma unroll 8
+  for (int j = 0; j <= i; j++) hh = hh - sums[j] * sums[j];
+  return sqrt(fabs(hh));
+}
+
+// The earlier columns' rotations applied to column i (a serial chain, its
+// running entry in a register): rows 0 .. i-1 to lh, row i returned.
+__device__ __forceinline__ double arnoldi_rotate(int i, const double* __restrict__ sums,
+                                                 const double* __restrict__ lcs, const double* __restrict__ lsn,
+                                                 double* __restrict__ lh)
+{
+#pragma clang fp contract(off)
+  double cur = sums[0];
+#pragma unroll 8
+  for (int j = 0; j < i; j++) {
+    const double nx = sums[j + 1];
+    lh[j] = lcs[j] * cur + lsn[j] * nx;
+    cur = -lsn[j] * cur + lcs[j] * nx;
+  }
+  return cur;
+}
+
+// Column i's rotation, the residual estimate and the stop tests
+// (gmres.cpp:568-592), by one lane.
+__device__ __forceinline__ void arnoldi_close(const FinArgs& A, double hh, double hi, double pre_err, double pre_eps,
+                                              int pre_itr, GmState* st, double* __restrict__ hc,
+                                              double* __restrict__ cs, double* __restrict__ sn,
+                                              double* __restrict__ err, volatile int* host_done)
+{
+#pragma clang fp contract(off)
+  const int i = A.i;
+  double tmp = sqrt(hi * hi + hh * hh);
+  double c = hi / tmp, sv = hh / tmp;
+  cs[i] = c;
+  sn[i] = sv;
+  hc[i] = tmp;
+  hc[i + 1] = 0.0;
+  double ei = pre_err;
+  double e1 = -sv * ei;
+  err[i + 1] = e1;
+  err[i] = c * ei;
+  st->itr = pre_itr + 1;
+  st->last_i = i;
+  if (fabs(e1) < pre_eps) {
+    st->suc = 1;
+    st->done = 1;
+    if (host_done) {
+      *host_done = 1;
+      __threadfence_system();
+    }
+  } else if (A.fbwin > 0 && !st->fallback) {
+    // an iteration counts as decreasing when it lowers the smallest residual
+    // estimate so far by at least FB_DROP (relative); a system that fell back
+    // keeps iterating without the check
+    if (fabs(e1) < st->best * (1.0 - FB_DROP)) {
+      st->best = fabs(e1);
+      st->nondec = 0;
+    } else if (++st->nondec >= A.fbwin) {
+      st->fallback = 1;
+      st->done = 1;
+      if (host_done) {
+        *host_done = 1;
+        __threadfence_system();
+      }
+    }
+  }
+}
+
 // The finaliser's work for one system: column j's partials at
 // partial[j * pstride + b], b < nblk.
 __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restrict__ partial, size_t pstride,
@@ -592,17 +685,7 @@ __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restr
   }
   constexpr int W = FIN_BS / 64;
   if (nblk <= 64) {
-    // one partial a lane: a wavefront's columns two at a time
-    for (int j = wv; j < m; j += 2 * W) {
-      const int b = min(lane, nblk - 1), k = min(j + W, m - 1);
-      const double x = partial[(size_t)j * pstride + b], y = partial[(size_t)k * pstride + b];
-      double acc[2] = {lane < nblk ? 0.0 + x : 0.0, lane < nblk ? 0.0 + y : 0.0};
-      wave_sums<2>(acc);
-      if (lane == 0) {
-        sums[j] = acc[0];
-        if (j + W < m) sums[j + W] = acc[1];
-      }
-    }
+    fin_sums64<W>(partial, pstride, nblk, m, sums);
   } else {
     for (int j = wv; j < m; j += W) {
       const double* pj = partial + (size_t)j * pstride;
@@ -705,64 +788,16 @@ __device__ __forceinline__ void fin_body(const FinArgs& A, const double* __restr
   // and the earlier columns' rotations (their running entry in a register)
   const int i = A.i, ldh = A.sD + 1;
   if (t == 0) {
-    double hh = sums[i + 1];
-#pragma unroll 8
-    for (int j = 0; j <= i; j++) hh = hh - sums[j] * sums[j];
-    hh = sqrt(fabs(hh));
-    S.hh = hh;
-    st->scale = 1.0 / hh;
+    S.hh = arnoldi_norm(i, sums);
+    st->scale = 1.0 / S.hh;
   } else if (t == 64) {
-    double cur = sums[0];
-#pragma unroll 8
-    for (int j = 0; j < i; j++) {
-      const double nx = sums[j + 1];
-      lh[j] = lcs[j] * cur + lsn[j] * nx;
-      cur = -lsn[j] * cur + lcs[j] * nx;
-    }
-    S.cur = cur;
+    S.cur = arnoldi_rotate(i, sums, lcs, lsn, lh);
   }
   __syncthreads();
   double* hc = h + (size_t)ldh * i;
   for (int j = t; j < i; j += FIN_BS) hc[j] = lh[j];
   for (int j = t; j <= i; j += FIN_BS) coef[j] = sums[j];
-  if (t == 0) {
-    const double hh = S.hh, hi = S.cur;
-    double tmp = sqrt(hi * hi + hh * hh);
-    double c = hi / tmp, sv = hh / tmp;
-    cs[i] = c;
-    sn[i] = sv;
-    hc[i] = tmp;
-    hc[i + 1] = 0.0;
-    double ei = pre_err;
-    double e1 = -sv * ei;
-    err[i + 1] = e1;
-    err[i] = c * ei;
-    st->itr = pre_itr + 1;
-    st->last_i = i;
-    if (fabs(e1) < pre_eps) {
-      st->suc = 1;
-      st->done = 1;
-      if (host_done) {
-        *host_done = 1;
-        __threadfence_system();
-      }
-    } else if (A.fbwin > 0 && !st->fallback) {
-      // an iteration counts as decreasing when it lowers the smallest residual
-      // estimate so far by at least FB_DROP (relative); a system that fell back
-      // keeps iterating without the check
-      if (fabs(e1) < st->best * (1.0 - FB_DROP)) {
-        st->best = fabs(e1);
-        st->nondec = 0;
-      } else if (++st->nondec >= A.fbwin) {
-        st->fallback = 1;
-        st->done = 1;
-        if (host_done) {
-          *host_done = 1;
-          __threadfence_system();
-        }
-      }
-    }
-  }
+  if (t == 0) arnoldi_close(A, S.hh, S.cur, pre_err, pre_eps, pre_itr, st, hc, cs, sn, err, host_done);
 }
 
 __global__ __launch_bounds__(FIN_BS) void k_fin(FinArgs A, const double* __restrict__ partial, int nblk, int m,
@@ -2566,6 +2601,84 @@ __global__ __launch_bounds__(256) void k_bgs_update_cb(int n, double* __restrict
   if (keep64) *reinterpret_cast<double2*>(w + k) = v;
 }
 
+// k_bfin and k_bgs_update_cb in one launch, for systems of up to 64 spans: a
+// workgroup per span finishes its system's sums and the norm for itself (a few
+// kilobytes read once more instead of a launch between them); the system's
+// first one also records the Hessenberg column, the rotation and the state.
+// That record may set `done` while others still start: they skip then, and
+// what they would write is not read (the cycle ends at column i). 230 spans:
+// 8.2 us a step, 4.9 + 7.5 and a launch gap as two.
+constexpr int BFU_BS = RED_SPAN / 2;
+__global__ __launch_bounds__(BFU_BS) void k_bfin_update_cb(
+    FinArgs A, const int* __restrict__ spanStart, const int* __restrict__ spanEnd, const int* __restrict__ spanSys,
+    const int* __restrict__ sysSpanOff, int nsp, const double* __restrict__ partial, GmState* st,
+    double* __restrict__ h0, double* __restrict__ cs0, double* __restrict__ sn0, double* __restrict__ err0,
+    double* __restrict__ w, float* __restrict__ v32, size_t ld, int keep64)
+{
+#pragma clang fp contract(off)
+  __shared__ FinLds S;
+  __shared__ int done;
+  const int b = blockIdx.x, t = threadIdx.x, sy = spanSys[b], i = A.i, sD = A.sD;
+  GmState* g = st + sy;
+  if (!g->act) return;
+  const int off = sysSpanOff[sy], nb = sysSpanOff[sy + 1] - off;
+  const bool rec = b == off;  // this workgroup records
+  double *h = h0 + (size_t)sy * (sD + 1) * sD, *cs = cs0 + (size_t)sy * sD, *sn = sn0 + (size_t)sy * sD,
+         *err = err0 + (size_t)sy * (sD + 1);
+  if (t == 0) done = g->done;
+  if (rec) {
+    if (t == 64) S.pre_err = err[i];
+    if (t == 128) S.pre_eps = g->eps;
+    if (t == 192) S.pre_itr = g->itr;
+    for (int j = t; j < i; j += BFU_BS) {
+      S.lcs[j] = cs[j];
+      S.lsn[j] = sn[j];
+    }
+  }
+  // this lane's two entries and the first eight vectors', on their way meanwhile
+  const size_t k = (size_t)spanStart[b] + 2 * t, kend = spanEnd[b], kc = k < kend ? k : kend - 2;
+  double2 v = *reinterpret_cast<const double2*>(w + kc);
+  float2 f[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) f[q] = *reinterpret_cast<const float2*>(v32 + (size_t)min(q, i) * ld + kc);
+  fin_sums64<BFU_BS / 64>(partial + off, (size_t)nsp, nb, i + 2, S.sums);
+  __syncthreads();
+  if (done) return;
+  if (t == 0)
+    S.hh = arnoldi_norm(i, S.sums);
+  else if (t == 64 && rec)
+    S.cur = arnoldi_rotate(i, S.sums, S.lcs, S.lsn, S.lh);
+  for (int j0 = 0; j0 <= i; j0 += 8) {
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (j0 + q <= i) {
+        const double cj = -S.sums[j0 + q];
+        v.x = v.x + cj * (double)f[q].x;
+        v.y = v.y + cj * (double)f[q].y;
+      }
+    if (j0 + 8 <= i) {
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        f[q] = *reinterpret_cast<const float2*>(v32 + (size_t)min(j0 + 8 + q, i) * ld + kc);
+    }
+  }
+  __syncthreads();
+  const double scale = 1.0 / S.hh;
+  v.x = scale * v.x;
+  v.y = scale * v.y;
+  if (k < kend) {
+    *reinterpret_cast<float2*>(v32 + (size_t)(i + 1) * ld + k) = make_float2((float)v.x, (float)v.y);
+    if (keep64) *reinterpret_cast<double2*>(w + k) = v;
+  }
+  if (!rec) return;
+  double* hc = h + (size_t)(sD + 1) * i;
+  for (int j = t; j < i; j += BFU_BS) hc[j] = S.lh[j];
+  if (t == 0) {
+    g->scale = scale;
+    arnoldi_close(A, S.hh, S.cur, S.pre_err, S.pre_eps, S.pre_itr, g, hc, cs, sn, err, nullptr);
+  }
+}
+
 __global__ __launch_bounds__(256) void k_bdiv(int n, double* __restrict__ u, const GmState* __restrict__ st,
                                               const int* __restrict__ sysOfNode, float* __restrict__ u32)
 {
@@ -2774,12 +2887,10 @@ static int batch_cycle(svg_batch* B, const double* Val, const double* R, const B
       // back keep z_i = u_i (their flexible basis is the plain one; the apply
       // writes it)
       if (mixed) {
-        coarse_apply_batch_dev(L, (const float*)(B->v32 + B->ld * i), nullptr, B->z32 + B->ld * i,
-                               (const GmState*)B->st, (const int*)B->d_sysOfNode, s);
+        coarse_apply_batch_dev(L, (const float*)(B->v32 + B->ld * i), nullptr, B->z32 + B->ld * i, B, s);
       } else {
         double* zi = B->z + B->ld * i;
-        coarse_apply_batch_dev(L, (const double*)ui, zi, nullptr, (const GmState*)B->st,
-                               (const int*)B->d_sysOfNode, s);
+        coarse_apply_batch_dev(L, (const double*)ui, zi, nullptr, B, s);
         sin = zi;
       }
     } else if (netStep(i)) {
@@ -2810,10 +2921,16 @@ static int batch_cycle(svg_batch* B, const double* Val, const double* R, const B
                          (size_t)RED_NW * cols * sizeof(double), s, (const int*)B->d_spanStart,
                          (const int*)B->d_spanEnd, (const int*)B->d_spanSys, B->nsp, (const double*)un,
                          (const float*)B->v32, B->ld, i + 1, cols, B->partial, (const GmState*)B->st);
-      batch_fin(B, fa, i + 2, s);
-      hipLaunchKernelGGL(k_bgs_update_cb, dim3(nbv2), dim3(256), 0, s, n, un, B->v32, B->ld, i, sD,
-                         (const double*)B->coef, (const GmState*)B->st, (const int*)B->d_sysOfNode,
-                         (i + 1 < sD && netStep(i + 1)) ? 1 : 0);
+      const int keep64 = (i + 1 < sD && netStep(i + 1)) ? 1 : 0;
+      if (B->maxSysSpans <= 64) {
+        hipLaunchKernelGGL(k_bfin_update_cb, dim3(B->nsp), dim3(BFU_BS), 0, s, fa, (const int*)B->d_spanStart,
+                           (const int*)B->d_spanEnd, (const int*)B->d_spanSys, (const int*)B->d_sysSpanOff, B->nsp,
+                           (const double*)B->partial, B->st, B->h, B->cs, B->sn, B->err, un, B->v32, B->ld, keep64);
+      } else {
+        batch_fin(B, fa, i + 2, s);
+        hipLaunchKernelGGL(k_bgs_update_cb, dim3(nbv2), dim3(256), 0, s, n, un, B->v32, B->ld, i, sD,
+                           (const double*)B->coef, (const GmState*)B->st, (const int*)B->d_sysOfNode, keep64);
+      }
     } else {
       op_apply(A, sin, un, nullptr, nullptr, s);
       batch_mdot(B, un, B->u, B->ld, i + 2, 2, s);
@@ -3359,6 +3476,7 @@ int svg_batch_create(svg_lhs* L, int nsys, const int* nodeOff, int sD, svg_batch
     }
   }
   sysSpanOff[nsys] = (int)spanStart.size();
+  for (int q = 0; q < nsys; q++) B->maxSysSpans = std::max(B->maxSysSpans, sysSpanOff[q + 1] - sysSpanOff[q]);
   B->nsp = (int)spanStart.size();
   int rc;
   if ((rc = dev_alloc(&B->d_sysOfNode, (size_t)L->nNo)) || (rc = dev_alloc(&B->d_spanStart, (size_t)B->nsp)) ||

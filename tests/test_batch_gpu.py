@@ -242,6 +242,41 @@ def test_batch_twolevel_equals_individual_twolevel(torch_cuda, precision):
     bn.free()
 
 
+@pytest.mark.parametrize("precision", [_lib.PRECISION_FP64, _lib.PRECISION_MIXED])
+@pytest.mark.parametrize("tets,agg", [((2e3, 1.2e4), 32), ((2e3, 1.2e4), 60), ((2e3, 1.2e4), 2000),
+                                      ((1.0e5, 1.2e5), 220)])
+def test_batch_twolevel_small_blocks(torch_cuda, precision, tets, agg):
+    """The batched two-level solve where a coarse block has at most 128 columns
+    (blocks of one aggregate, of 64 and of 128 columns, both in one batch), with
+    systems of up to 64 reduction spans and of more: each mesh's solution is bit
+    for bit the single-system two-level solve."""
+    torch = torch_cuda
+    meshes = B.make_batch(W.bifurcation_batch(2, seed=31, tets_min=tets[0], tets_max=tets[1]))
+    bn = _assembled_union(torch, meshes, W.Physics())
+    Rb, Vb = bn.fn.R.clone(), bn.fn.Val.clone()
+    boff = np.concatenate([[0], np.cumsum([m.nnz for m in meshes])])
+    bn.proto.mItr, bn.proto.relTol = 3, 1e-9
+    opts = _lib.SolveOpts()
+    opts.precision, opts.method, opts.coarse, opts.fallback_window = precision, _lib.METHOD_LEARNED, agg, 20
+    _lib.check(_lib.load().svg_batch_fsils_solve_ex(bn.h, C.byref(bn.proto), Rb.data_ptr(), Vb.data_ptr(),
+                                                    C.byref(opts), bn.out, None))
+    torch.cuda.synchronize()
+    for q, m in enumerate(meshes):
+        a, b = int(bn.noff[q]), int(bn.noff[q + 1])
+        Rq, Vq = bn.fn.R[a:b].clone(), bn.fn.Val[boff[q]:boff[q + 1]].clone()
+        L = DeviceLhs(m)
+        ls = ls_create(_lib.LS_GMRES, relTol=1e-9, absTol=1e-30, maxItr=3, dimKry=50)
+        fsils_solve(L, ls, 4, Rq, Vq, precision=precision, coarse=agg, fallback_window=20)
+        na = C.c_int()
+        _lib.check(_lib.load().svg_coarse_info(L.h, C.byref(na), None))
+        print(f"mesh {q}: nNo {m.nNo} aggregates {na.value} itr {ls.RI.itr}")
+        assert na.value <= 128
+        assert (bn.out[q].itr, bn.out[q].suc, bn.out[q].iNorm) == (ls.RI.itr, ls.RI.suc, ls.RI.iNorm)
+        assert torch.equal(Rb[a:b], Rq)
+        L.free()
+    bn.free()
+
+
 def test_batch_twolevel_newton_graph_equals_eager(torch_cuda):
     """The graph-captured Newton iteration with the two-level preconditioner
     (its coarse blocks assembled and inverted inside the captured graph)
