@@ -132,15 +132,15 @@ int svg_lhs_pattern(const svg_lhs* lhs, int* rowPtr, int* colPtr); /* host copie
 /* with constant viscosity, one fluid domain, fixed mesh (mvMsh false).       */
 typedef struct svg_msh svg_msh;
 
-/* Uploads x and IEN, colours the elements, builds the element -> block slot
- * map over `lhs`'s pattern (the binary search of do_assem, lhsa.cpp:123-134)
- * and, for svg_construct_fluid, its inverse: per block slot the element
- * entries (e, a, b) that add to it, in element order. */
+/* Uploads x and IEN, colours the elements and builds, for
+ * svg_construct_fluid, the element entries (e, a, b) that add to each block
+ * slot of `lhs`'s pattern, in element order (do_assem's search for an entry's
+ * slot, lhsa.cpp:123-134, the other way round). */
 int svg_msh_create(const svg_lhs* lhs, int nEl, const int* IEN, int nNo, const double* x, svg_msh** msh);
 /* The same from device-resident IEN (4, nEl) and x (3, nNo), every step on
  * the device: Jones-Plassmann colouring (the sequential greedy colouring in
  * a fixed pseudo-random element order; no two elements of one colour share a
- * node; at most 256 colours), the stable colour order and the slot map.
+ * node; at most 256 colours), the stable colour order and the slots' entries.
  * Synchronises `stream`. */
 int svg_msh_create_dev(const svg_lhs* lhs, int nEl, const int* d_IEN, const double* d_x, svg_msh** msh,
                        void* stream);
@@ -379,7 +379,8 @@ int svg_spar_mul_vv(const svg_lhs* lhs, int dof, const double* d_K, const double
  * launch variants (unroll depth, non-temporal matrix streaming, per-XCD row
  * bands) compute bit-identical products; svg_spmv_tune times each on d_K over
  * lhs's pattern and keeps the fastest for this lhs (run automatically at the
- * first GMRES solve). */
+ * first GMRES solve that launches the product step by step; a small system's
+ * restart cycles are one launch and use none of the variants). */
 int svg_spmv_num_variants(int* count);
 int svg_spmv_time_variant(const svg_lhs* lhs, int variant, const double* d_K, const double* d_U, double* d_KU,
                           int launches, double* avg_us, void* stream);

@@ -4,7 +4,7 @@
 //     for every node, the sorted set of nodes that share an element with it,
 //   * the FSILS views of it (inclusive rowPtr pairs and diagPtr, lhs.cpp:95-120),
 //   * element colouring (no two elements of one colour share a node) and the
-//     element -> block-slot map that replaces do_assem's binary search
+//     face elements' block slots, which replace do_assem's binary search
 //     (lhsa.cpp:123-134) on the device.
 #include "svg_internal.h"
 

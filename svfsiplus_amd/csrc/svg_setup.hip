@@ -1,7 +1,8 @@
 // Mesh setup on the device: the block-CSR pattern of the FSILS lhs (what
 // lhsa builds, lhsa.cpp:153-380, handed to fsils_lhs_create, lhs.cpp:57-120)
-// and the element colouring, colour order and element -> block slot map the
-// assembly kernel scatters through (do_assem's search, lhsa.cpp:123-134).
+// and the element colouring, colour order and the element entries of each block
+// slot that the assembly gathers (do_assem's search, lhsa.cpp:123-134, the other
+// way round).
 //
 // Pattern: every element contributes its 16 node pairs and every node its
 // diagonal pair as a 64-bit key row * nNo + col; one radix sort and one

@@ -85,11 +85,11 @@ def device_arrays(pipe: Pipe):
 
 
 class DeviceMesh:
-    """Device-resident element data (coordinates, connectivity, colours, slot map)."""
+    """Device-resident element data (coordinates, connectivity, colours, the slots' element entries)."""
 
     def __init__(self, lhs: DeviceLhs, pipe: Pipe, d_ien=None, d_x=None):
         """With d_ien and d_x (device tensors holding pipe.IEN and pipe.x) the
-        colouring, colour order and slot map are built on the device
+        colouring, colour order and the slots' element entries are built on the device
         (svg_msh_create_dev)."""
         lib = _lib.load()
         h = C.c_void_p()
@@ -243,7 +243,7 @@ class FluidNewton:
     def __init__(self, pipe: Pipe, phys: Physics, ls: _lib.Ls, eq: EqState | None = None, device="cuda",
                  precision: int = _lib.PRECISION_FP64, lpc=None, outlet: bool = True, net_period: int = 1,
                  device_setup: bool = False, coarse: int = 0, coarse_keep: bool = False):
-        """device_setup: build the block pattern, colouring and slot map on the
+        """device_setup: build the block pattern, colouring and assembly lists on the
         device (svg_lhs_create_dev, svg_msh_create_dev) from IEN and x;
         coarse_keep: the Newton iterations after the first of a time step keep
         the coarse inverse of the first (the two-level preconditioner)."""
