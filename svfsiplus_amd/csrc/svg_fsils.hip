@@ -409,7 +409,8 @@ constexpr double FB_DROP = 1e-4;  // learned preconditioner: smallest relative d
 // Loads are unconditional (indices clamped into the span; the clamped values
 // are not used) and G columns are loaded and reduced together, so one memory
 // latency is spent per G columns (FP32 columns, half the bytes of FP64 ones,
-// need more in flight to keep HBM busy).
+// need more in flight to keep HBM busy). SHUF: wave_sum's butterfly by shuffles
+// in the one-column form (see k_mdot).
 // Basis entries of the dots. The FP32 (compressed) basis of the mixed and
 // flexible solves is streamed with non-temporal loads (and written with
 // non-temporal stores by the update): its passes then leave the memory-side
@@ -419,7 +420,7 @@ constexpr double FB_DROP = 1e-4;  // learned preconditioner: smallest relative d
 __device__ __forceinline__ float basis_load(const float* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ double basis_load(const double* p) { return *p; }
 
-template <int G, typename T, typename TWv = double>
+template <int G, bool SHUF, typename T, typename TWv>
 __device__ __forceinline__ void span_dots(const TWv* __restrict__ w, const T* __restrict__ base, size_t ld, int m,
                                           bool self, size_t k0, size_t kend, double* lds, int mc)
 {
@@ -474,7 +475,12 @@ __device__ __forceinline__ void span_dots(const TWv* __restrict__ w, const T* __
       const double v = in[r] ? (double)c[r] : 0.0;
       acc = acc + v * wr[r];
     }
-    acc = wave_sum(acc);
+    if constexpr (SHUF) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    } else {
+      acc = wave_sum(acc);
+    }
     if (lane == 0) lds[wv * mc + j] = acc;
   }
   if (self) {
@@ -506,7 +512,7 @@ static int dot_cols(int nblk, int mc, int wgs)
 // b (1024 elements [k0, kend)): 256 lanes x 4 elements at stride 256, in order,
 // butterflies inside each wavefront, the 4 wavefront sums added in order;
 // partial[j*nblk + b].
-template <int G, typename T, typename TWv>
+template <int G, bool SHUF, typename T, typename TWv>
 __device__ __forceinline__ void mdot_body(const TWv* __restrict__ w, const T* __restrict__ base, size_t ld, int m,
                                           bool self, int cols, size_t k0, size_t kend, double* __restrict__ partial,
                                           int nblk, double* lds)
@@ -514,7 +520,7 @@ __device__ __forceinline__ void mdot_body(const TWv* __restrict__ w, const T* __
 #pragma clang fp contract(off)
   const int t = threadIdx.x, j0 = blockIdx.y * cols, mc = min(m + (self ? 1 : 0) - j0, cols);
   const bool own = self && j0 + mc == m + 1;  // column m is this workgroup's last
-  span_dots<G>(w, base + (size_t)j0 * ld, ld, own ? mc - 1 : mc, own, k0 + t, kend, lds, mc);
+  span_dots<G, SHUF>(w, base + (size_t)j0 * ld, ld, own ? mc - 1 : mc, own, k0 + t, kend, lds, mc);
   __syncthreads();
   for (int j = t; j < mc; j += RED_BS) {
     double v = lds[j];
@@ -523,17 +529,23 @@ __device__ __forceinline__ void mdot_body(const TWv* __restrict__ w, const T* __
   }
 }
 
-__global__ __launch_bounds__(RED_BS) void k_mdot(int n, const double* __restrict__ w, const double* __restrict__ base,
+// G = 1 where a workgroup takes all columns, 4 where they are split: kernels of
+// their own, each with the registers of its own form. The unsplit form streams
+// the basis at what HBM gives, and there more loads in flight are slower, not
+// faster, so it keeps to four wavefronts a SIMD (its registers allow eight) and
+// to butterflies by shuffles, after which the next column's loads come later
+// than after register moves. A step of the 4.2M-tet pipe (2 865 spans): 102.9 us;
+// 111.9 with eight wavefronts, 105.0 with register moves. The 1.2M-tet pipe's
+// 819 spans make four wavefronts a SIMD at most: 31.0 us, 31.5 with register
+// moves, 32.7 with the next column's loads issued ahead of the sums.
+template <int G>
+__global__ __launch_bounds__(RED_BS) __attribute__((amdgpu_waves_per_eu(1, G == 1 ? 4 : 8))) void k_mdot(int n, const double* __restrict__ w, const double* __restrict__ base,
                                                  size_t ld, int m, int cols, double* __restrict__ partial,
                                                  const int* __restrict__ skip)
 {
   extern __shared__ double lds[];  // [RED_NW waves][cols]
   if (skip && *skip) return;
-  const size_t k0 = (size_t)blockIdx.x * RED_SPAN;
-  if (gridDim.y > 1)
-    mdot_body<4>(w, base, ld, m, false, cols, k0, (size_t)n, partial, gridDim.x, lds);
-  else
-    mdot_body<1>(w, base, ld, m, false, cols, k0, (size_t)n, partial, gridDim.x, lds);
+  mdot_body<G, G == 1>(w, base, ld, m, false, cols, (size_t)blockIdx.x * RED_SPAN, (size_t)n, partial, gridDim.x, lds);
 }
 
 // The mixed-precision solve keeps its Krylov basis in FP32 (a compressed
@@ -546,7 +558,7 @@ __global__ __launch_bounds__(RED_BS) void k_mdot_cb(int n, const TWv* __restrict
 {
   extern __shared__ double lds[];  // [RED_NW waves][cols]
   if (skip && *skip) return;
-  mdot_body<MDOT_CB_G>(w, base, ld, m, true, cols, (size_t)blockIdx.x * RED_SPAN, (size_t)n, partial, gridDim.x, lds);
+  mdot_body<MDOT_CB_G, false>(w, base, ld, m, true, cols, (size_t)blockIdx.x * RED_SPAN, (size_t)n, partial, gridDim.x, lds);
 }
 
 constexpr int FIN_BS = 1024;  // finaliser: one workgroup of 16 wavefronts
@@ -1462,8 +1474,9 @@ static int dot_device(int n, const double* w, const double* base, size_t ld, int
   const int* skip = (fa.mode == FIN_ARNOLDI) ? &st->done : nullptr;
   // algorithmic bytes: w and the m - 1 basis vectors read, the partials written; the finaliser reads them
   const int cols = dot_cols(nblk, m, DOT_WGS_F64);
-  launch_b("mdot", 8.0 * n * m + 8.0 * m * nblk, k_mdot, dim3(nblk, (m + cols - 1) / cols), dim3(RED_BS),
-           (size_t)RED_NW * cols * sizeof(double), s, n, w, base, ld, m, cols, partial, skip);
+  launch_b("mdot", 8.0 * n * m + 8.0 * m * nblk, cols < m ? k_mdot<4> : k_mdot<1>,
+           dim3(nblk, (m + cols - 1) / cols), dim3(RED_BS), (size_t)RED_NW * cols * sizeof(double), s, n, w, base, ld,
+           m, cols, partial, skip);
   launch_b("mdot_fin", 8.0 * m * nblk, k_fin, dim3(1), dim3(FIN_BS), 0, s, fa, (const double*)partial, nblk, m, st,
            h, cs, sn, err, coef, out, (volatile int*)host_done);
   return SVG_OK;
@@ -2480,7 +2493,11 @@ static int precond_diag_dev(svg_lhs* L, int dof, double* Val, double* R, double*
 // arithmetic is the single-system gmres_v's, bit for bit), and every system
 // has its own Hessenberg, Givens, state and convergence. One restart cycle of
 // all systems is captured once into a hipGraph and replayed.
-__global__ __launch_bounds__(RED_BS) void k_bmdot(const int* __restrict__ spanStart, const int* __restrict__ spanEnd,
+// As k_mdot, except that the unsplit form does as well with register moves (a
+// Newton iteration of 256 FP64 meshes: 404.4 ms, 406.2 with shuffles, 410 to 412
+// with eight wavefronts a SIMD).
+template <int G>
+__global__ __launch_bounds__(RED_BS) __attribute__((amdgpu_waves_per_eu(1, G == 1 ? 4 : 8))) void k_bmdot(const int* __restrict__ spanStart, const int* __restrict__ spanEnd,
                                                   const int* __restrict__ spanSys, int nsp,
                                                   const double* __restrict__ w, const double* __restrict__ base,
                                                   size_t ld, int m, int cols, double* __restrict__ partial,
@@ -2492,10 +2509,7 @@ __global__ __launch_bounds__(RED_BS) void k_bmdot(const int* __restrict__ spanSt
     const GmState& S = st[spanSys[b]];
     if (!S.act || (check == 2 && S.done)) return;
   }
-  if (gridDim.y > 1)
-    mdot_body<4>(w, base, ld, m, false, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
-  else
-    mdot_body<1>(w, base, ld, m, false, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
+  mdot_body<G, false>(w, base, ld, m, false, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
 }
 
 // k_mdot_cb per span of the batched solve (FP32 basis, then w.w as column m).
@@ -2509,7 +2523,7 @@ __global__ __launch_bounds__(RED_BS) void k_bmdot_cb(const int* __restrict__ spa
   const int b = blockIdx.x;
   const GmState& S = st[spanSys[b]];
   if (!S.act || S.done) return;
-  mdot_body<MDOT_CB_G>(w, base, ld, m, true, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
+  mdot_body<MDOT_CB_G, false>(w, base, ld, m, true, cols, (size_t)spanStart[b], (size_t)spanEnd[b], partial, nsp, lds);
 }
 
 // The FP32 SpMV of the batched solve: rows of systems that converged or
@@ -2807,7 +2821,7 @@ static void batch_graph_free(svg_batch* B)
 static void batch_mdot(svg_batch* B, const double* w, const double* base, size_t ld, int m, int check, hipStream_t s)
 {
   const int cols = dot_cols(B->nsp, m, DOT_WGS_F64);
-  hipLaunchKernelGGL(k_bmdot, dim3(B->nsp, (m + cols - 1) / cols), dim3(RED_BS),
+  hipLaunchKernelGGL(cols < m ? k_bmdot<4> : k_bmdot<1>, dim3(B->nsp, (m + cols - 1) / cols), dim3(RED_BS),
                      (size_t)RED_NW * cols * sizeof(double), s, (const int*)B->d_spanStart, (const int*)B->d_spanEnd,
                      (const int*)B->d_spanSys, B->nsp, w, base, ld, m, cols, B->partial, (const GmState*)B->st, check);
 }
