@@ -397,6 +397,22 @@ int svg_spmv32(const svg_lhs* lhs, const float* d_K32, const float* d_U32, doubl
 int svg_spmv32_tune(svg_lhs* lhs, const float* d_K32, float* d_U32, double* d_KU, int* best_variant, void* stream);
 /* The launch variants the autotuners picked for lhs (-1: not tuned yet). */
 int svg_spmv_variants(const svg_lhs* lhs, int* fp64_variant, int* fp32_variant);
+/* Small systems' restart cycles and Schur CG as one launch each (no
+ * counterpart in the reference): which solves of lhs took that path. gmres,
+ * cg: solves that ran so; cg_rows: rows of a workgroup of the CG (0 not looked
+ * at yet, -1 the system does not fit); missed: launches whose workgroups did
+ * not all meet at a barrier within its bounded wait, or that were refused. A
+ * solve that missed is done again by the launches of larger systems, with the
+ * same result, and so are the lhs's later ones. */
+typedef struct {
+  long long gmres, cg;
+  int cg_rows, missed;
+} svg_one_launch;
+int svg_one_launch_info(const svg_lhs* lhs, svg_one_launch* info);
+/* on: whether lhs's solves may take the path (also after a miss); polls: the
+ * bounded wait, in looks at the barrier (0.7 us each; negative: the default,
+ * 2^20). A new lhs has (1, -1). */
+int svg_one_launch_set(svg_lhs* lhs, int on, int polls);
 /* precond_diag (precond.cpp:122-257) with every registered face included. */
 int svg_precond_diag(svg_lhs* lhs, int dof, double* d_Val, double* d_R, double* d_W, void* stream);
 /* fsils_dot_v / fsi_ls_normv (dot.cpp:69-117, norm.cpp:67-112); blocking. */

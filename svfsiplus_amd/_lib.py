@@ -62,6 +62,10 @@ class SolveOpts(C.Structure):
                 ("lpc", C.c_void_p)]
 
 
+class OneLaunch(C.Structure):
+    _fields_ = [("gmres", C.c_longlong), ("cg", C.c_longlong), ("cg_rows", C.c_int), ("missed", C.c_int)]
+
+
 PRECISION_FP64, PRECISION_MIXED = 0, 1
 COARSE_APPLY, COARSE_RESIDUAL, COARSE_SMOOTH = 0, 1, 2
 METHOD_PLAIN, METHOD_LEARNED = 0, 1
@@ -107,6 +111,8 @@ _SIGS = {
     "svg_fsils_solve": (_I, [_P, C.POINTER(Ls), _I, _P, _P, _I, _I, _P, _P, _P]),
     "svg_fsils_solve_ex": (_I, [_P, C.POINTER(Ls), _I, _P, _P, _I, _I, _P, _P, C.POINTER(SolveOpts), _P]),
     "svg_spar_mul_vv": (_I, [_P, _I, _P, _P, _P, _P]),
+    "svg_one_launch_info": (_I, [_P, C.POINTER(OneLaunch)]),
+    "svg_one_launch_set": (_I, [_P, _I, _I]),
     "svg_precond_diag": (_I, [_P, _I, _P, _P, _P, _P]),
     "svg_spmv32": (_I, [_P, _P, _P, _P, _P]),
     "svg_spmv32_tune": (_I, [_P, _P, _P, _P, _IP, _P]),

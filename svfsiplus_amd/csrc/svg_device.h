@@ -323,6 +323,9 @@ struct svg_lhs {
   svg::KrylovWork kw;    // gmres_v on the 4x4 system
   svg::KrylovWork kw3;   // inner GMRES of the NS solver on the 3x3 momentum block
   svg::NsWork ns;
+  bool oneLaunch = true;         // small systems' solves may run as one launch (off after a miss)
+  int oneLaunchPolls = -1;       // its barriers' bounded wait (negative: the default)
+  svg_one_launch oneLaunchRuns{};  // solves that took that path, and misses
 };
 
 // Batched GMRES over a block-diagonal union of independent systems (one lhs

@@ -10,7 +10,8 @@
 // (vmcnt 0) before the barrier's arrival, and loads past the barrier. The
 // barrier's wait is bounded: if the workgroups do not meet, each leaves and
 // flags it, and the host takes the per-launch path, whose inputs a kernel here
-// never overwrites before its last barrier.
+// never overwrites before its last barrier. The lhs's later solves go there
+// straight away: a wait that ran out took most of a second.
 #include "svg_device.h"
 
 #include <algorithm>
@@ -20,7 +21,7 @@ namespace svg {
 
 namespace {
 
-constexpr int SPIN_MAX = 1 << 20;  // polls of about 0.7 us
+constexpr int SPIN_MAX = 1 << 20;  // polls of about 0.7 us (svg_one_launch_set changes it)
 
 __device__ __forceinline__ double ld_agent(const double* p)
 {
@@ -45,15 +46,15 @@ struct AgentBuf {
   }
 };
 
-// All workgroups of the launch meet; false: they did not within SPIN_MAX polls.
-__device__ __forceinline__ bool grid_sync(int* ctr, int& target, int* ok)
+// All workgroups of the launch meet; false: they did not within `polls` polls.
+__device__ __forceinline__ bool grid_sync(int* ctr, int& target, int* ok, int polls)
 {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   target += gridDim.x;
   if (threadIdx.x == 0) {
     int c = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-    for (int n = 0; c < target && n < SPIN_MAX; n++)
+    for (int n = 0; c < target && n < polls; n++)
       c = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *ok = c >= target;
   }
@@ -140,8 +141,8 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
                                                     const double* __restrict__ Gt, const double* __restrict__ mL,
                                                     const double* __restrict__ R0, double* __restrict__ X, double* pr,
                                                     double* gpp, double* prod, double* rc, CgState* cg, int* ctr,
-                                                    int rows, int cap, int capU, int mItr, double absTol,
-                                                    double relTol)
+                                                    int rows, int cap, int capU, int polls, int mItr,
+                                                    double absTol, double relTol)
 {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
     suc = 1;
     stop = true;
   }
-  bool ok = grid_sync(ctr, target, &okf);
+  bool ok = grid_sync(ctr, target, &okf, polls);
   double c1 = 0.0, c2 = 0.0;
   for (int i = 0; ok && !stop && mItr > 0; i++) {
     // 1: the listed columns' P and R (the first two per lane on their way while
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
       st_agent(o + 2, g2);
       st_agent(o + 3, P);
     }
-    if (!(ok = grid_sync(ctr, target, &okf))) break;
+    if (!(ok = grid_sync(ctr, target, &okf, polls))) break;
     // 2: SP = L P - G^T GP
     for (int q = t; q < nu; q += CG_BS) {
       const double2 x = bgp.ld2(32 * list[q]), y = bgp.ld2(32 * list[q] + 16);
@@ -289,7 +290,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
       sp = sp + (-1.0) * dgp;
       st_agent(prod + row, P * sp);
     }
-    if (!(ok = grid_sync(ctr, target, &okf))) break;
+    if (!(ok = grid_sync(ctr, target, &okf, polls))) break;
     // 3: alpha, X and R
     const double alpha = errO / sum_all(nNo, ws, [&](int k) { return ld_agent(prod + k); });
     if (own) {
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
       st_agent(pr + 2 * (size_t)row + 1, R);
       st_agent(rc + row, R);
     }
-    ok = grid_sync(ctr, target, &okf);
+    ok = grid_sync(ctr, target, &okf, polls);
   }
   if (own) X[row] = Xr;
   if (t == 0) {
@@ -339,7 +340,7 @@ constexpr int GM_PF = 24;
 constexpr int GM_BLK_B = 16 * 8 + 2, GM_COL_B = 4 + 32;  // LDS bytes per block and per listed column
 
 struct GmSmall {
-  int nNo, sD, cap, capU, cycles;
+  int nNo, sD, cap, capU, cycles, polls;
   const int *rowPtr, *colPtr;
   const double *K, *R;
   double *X, *u, *ex, *part, *h, *y;
@@ -457,7 +458,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
     fPrev = fNorm;
     // u_0 = (R - A X) / |R - A X|
     if (own) st_agent(A.ex + k, x);
-    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
     double v = rhs - product(0);
     if (wv < 4) wl[wv][lane] = own ? v : 0.0;
     __syncthreads();
@@ -467,7 +468,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
       for (int r = 0; r < 4; r++) a = a + wl[r][lane] * wl[r][lane];
       put_part(0, wave_sum(a));
     }
-    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
     {
       const int c = 32 * min(lane, nblk - 1);
       const double e0 = sqrt(finish(bpart.ld2(c), bpart.ld2(c + 16)));
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
       st_agent(A.ex + n + k, v);
     }
     if (t == 0) stopf = 0;
-    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
     int i = 0;
     for (;; i++) {
       // the share's entries of u_0 .. u_i for the dots, column wv + 4 q, on their
@@ -536,7 +537,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
         pv[q] = 0.0;
         if (wv < 4 && q <= i) pv[q] = A.u[(size_t)q * A.ld + min(k, n - 1)];
       }
-      if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+      if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
       for (int c = wv; wv < 4 && c <= i + 1; c += 16) {
         double2 p0[4], p1[4];
 #pragma unroll
@@ -605,7 +606,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
           st_agent(A.ex + (size_t)(i & 1) * n + k, z);
         }
       }
-      ok = grid_sync(A.ctr, target, &okf);
+      ok = grid_sync(A.ctr, target, &okf, A.polls);
       itr++;
       if (blockIdx.x == 0) {
         // column i of the triangle and err(i), for the back substitution
@@ -653,7 +654,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
       }
       for (int j = lane; j <= last_i; j += 64) st_agent(A.y + GM_MAX + j, y[j]);
     }
-    if (!(ok = grid_sync(A.ctr, target, &okf))) break;
+    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
     for (int j = t; j <= last_i; j += GM_BS) sums[j] = ld_agent(A.y + GM_MAX + j);
     __syncthreads();
     for (int jq = 0; jq <= last_i; jq += 8) {
@@ -699,6 +700,17 @@ __global__ void k_clear_small(int* ctr, int* flag)
   *flag = 0;
 }
 
+int polls_of(const svg_lhs* L) { return L->oneLaunchPolls < 0 ? SPIN_MAX : L->oneLaunchPolls; }
+
+// No memory for its buffers, the launch refused, or its workgroups did not meet:
+// the per-launch path, for the lhs's later solves too.
+int missed(svg_lhs* L)
+{
+  L->oneLaunch = false;
+  L->oneLaunchRuns.missed++;
+  return SVG_OK;
+}
+
 }  // namespace
 
 // The most blocks of a group of `rows` consecutive rows.
@@ -717,7 +729,7 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
 {
   auto& w = L->ns;
   *ran = 0;
-  if (w.smallRows < 0) return SVG_OK;
+  if (!L->oneLaunch || w.smallRows < 0) return SVG_OK;
   const int nNo = L->nNo;
   int rc;
   auto bytes = [&](int cap) {
@@ -736,29 +748,35 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
         (void)hipGetLastError();
         return SVG_OK;
       }
-      if ((rc = dev_alloc(&w.cgEx, (size_t)8 * nNo)) || (rc = dev_alloc(&w.ctr, 1))) return rc;
+      if (dev_alloc(&w.cgEx, (size_t)8 * nNo) || dev_alloc(&w.ctr, 1)) {
+        dev_free(w.cgEx);
+        (void)hipGetLastError();
+        return missed(L);
+      }
       w.smallRows = rows;
       w.smallCap = cap;
       break;
     }
     if (w.smallRows < 0) return SVG_OK;
   }
-  int rows = w.smallRows, cap = w.smallCap, capU = std::min(cap, nNo), n = nNo;
+  int rows = w.smallRows, cap = w.smallCap, capU = std::min(cap, nNo), n = nNo, polls = polls_of(L);
   hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, w.ctr, &w.cg->pad);
   const int *rp = L->d_rowPtr, *cp = L->d_colPtr;
   const double *mG = w.mG, *Gt = w.Gt, *mL = w.mL;
   double *X = w.cgX, *gpp = w.cgEx, *pr = w.cgEx + (size_t)4 * nNo, *prod = w.cgEx + (size_t)6 * nNo,
          *rcv = w.cgEx + (size_t)7 * nNo;
   void* args[] = {&n,    &rp,   &cp,   &mG,    &Gt,  &mL,   &R,    &X,    &pr,     &gpp,
-                  &prod, &rcv,  &w.cg, &w.ctr, &rows, &cap, &capU, &mItr, &absTol, &relTol};
+                  &prod, &rcv,  &w.cg, &w.ctr, &rows, &cap, &capU, &polls, &mItr, &absTol, &relTol};
   if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_cg_small), dim3(blocks_for(nNo, rows)), dim3(CG_BS),
                                  args, (unsigned)bytes(cap), s) != hipSuccess) {
-    (void)hipGetLastError();  // not launched: the per-launch path
-    return SVG_OK;
+    (void)hipGetLastError();
+    return missed(L);
   }
   SVG_HIP(hipMemcpyAsync(w.h_cg, w.cg, sizeof(CgState), hipMemcpyDeviceToHost, s));
   SVG_HIP(hipStreamSynchronize(s));
-  *ran = w.h_cg->pad ? 0 : 1;
+  if (w.h_cg->pad) return missed(L);
+  *ran = 1;
+  L->oneLaunchRuns.cg++;
   return SVG_OK;
 }
 
@@ -773,6 +791,7 @@ constexpr int GM_LDS = 149 * 1024;  // of 160 KB, 10 KB are the kernel's own arr
 bool gmres_small_fits(svg_lhs* L, int sD)
 {
   auto& k = L->kw;
+  if (!L->oneLaunch) return false;
   if (k.smallCap == 0) {
     k.smallCap = -1;
     const int nNo = L->nNo, nblk = (4 * nNo + 1023) / 1024;
@@ -808,12 +827,14 @@ int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double
   *ran = 0;
   const int n = k.n, nblk = (n + 1023) / 1024;
   const size_t nPart = (size_t)4 * nblk * (k.sD + 1);
-  int rc;
-  if (!k.small && (rc = dev_alloc(&k.small, nPart + 2 * (size_t)n + 2 * GM_MAX))) return rc;
-  if (!k.ctr && (rc = dev_alloc(&k.ctr, 1))) return rc;
+  if ((!k.small && dev_alloc(&k.small, nPart + 2 * (size_t)n + 2 * GM_MAX)) || (!k.ctr && dev_alloc(&k.ctr, 1))) {
+    (void)hipGetLastError();
+    return missed(L);
+  }
   GmSmall A{};
   A.nNo = L->nNo;
   A.sD = ls->sD;
+  A.polls = polls_of(L);
   A.cap = k.smallCap;
   A.capU = k.smallCapU;
   A.rowPtr = L->d_rowPtr;
@@ -836,17 +857,36 @@ int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double
     void* args[] = {&A};
     if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_gmres_small), dim3(4 * nblk), dim3(GM_BS), args,
                                    bytes, s) != hipSuccess) {
-      (void)hipGetLastError();  // not launched: the per-launch path
-      return SVG_OK;
+      (void)hipGetLastError();
+      return missed(L);
     }
     SVG_HIP(hipMemcpyAsync(k.h_st, k.st, sizeof(GmState), hipMemcpyDeviceToHost, s));
     SVG_HIP(hipStreamSynchronize(s));
-    if (k.h_st->pad) return SVG_OK;
+    if (k.h_st->pad) return missed(L);
     done += A.cycles;
     if (k.h_st->suc || k.h_st->divzero) break;
   }
   *ran = 1;
+  L->oneLaunchRuns.gmres++;
   return SVG_OK;
 }
 
 }  // namespace svg
+
+using namespace svg;
+
+extern "C" int svg_one_launch_info(const svg_lhs* L, svg_one_launch* info)
+{
+  if (!L || !info) return set_error(SVG_ERR_ARG, "svg_one_launch_info: null argument");
+  *info = L->oneLaunchRuns;
+  info->cg_rows = L->ns.smallRows;
+  return SVG_OK;
+}
+
+extern "C" int svg_one_launch_set(svg_lhs* L, int on, int polls)
+{
+  if (!L) return set_error(SVG_ERR_ARG, "svg_one_launch_set: null lhs");
+  L->oneLaunch = on != 0;
+  L->oneLaunchPolls = polls;
+  return SVG_OK;
+}

@@ -226,6 +226,14 @@ def test_gmres_solve(torch_cuda, phys, n):
     assert rel <= 10 * tol
 
 
+def _one_launch(L):
+    """The lhs's solves that ran as one launch (GMRES, Schur CG) and the misses."""
+    import ctypes as C
+    info = _lib.OneLaunch()
+    _lib.call("svg_one_launch_info", L.h, C.byref(info))
+    return info.gmres, info.cg, info.missed
+
+
 @pytest.mark.parametrize("n,nz,sD,cycles", [(2, 3, 50, 1000), (4, 9, 1, 40), (4, 20, 250, 1000), (6, 11, 100, 3),
                                             (10, 24, 50, 1000), (12, 61, 50, 20)])
 def test_gmres_one_launch_cycles(torch_cuda, phys, n, nz, sD, cycles):
@@ -251,6 +259,38 @@ def test_gmres_one_launch_cycles(torch_cuda, phys, n, nz, sD, cycles):
         assert (ls.RI.itr, ls.RI.suc, ls.RI.iNorm, ls.RI.fNorm) == (ols.RI.itr, ols.RI.suc, ols.RI.iNorm, ols.RI.fNorm)
         assert abs(ls.RI.dB - ols.RI.dB) <= 1e-12 * abs(ols.RI.dB)
         assert np.array_equal(dR.cpu().numpy(), x0)
+    assert _one_launch(L) == (2, 0, 0)
+
+
+@pytest.mark.parametrize("how", ["off", "missed"])
+@pytest.mark.parametrize("n,nz", [(4, 9), (10, 24)])
+def test_gmres_small_by_launches(torch_cuda, phys, n, nz, how):
+    """gmres_v of a small system without the one launch per cycles: switched off,
+    and given up because the workgroups found no one at their first barrier (a
+    wait of no polls; the solve after it takes the launches at once). Bit for bit
+    the device-order oracle."""
+    from svfsiplus_amd.newton import DeviceLhs, fsils_solve, ls_create
+    torch = torch_cuda
+    p = W.make_pipe(n, nz=nz)
+    Ag, Yg = _state(p, phys, seed=n)
+    R, V = oracle.construct_fluid(p, phys, Ag, Yg)
+    with oracle.device_order():
+        x0, _, ols = oracle.fsils_solve(
+            p, oracle.ls_create(oracle.LS_GMRES, relTol=1e-6, absTol=1e-30, maxItr=40, dimKry=50), R, V)
+    ls = ls_create(_lib.LS_GMRES, relTol=1e-6, absTol=1e-30, maxItr=40, dimKry=50)
+    L = DeviceLhs(p)
+    _lib.call("svg_one_launch_set", L.h, 0 if how == "off" else 1, 0)
+    for _ in range(2):
+        dR, dV = _dev(torch, R), _dev(torch, V)
+        fsils_solve(L, ls, 4, dR, dV)
+        assert (ls.RI.itr, ls.RI.suc, ls.RI.iNorm, ls.RI.fNorm) == (ols.RI.itr, ols.RI.suc, ols.RI.iNorm, ols.RI.fNorm)
+        assert np.array_equal(dR.cpu().numpy(), x0)
+        assert _one_launch(L) == (0, 0, 0 if how == "off" else 1)
+    _lib.call("svg_one_launch_set", L.h, 1, -1)  # on again
+    dR, dV = _dev(torch, R), _dev(torch, V)
+    fsils_solve(L, ls, 4, dR, dV)
+    assert np.array_equal(dR.cpu().numpy(), x0)
+    assert _one_launch(L)[0] == 1
 
 
 @pytest.mark.parametrize("n,nz,sD", [(16, 60, 50), (24, 125, 27), (28, 125, 18)])
@@ -447,14 +487,19 @@ def test_coupled_ns_solver(torch_cuda):
     assert rel <= 1e-2
 
 
+@pytest.mark.parametrize("how", ["one launch", "off", "missed"])
 @pytest.mark.parametrize("n,nz", [(2, 3), (4, 7), (12, 30), (16, 40)])
-def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz):
-    """The NS solver where its Schur CG runs as one launch: less than one
-    workgroup's rows, a ragged last one, 6 and 12 reduction spans (four are
-    summed at a time); bit for bit the device-order oracle, counts and all."""
+def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz, how):
+    """The NS solver with its Schur CG as one launch (less than one workgroup's
+    rows, a ragged last one, 6 and 12 reduction spans, four of which are summed at
+    a time), by the launches of larger systems, and by those after the first CG's
+    workgroups found no one at their barrier (a wait of no polls): bit for bit
+    the device-order oracle, counts and all."""
     from svfsiplus_amd.newton import DeviceLhs, fsils_solve
     import ctypes as C
     torch = torch_cuda
+    if how == "missed" and n == 2:
+        pytest.skip("a single workgroup always meets itself")
     p = W.make_pipe(n, nz=nz)
     Ag, Yg = _state(p, phys, seed=n)
     R, V = oracle.construct_fluid(p, phys, Ag, Yg)
@@ -462,12 +507,17 @@ def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz):
     ls = _lib.Ls()
     C.memmove(C.byref(ls), C.byref(ols), C.sizeof(ls))
     dR, dV = _dev(torch, R), _dev(torch, V)
-    fsils_solve(DeviceLhs(p), ls, 4, dR, dV)
+    L = DeviceLhs(p)
+    if how != "one launch":
+        _lib.call("svg_one_launch_set", L.h, 0 if how == "off" else 1, 0)
+    fsils_solve(L, ls, 4, dR, dV)
     with oracle.device_order():
         x0, _, ols = oracle.fsils_solve(p, ols, R, V)
     assert (ls.RI.itr, ls.GM.itr, ls.CG.itr, ls.CG.suc) == (ols.RI.itr, ols.GM.itr, ols.CG.itr, ols.CG.suc)
     assert (ls.RI.fNorm, ls.CG.fNorm, ls.CG.iNorm) == (ols.RI.fNorm, ols.CG.fNorm, ols.CG.iNorm)
     assert np.array_equal(dR.cpu().numpy(), x0)
+    # one CG in each of the two outer iterations; after a miss none tries again
+    assert _one_launch(L) == (0, 2 if how == "one launch" else 0, 1 if how == "missed" else 0)
 
 
 @pytest.mark.parametrize("name", ["pipe_n2", "pipe_n4"])
