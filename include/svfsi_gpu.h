@@ -455,7 +455,9 @@ int svg_fill(double* d, size_t n, double v, void* stream);
 /* ------------------------------------------------------------------------ */
 /* Kernel timing with HIP events on the launching stream.                    */
 /* When enabled, every launch of the named kernels is bracketed by events;   */
-/* svg_prof_get returns the launch count and summed duration (ms).           */
+/* svg_prof_get returns the launch count and summed duration (ms). A small   */
+/* system's solve shows as "gmres_small" (up to 16 restart cycles a launch)  */
+/* and "cg_small" (a whole Schur CG) in place of its steps' kernels.         */
 int svg_prof_enable(int on);
 /* Restricts the event timing to the kernels named in the comma-separated
  * list (NULL or "": every named kernel). Events cost time between launches,

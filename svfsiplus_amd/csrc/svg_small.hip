@@ -700,6 +700,23 @@ __global__ void k_clear_small(int* ctr, int* flag)
   *flag = 0;
 }
 
+// A cooperative launch, timed by events around it (the launch has no event
+// arguments of its own: a few microseconds of dispatch are timed with it).
+hipError_t launch_cooperative(const char* name, const void* kernel, unsigned grid, unsigned block, void** args,
+                              unsigned lds, hipStream_t s)
+{
+  hipEvent_t a = nullptr, b = nullptr;
+  const size_t mark = prof_mark();
+  const bool timed = prof_begin(name, s, 0.0, &a, &b) >= 0;
+  if (timed) (void)hipEventRecord(a, s);
+  const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(block), args, lds, s);
+  if (timed && e == hipSuccess)
+    (void)hipEventRecord(b, s);
+  else if (timed)
+    prof_drop(mark, mark + 1);
+  return e;
+}
+
 int polls_of(const svg_lhs* L) { return L->oneLaunchPolls < 0 ? SPIN_MAX : L->oneLaunchPolls; }
 
 // No memory for its buffers, the launch refused, or its workgroups did not meet:
@@ -767,8 +784,8 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
          *rcv = w.cgEx + (size_t)7 * nNo;
   void* args[] = {&n,    &rp,   &cp,   &mG,    &Gt,  &mL,   &R,    &X,    &pr,     &gpp,
                   &prod, &rcv,  &w.cg, &w.ctr, &rows, &cap, &capU, &polls, &mItr, &absTol, &relTol};
-  if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_cg_small), dim3(blocks_for(nNo, rows)), dim3(CG_BS),
-                                 args, (unsigned)bytes(cap), s) != hipSuccess) {
+  if (launch_cooperative("cg_small", reinterpret_cast<const void*>(&k_cg_small), blocks_for(nNo, rows), CG_BS, args,
+                         (unsigned)bytes(cap), s) != hipSuccess) {
     (void)hipGetLastError();
     return missed(L);
   }
@@ -855,8 +872,8 @@ int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double
     A.cycles = std::min(GM_CYCLES, ls->mItr - done);
     hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, k.ctr, &k.st->pad);
     void* args[] = {&A};
-    if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_gmres_small), dim3(4 * nblk), dim3(GM_BS), args,
-                                   bytes, s) != hipSuccess) {
+    if (launch_cooperative("gmres_small", reinterpret_cast<const void*>(&k_gmres_small), 4 * nblk, GM_BS, args, bytes,
+                           s) != hipSuccess) {
       (void)hipGetLastError();
       return missed(L);
     }

@@ -520,6 +520,36 @@ def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz, how):
     assert _one_launch(L) == (0, 2 if how == "one launch" else 0, 1 if how == "missed" else 0)
 
 
+def test_one_launch_solves_are_timed(torch_cuda, phys):
+    """Event timing sees the solves that run as one launch: a launch per 16
+    restart cycles of gmres_v, and one per Schur CG."""
+    import ctypes as C
+    import time
+    from svfsiplus_amd.newton import DeviceLhs, fsils_solve, ls_create
+    torch = torch_cuda
+    p = W.make_pipe(4, nz=20)
+    R, V = oracle.construct_fluid(p, phys, *_state(p, phys, seed=4))
+    L, lib = DeviceLhs(p), _lib.load()
+    ls = ls_create(_lib.LS_GMRES, relTol=1e-12, absTol=1e-30, maxItr=20, dimKry=2)
+    ns = _lib.Ls()
+    _lib.call("svg_ls_create", C.byref(ns), _lib.LS_NS)
+    for name, q, launches in (("gmres_small", ls, 2), ("cg_small", ns, None)):
+        fsils_solve(L, q, 4, _dev(torch, R), _dev(torch, V))
+        before = _one_launch(L)[1]
+        lib.svg_prof_reset()
+        lib.svg_prof_enable(1)
+        t = time.perf_counter()
+        fsils_solve(L, q, 4, _dev(torch, R), _dev(torch, V))
+        t = time.perf_counter() - t
+        lib.svg_prof_enable(0)
+        n, ms = C.c_int(), C.c_double()
+        lib.svg_prof_get(name.encode(), C.byref(n), C.byref(ms))
+        print(f"{name}: {n.value} launches, {ms.value:.3f} of {1e3 * t:.3f} ms")
+        assert n.value == (launches or _one_launch(L)[1] - before) > 0
+        assert 0.0 < ms.value < 1e3 * t
+    lib.svg_prof_reset()
+
+
 @pytest.mark.parametrize("name", ["pipe_n2", "pipe_n4"])
 def test_ns_solver_against_reference_golden(torch_cuda, name):
     """Bipartitioned NS solver (ns_solver.cpp) on the device against the reference's record."""
