@@ -409,10 +409,10 @@ typedef struct {
   int cg_rows, missed;
 } svg_one_launch;
 int svg_one_launch_info(const svg_lhs* lhs, svg_one_launch* info);
-/* on: whether lhs's solves may take the path (also after a miss); polls: the
- * bounded wait, in looks at the barrier (0.7 us each; negative: the default,
- * 2^20). A new lhs has (1, -1). */
-int svg_one_launch_set(svg_lhs* lhs, int on, int polls);
+/* on: whether lhs's solves may take the path (also after a miss); wait: whether
+ * its barriers wait (up to 2^20 looks of about 0.7 us) or give up at once, so
+ * that a launch of several workgroups misses. A new lhs has (1, 1). */
+int svg_one_launch_set(svg_lhs* lhs, int on, int wait);
 /* precond_diag (precond.cpp:122-257) with every registered face included. */
 int svg_precond_diag(svg_lhs* lhs, int dof, double* d_Val, double* d_R, double* d_W, void* stream);
 /* fsils_dot_v / fsi_ls_normv (dot.cpp:69-117, norm.cpp:67-112); blocking. */

@@ -324,7 +324,7 @@ struct svg_lhs {
   svg::KrylovWork kw3;   // inner GMRES of the NS solver on the 3x3 momentum block
   svg::NsWork ns;
   bool oneLaunch = true;         // small systems' solves may run as one launch (off after a miss)
-  int oneLaunchPolls = -1;       // its barriers' bounded wait (negative: the default)
+  bool oneLaunchWait = true;     // its barriers wait (bounded); false: they give up at once
   svg_one_launch oneLaunchRuns{};  // solves that took that path, and misses
 };
 

@@ -21,7 +21,10 @@ namespace svg {
 
 namespace {
 
-constexpr int SPIN_MAX = 1 << 20;  // polls of about 0.7 us (svg_one_launch_set changes it)
+// Most polls of a barrier, about 0.7 us each. The kernels' other form does not
+// wait at all, so that giving up can be tested; the limit as an argument takes a
+// register that k_gmres_small does not have (0.5 % of a Newton iteration).
+constexpr int SPIN_MAX = 1 << 20;
 
 __device__ __forceinline__ double ld_agent(const double* p)
 {
@@ -46,15 +49,16 @@ struct AgentBuf {
   }
 };
 
-// All workgroups of the launch meet; false: they did not within `polls` polls.
-__device__ __forceinline__ bool grid_sync(int* ctr, int& target, int* ok, int polls)
+// All workgroups of the launch meet; false: they did not within SPIN polls.
+template <int SPIN>
+__device__ __forceinline__ bool grid_sync(int* ctr, int& target, int* ok)
 {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   target += gridDim.x;
   if (threadIdx.x == 0) {
     int c = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-    for (int n = 0; c < target && n < polls; n++)
+    for (int n = 0; c < target && n < SPIN; n++)
       c = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *ok = c >= target;
   }
@@ -136,12 +140,13 @@ constexpr int CG_BS = 256;
 // id and up to four values), and of the column bitmap
 constexpr int CG_BLK_B = 7 * 8 + 2, CG_COL_B = 4 + 32;
 
+template <int SPIN>
 __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restrict__ rowPtr,
                                                     const int* __restrict__ colPtr, const double* __restrict__ mG,
                                                     const double* __restrict__ Gt, const double* __restrict__ mL,
                                                     const double* __restrict__ R0, double* __restrict__ X, double* pr,
                                                     double* gpp, double* prod, double* rc, CgState* cg, int* ctr,
-                                                    int rows, int cap, int capU, int polls, int mItr,
+                                                    int rows, int cap, int capU, int mItr,
                                                     double absTol, double relTol)
 {
 #pragma clang fp contract(off)
@@ -218,7 +223,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
     suc = 1;
     stop = true;
   }
-  bool ok = grid_sync(ctr, target, &okf, polls);
+  bool ok = grid_sync<SPIN>(ctr, target, &okf);
   double c1 = 0.0, c2 = 0.0;
   for (int i = 0; ok && !stop && mItr > 0; i++) {
     // 1: the listed columns' P and R (the first two per lane on their way while
@@ -268,7 +273,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
       st_agent(o + 2, g2);
       st_agent(o + 3, P);
     }
-    if (!(ok = grid_sync(ctr, target, &okf, polls))) break;
+    if (!(ok = grid_sync<SPIN>(ctr, target, &okf))) break;
     // 2: SP = L P - G^T GP
     for (int q = t; q < nu; q += CG_BS) {
       const double2 x = bgp.ld2(32 * list[q]), y = bgp.ld2(32 * list[q] + 16);
@@ -290,7 +295,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
       sp = sp + (-1.0) * dgp;
       st_agent(prod + row, P * sp);
     }
-    if (!(ok = grid_sync(ctr, target, &okf, polls))) break;
+    if (!(ok = grid_sync<SPIN>(ctr, target, &okf))) break;
     // 3: alpha, X and R
     const double alpha = errO / sum_all(nNo, ws, [&](int k) { return ld_agent(prod + k); });
     if (own) {
@@ -300,7 +305,7 @@ __global__ __launch_bounds__(CG_BS) void k_cg_small(int nNo, const int* __restri
       st_agent(pr + 2 * (size_t)row + 1, R);
       st_agent(rc + row, R);
     }
-    ok = grid_sync(ctr, target, &okf, polls);
+    ok = grid_sync<SPIN>(ctr, target, &okf);
   }
   if (own) X[row] = Xr;
   if (t == 0) {
@@ -340,7 +345,7 @@ constexpr int GM_PF = 24;
 constexpr int GM_BLK_B = 16 * 8 + 2, GM_COL_B = 4 + 32;  // LDS bytes per block and per listed column
 
 struct GmSmall {
-  int nNo, sD, cap, capU, cycles, polls;
+  int nNo, sD, cap, capU, cycles;
   const int *rowPtr, *colPtr;
   const double *K, *R;
   double *X, *u, *ex, *part, *h, *y;
@@ -349,6 +354,7 @@ struct GmSmall {
   int* ctr;
 };
 
+template <int SPIN>
 __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
 {
 #pragma clang fp contract(off)
@@ -458,7 +464,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
     fPrev = fNorm;
     // u_0 = (R - A X) / |R - A X|
     if (own) st_agent(A.ex + k, x);
-    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
+    if (!(ok = grid_sync<SPIN>(A.ctr, target, &okf))) break;
     double v = rhs - product(0);
     if (wv < 4) wl[wv][lane] = own ? v : 0.0;
     __syncthreads();
@@ -468,7 +474,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
       for (int r = 0; r < 4; r++) a = a + wl[r][lane] * wl[r][lane];
       put_part(0, wave_sum(a));
     }
-    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
+    if (!(ok = grid_sync<SPIN>(A.ctr, target, &okf))) break;
     {
       const int c = 32 * min(lane, nblk - 1);
       const double e0 = sqrt(finish(bpart.ld2(c), bpart.ld2(c + 16)));
@@ -485,7 +491,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
       st_agent(A.ex + n + k, v);
     }
     if (t == 0) stopf = 0;
-    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
+    if (!(ok = grid_sync<SPIN>(A.ctr, target, &okf))) break;
     int i = 0;
     for (;; i++) {
       // the share's entries of u_0 .. u_i for the dots, column wv + 4 q, on their
@@ -537,7 +543,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
         pv[q] = 0.0;
         if (wv < 4 && q <= i) pv[q] = A.u[(size_t)q * A.ld + min(k, n - 1)];
       }
-      if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
+      if (!(ok = grid_sync<SPIN>(A.ctr, target, &okf))) break;
       for (int c = wv; wv < 4 && c <= i + 1; c += 16) {
         double2 p0[4], p1[4];
 #pragma unroll
@@ -606,7 +612,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
           st_agent(A.ex + (size_t)(i & 1) * n + k, z);
         }
       }
-      ok = grid_sync(A.ctr, target, &okf, A.polls);
+      ok = grid_sync<SPIN>(A.ctr, target, &okf);
       itr++;
       if (blockIdx.x == 0) {
         // column i of the triangle and err(i), for the back substitution
@@ -654,7 +660,7 @@ __global__ __launch_bounds__(GM_BS) void k_gmres_small(GmSmall A)
       }
       for (int j = lane; j <= last_i; j += 64) st_agent(A.y + GM_MAX + j, y[j]);
     }
-    if (!(ok = grid_sync(A.ctr, target, &okf, A.polls))) break;
+    if (!(ok = grid_sync<SPIN>(A.ctr, target, &okf))) break;
     for (int j = t; j <= last_i; j += GM_BS) sums[j] = ld_agent(A.y + GM_MAX + j);
     __syncthreads();
     for (int jq = 0; jq <= last_i; jq += 8) {
@@ -717,7 +723,15 @@ hipError_t launch_cooperative(const char* name, const void* kernel, unsigned gri
   return e;
 }
 
-int polls_of(const svg_lhs* L) { return L->oneLaunchPolls < 0 ? SPIN_MAX : L->oneLaunchPolls; }
+const void* cg_kernel(bool wait)
+{
+  return wait ? reinterpret_cast<const void*>(&k_cg_small<SPIN_MAX>) : reinterpret_cast<const void*>(&k_cg_small<0>);
+}
+const void* gmres_kernel(bool wait)
+{
+  return wait ? reinterpret_cast<const void*>(&k_gmres_small<SPIN_MAX>)
+              : reinterpret_cast<const void*>(&k_gmres_small<0>);
+}
 
 // No memory for its buffers, the launch refused, or its workgroups did not meet:
 // the per-launch path, for the lhs's later solves too.
@@ -760,11 +774,12 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
     for (int rows : {128, 64}) {
       const int cap = most_blocks(L, rows);
       if ((int)blocks_for(nNo, rows) > cus || bytes(cap) > 148 * 1024) continue;
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cg_small), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              148 * 1024) != hipSuccess) {
-        (void)hipGetLastError();
-        return SVG_OK;
-      }
+      for (bool wait : {false, true})
+        if (hipFuncSetAttribute(cg_kernel(wait), hipFuncAttributeMaxDynamicSharedMemorySize, 148 * 1024) !=
+            hipSuccess) {
+          (void)hipGetLastError();
+          return SVG_OK;
+        }
       if (dev_alloc(&w.cgEx, (size_t)8 * nNo) || dev_alloc(&w.ctr, 1)) {
         dev_free(w.cgEx);
         (void)hipGetLastError();
@@ -776,15 +791,15 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
     }
     if (w.smallRows < 0) return SVG_OK;
   }
-  int rows = w.smallRows, cap = w.smallCap, capU = std::min(cap, nNo), n = nNo, polls = polls_of(L);
+  int rows = w.smallRows, cap = w.smallCap, capU = std::min(cap, nNo), n = nNo;
   hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, w.ctr, &w.cg->pad);
   const int *rp = L->d_rowPtr, *cp = L->d_colPtr;
   const double *mG = w.mG, *Gt = w.Gt, *mL = w.mL;
   double *X = w.cgX, *gpp = w.cgEx, *pr = w.cgEx + (size_t)4 * nNo, *prod = w.cgEx + (size_t)6 * nNo,
          *rcv = w.cgEx + (size_t)7 * nNo;
   void* args[] = {&n,    &rp,   &cp,   &mG,    &Gt,  &mL,   &R,    &X,    &pr,     &gpp,
-                  &prod, &rcv,  &w.cg, &w.ctr, &rows, &cap, &capU, &polls, &mItr, &absTol, &relTol};
-  if (launch_cooperative("cg_small", reinterpret_cast<const void*>(&k_cg_small), blocks_for(nNo, rows), CG_BS, args,
+                  &prod, &rcv,  &w.cg, &w.ctr, &rows, &cap, &capU, &mItr, &absTol, &relTol};
+  if (launch_cooperative("cg_small", cg_kernel(L->oneLaunchWait), blocks_for(nNo, rows), CG_BS, args,
                          (unsigned)bytes(cap), s) != hipSuccess) {
     (void)hipGetLastError();
     return missed(L);
@@ -827,11 +842,11 @@ bool gmres_small_fits(svg_lhs* L, int sD)
       capU = std::max(capU, nu);
     }
     if ((size_t)GM_BLK_B * cap + (size_t)GM_COL_B * capU > GM_LDS) return false;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gmres_small), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            GM_LDS) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
+    for (bool wait : {false, true})
+      if (hipFuncSetAttribute(gmres_kernel(wait), hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
     k.smallCap = cap;
     k.smallCapU = capU;
   }
@@ -851,7 +866,6 @@ int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double
   GmSmall A{};
   A.nNo = L->nNo;
   A.sD = ls->sD;
-  A.polls = polls_of(L);
   A.cap = k.smallCap;
   A.capU = k.smallCapU;
   A.rowPtr = L->d_rowPtr;
@@ -872,8 +886,7 @@ int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double
     A.cycles = std::min(GM_CYCLES, ls->mItr - done);
     hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, k.ctr, &k.st->pad);
     void* args[] = {&A};
-    if (launch_cooperative("gmres_small", reinterpret_cast<const void*>(&k_gmres_small), 4 * nblk, GM_BS, args, bytes,
-                           s) != hipSuccess) {
+    if (launch_cooperative("gmres_small", gmres_kernel(L->oneLaunchWait), 4 * nblk, GM_BS, args, bytes, s) != hipSuccess) {
       (void)hipGetLastError();
       return missed(L);
     }
@@ -900,10 +913,10 @@ extern "C" int svg_one_launch_info(const svg_lhs* L, svg_one_launch* info)
   return SVG_OK;
 }
 
-extern "C" int svg_one_launch_set(svg_lhs* L, int on, int polls)
+extern "C" int svg_one_launch_set(svg_lhs* L, int on, int wait)
 {
   if (!L) return set_error(SVG_ERR_ARG, "svg_one_launch_set: null lhs");
   L->oneLaunch = on != 0;
-  L->oneLaunchPolls = polls;
+  L->oneLaunchWait = wait != 0;
   return SVG_OK;
 }

@@ -286,7 +286,7 @@ def test_gmres_small_by_launches(torch_cuda, phys, n, nz, how):
         assert (ls.RI.itr, ls.RI.suc, ls.RI.iNorm, ls.RI.fNorm) == (ols.RI.itr, ols.RI.suc, ols.RI.iNorm, ols.RI.fNorm)
         assert np.array_equal(dR.cpu().numpy(), x0)
         assert _one_launch(L) == (0, 0, 0 if how == "off" else 1)
-    _lib.call("svg_one_launch_set", L.h, 1, -1)  # on again
+    _lib.call("svg_one_launch_set", L.h, 1, 1)  # on again
     dR, dV = _dev(torch, R), _dev(torch, V)
     fsils_solve(L, ls, 4, dR, dV)
     assert np.array_equal(dR.cpu().numpy(), x0)
