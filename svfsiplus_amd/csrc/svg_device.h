@@ -223,8 +223,9 @@ struct NsWork {
   double* h_dots = nullptr;
   double* partial = nullptr;
   int partialCap = 0;
-  // the Schur CG as one launch (cg_small): rows of a workgroup (0 not looked at, -1 does not fit), its most blocks
-  int smallRows = 0, smallCap = 0;
+  // the Schur CG as one launch (cg_small): rows of a workgroup (0 not looked at, -1 does not fit), its most
+  // blocks and most columns
+  int smallRows = 0, smallCap = 0, smallCapU = 0;
   double* cgEx = nullptr;   // its exchanged vectors (8 nNo)
   int* ctr = nullptr;       // its barrier
 };

@@ -125,16 +125,18 @@ __device__ __forceinline__ double sum_all(int n, double* ws, Get get)
 // cgrad::schur (cgrad.cpp:50-160) without coupled faces, as k_cg_init ..
 // k_cg_p compute it. A workgroup owns `rows` rows; its blocks of G, G^T and L
 // stay in LDS for the whole solve, and so does the list of the columns they
-// touch, whose entries of the exchanged vectors it loads once a phase (about
-// 300 for 128 rows; a load per block went past the caches 13 times a row).
+// touch, whose entries of the exchanged vectors it loads once a phase (300 to
+// 470 for 128 rows; a load per block went past the caches 13 times a row).
 // Three barriers an iteration:
 //   1  |R|^2 and the stop test; P = c2 (P + c1 R) of the listed columns, and
 //      GP = G P                                          -> gpp = (GP, P)
 //   2  SP = L P - G^T GP; P SP                           -> prod
 //   3  <P, SP>, alpha; X += alpha P; R -= alpha SP       -> pr = (P, R), rc = R
-// On the 15k-tet pipe (3 321 nodes, 26 workgroups) an iteration takes 15 us, 6
-// of them at the barriers; as four launches it took 52 us, 31 of them in a
-// product of one lane per four rows.
+// On the 15k-tet pipe (3 321 nodes, 26 workgroups) an iteration takes 13.2 us, 6
+// of them at the barriers (14.9 with 64 rows a workgroup); as four launches it
+// took 52 us, 31 of them in a product of one lane per four rows. The two sums
+// over all rows grow with the system: 44 us at 32 490 nodes (84 as launches,
+// 45 of them in the product).
 constexpr int CG_BS = 256;
 // LDS bytes per block (seven values, the column's place in the list) and per listed column (its place's
 // id and up to four values), and of the column bitmap
@@ -744,13 +746,25 @@ int missed(svg_lhs* L)
 
 }  // namespace
 
-// The most blocks of a group of `rows` consecutive rows.
-static int most_blocks(const svg_lhs* L, int rows)
+// The most blocks of a workgroup and the most different columns they touch:
+// workgroup w's rows are the ranges [a, e) that part(w, r, a, e) gives for r < parts.
+template <typename Part>
+static void most_blocks(const svg_lhs* L, int wgs, int parts, Part part, int* cap, int* capU)
 {
-  int most = 0;
-  for (int r = 0; r < L->nNo; r += rows)
-    most = std::max(most, L->rowPtr[std::min(L->nNo, r + rows)] - L->rowPtr[r]);
-  return most;
+  *cap = *capU = 0;
+  std::vector<int> seen(L->nNo, -1);
+  for (int w = 0; w < wgs; w++) {
+    int nb = 0, nu = 0;
+    for (int r = 0; r < parts; r++) {
+      int a, e;
+      part(w, r, a, e);
+      nb += L->rowPtr[e] - L->rowPtr[a];
+      for (int j = L->rowPtr[a]; j < L->rowPtr[e]; j++)
+        if (seen[L->colPtr[j]] != w) seen[L->colPtr[j]] = w, nu++;
+    }
+    *cap = std::max(*cap, nb);
+    *capU = std::max(*capU, nu);
+  }
 }
 
 // The Schur CG of w's split system as one launch: *ran = 0 when the system does
@@ -763,17 +777,19 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
   if (!L->oneLaunch || w.smallRows < 0) return SVG_OK;
   const int nNo = L->nNo;
   int rc;
-  auto bytes = [&](int cap) {
-    return (size_t)CG_BLK_B * cap + (size_t)CG_COL_B * std::min(cap, nNo);
-  };
+  auto bytes = [](int cap, int capU) { return (size_t)CG_BLK_B * cap + (size_t)CG_COL_B * capU; };
   if (w.smallRows == 0) {
     int cus = 0;
     w.smallRows = -1;
     if ((rc = num_cus(&cus))) return rc;
     if (nNo > 1024 * SUM_SPANS) return SVG_OK;
     for (int rows : {128, 64}) {
-      const int cap = most_blocks(L, rows);
-      if ((int)blocks_for(nNo, rows) > cus || bytes(cap) > 148 * 1024) continue;
+      const int wgs = (int)blocks_for(nNo, rows);
+      if (wgs > cus) continue;
+      int cap, capU;
+      auto part = [&](int w, int, int& a, int& e) { a = w * rows, e = std::min(nNo, a + rows); };
+      most_blocks(L, wgs, 1, part, &cap, &capU);
+      if (bytes(cap, capU) > 148 * 1024) continue;
       for (bool wait : {false, true})
         if (hipFuncSetAttribute(cg_kernel(wait), hipFuncAttributeMaxDynamicSharedMemorySize, 148 * 1024) !=
             hipSuccess) {
@@ -787,11 +803,12 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
       }
       w.smallRows = rows;
       w.smallCap = cap;
+      w.smallCapU = capU;
       break;
     }
     if (w.smallRows < 0) return SVG_OK;
   }
-  int rows = w.smallRows, cap = w.smallCap, capU = std::min(cap, nNo), n = nNo;
+  int rows = w.smallRows, cap = w.smallCap, capU = w.smallCapU, n = nNo;
   hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, w.ctr, &w.cg->pad);
   const int *rp = L->d_rowPtr, *cp = L->d_colPtr;
   const double *mG = w.mG, *Gt = w.Gt, *mL = w.mL;
@@ -800,7 +817,7 @@ int cg_small(svg_lhs* L, const double* R, int mItr, double absTol, double relTol
   void* args[] = {&n,    &rp,   &cp,   &mG,    &Gt,  &mL,   &R,    &X,    &pr,     &gpp,
                   &prod, &rcv,  &w.cg, &w.ctr, &rows, &cap, &capU, &mItr, &absTol, &relTol};
   if (launch_cooperative("cg_small", cg_kernel(L->oneLaunchWait), blocks_for(nNo, rows), CG_BS, args,
-                         (unsigned)bytes(cap), s) != hipSuccess) {
+                         (unsigned)bytes(cap, capU), s) != hipSuccess) {
     (void)hipGetLastError();
     return missed(L);
   }
@@ -829,18 +846,10 @@ bool gmres_small_fits(svg_lhs* L, int sD)
     const int nNo = L->nNo, nblk = (4 * nNo + 1023) / 1024;
     int cus = 0, cap = 0, capU = 0;
     if (num_cus(&cus) != SVG_OK || 4 * nblk > cus || nblk > 64) return false;
-    std::vector<int> seen(nNo, -1);
-    for (int w = 0; w < 4 * nblk; w++) {
-      int nb = 0, nu = 0;
-      for (int r = 0; r < 4; r++) {
-        const int a = std::min(nNo, 256 * (w / 4) + 64 * r + 16 * (w % 4)), e = std::min(nNo, a + 16);
-        nb += L->rowPtr[e] - L->rowPtr[a];
-        for (int j = L->rowPtr[a]; j < L->rowPtr[e]; j++)
-          if (seen[L->colPtr[j]] != w) seen[L->colPtr[j]] = w, nu++;
-      }
-      cap = std::max(cap, nb);
-      capU = std::max(capU, nu);
-    }
+    auto part = [&](int w, int r, int& a, int& e) {
+      a = std::min(nNo, 256 * (w / 4) + 64 * r + 16 * (w % 4)), e = std::min(nNo, a + 16);
+    };
+    most_blocks(L, 4 * nblk, 4, part, &cap, &capU);
     if ((size_t)GM_BLK_B * cap + (size_t)GM_COL_B * capU > GM_LDS) return false;
     for (bool wait : {false, true})
       if (hipFuncSetAttribute(gmres_kernel(wait), hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS) != hipSuccess) {
@@ -886,7 +895,8 @@ int gmres_small(svg_lhs* L, const svg_subls* ls, const double* Val, const double
     A.cycles = std::min(GM_CYCLES, ls->mItr - done);
     hipLaunchKernelGGL(k_clear_small, dim3(1), dim3(1), 0, s, k.ctr, &k.st->pad);
     void* args[] = {&A};
-    if (launch_cooperative("gmres_small", gmres_kernel(L->oneLaunchWait), 4 * nblk, GM_BS, args, bytes, s) != hipSuccess) {
+    if (launch_cooperative("gmres_small", gmres_kernel(L->oneLaunchWait), 4 * nblk, GM_BS, args, bytes, s) !=
+        hipSuccess) {
       (void)hipGetLastError();
       return missed(L);
     }

@@ -163,7 +163,10 @@ def _shuffled(n):
     x = np.empty_like(p.x)
     x[to] = p.x
     ien = to[p.IEN][rng.permutation(p.nEl)].astype(np.int32)
-    return W.Pipe(n, 5 * n, x, ien, p.flags, *W.pattern(p.nNo, ien), p.radius, p.length)
+    flags = np.empty_like(p.flags)
+    flags[to] = p.flags
+    faces = [(kind, to[g].astype(np.int32)) for kind, g in p.faces]
+    return W.Pipe(n, 5 * n, x, ien, flags, *W.pattern(p.nNo, ien), p.radius, p.length, faces)
 
 
 @pytest.mark.parametrize("mesh", ["one_tet", "shuffled6", "fan9", "fan31", "fan33", "fan64", "fan65", "fan120"])
@@ -226,11 +229,12 @@ def test_gmres_solve(torch_cuda, phys, n):
     assert rel <= 10 * tol
 
 
-def _one_launch(L):
+def _one_launch(L, rows=128):
     """The lhs's solves that ran as one launch (GMRES, Schur CG) and the misses."""
     import ctypes as C
     info = _lib.OneLaunch()
     _lib.call("svg_one_launch_info", L.h, C.byref(info))
+    assert info.cg_rows == rows or info.cg == 0
     return info.gmres, info.cg, info.missed
 
 
@@ -488,11 +492,12 @@ def test_coupled_ns_solver(torch_cuda):
 
 
 @pytest.mark.parametrize("how", ["one launch", "off", "missed"])
-@pytest.mark.parametrize("n,nz", [(2, 3), (4, 7), (12, 30), (16, 40)])
+@pytest.mark.parametrize("n,nz", [(2, 3), (4, 7), (12, 30), (16, 40), (16, 60), (10, 0)])
 def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz, how):
     """The NS solver with its Schur CG as one launch (less than one workgroup's
-    rows, a ragged last one, 6 and 12 reduction spans, four of which are summed at
-    a time), by the launches of larger systems, and by those after the first CG's
+    rows, a ragged last one, 6, 12 and 18 reduction spans, four of which are summed
+    at a time; 128 rows a workgroup, so that the largest has 138; with the nodes in
+    no order, 64 rows, whose blocks touch more columns), by the launches of larger systems, and by those after the first CG's
     workgroups found no one at their barrier (a wait of no polls): bit for bit
     the device-order oracle, counts and all."""
     from svfsiplus_amd.newton import DeviceLhs, fsils_solve
@@ -500,7 +505,7 @@ def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz, how):
     torch = torch_cuda
     if how == "missed" and n == 2:
         pytest.skip("a single workgroup always meets itself")
-    p = W.make_pipe(n, nz=nz)
+    p = W.make_pipe(n, nz=nz) if nz else _shuffled(n)
     Ag, Yg = _state(p, phys, seed=n)
     R, V = oracle.construct_fluid(p, phys, Ag, Yg)
     ols = oracle.ls_create(oracle.LS_NS, absTol=1e-30, maxItr=2)
@@ -517,7 +522,7 @@ def test_ns_solver_one_launch_cg(torch_cuda, phys, n, nz, how):
     assert (ls.RI.fNorm, ls.CG.fNorm, ls.CG.iNorm) == (ols.RI.fNorm, ols.CG.fNorm, ols.CG.iNorm)
     assert np.array_equal(dR.cpu().numpy(), x0)
     # one CG in each of the two outer iterations; after a miss none tries again
-    assert _one_launch(L) == (0, 2 if how == "one launch" else 0, 1 if how == "missed" else 0)
+    assert _one_launch(L, 128 if nz else 64) == (0, 2 if how == "one launch" else 0, 1 if how == "missed" else 0)
 
 
 def test_one_launch_solves_are_timed(torch_cuda, phys):
