@@ -318,7 +318,10 @@ __global__ __launch_bounds__(256) void k_contrib_keys(int nEl, const int4* __res
 // of more entries alone), packed greedily along each window of kGatherRows
 // rows, one lane per window: FILL = false counts a window's chunks, true
 // writes their first slots from off[window] on. 16 rows (about 1440 entries)
-// leave half a chunk of 23 unfilled at a window's end.
+// leave half a chunk of 23 unfilled at a window's end. A chunk's slots all have
+// entries or none has: the gather writes every slot of a chunk that has any, and
+// the slots without are other meshes' of the same lhs, which another stream may
+// be assembling.
 constexpr int kGatherRows = 16;
 template <bool FILL>
 __global__ __launch_bounds__(64) void k_chunks(int nWin, int nNo, int nnz, const int* __restrict__ rowPtr,
@@ -332,19 +335,23 @@ __global__ __launch_bounds__(64) void k_chunks(int nWin, int nNo, int nnz, const
   int first = rowPtr[w * kGatherRows], c0 = cptr[first];
   if (FILL && first < s1) chunk[n] = make_int2(first, c0);
   const int open = first < s1 ? 1 : 0;
+  int last = c0;  // the first entry of slot s + q
   for (int s = first; s < s1; s += 8) {
     int end[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) end[q] = cptr[min(s + q, s1 - 1) + 1];
 #pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (s + q < s1 && s + q > first && (end[q] - c0 > 64 || s + q - first >= 64)) {
+    for (int q = 0; q < 8; q++) {
+      const bool mixed = (end[q] == last) != (last == c0);
+      if (s + q < s1 && s + q > first && (end[q] - c0 > 64 || s + q - first >= 64 || mixed)) {
         // slot s + q opens the next chunk
         n++;
         first = s + q;
-        c0 = q > 0 ? end[q - 1] : cptr[s];
+        c0 = last;
         if (FILL) chunk[n] = make_int2(first, c0);
       }
+      last = end[q];
+    }
   }
   if (!FILL) off[w] = n + open;
   if (FILL && w == nWin - 1) chunk[n + open] = make_int2(nnz, cptr[nnz]);

@@ -229,6 +229,52 @@ def test_gmres_solve(torch_cuda, phys, n):
     assert rel <= 10 * tol
 
 
+def test_construct_fluid_of_two_meshes_at_once(torch_cuda, phys):
+    """Two meshes of one lhs, whose nodes alternate and which share none, assembled
+    into one R and Val by two threads on streams of their own: each adds to its own
+    block slots and rows only, whatever the other is doing to the slots between."""
+    import threading
+    from svfsiplus_amd.newton import DeviceLhs, DeviceMesh, construct_fluid
+    torch = torch_cuda
+    p = W.make_pipe(8)
+    x = np.repeat(p.x, 2, axis=0)
+    ien = [2 * p.IEN, 2 * p.IEN + 1]
+    both = np.concatenate(ien).astype(np.int32)
+    full = W.Pipe(0, 0, x, both, np.zeros(len(x), np.int32), *W.pattern(len(x), both), p.radius, p.length)
+    L = DeviceLhs(full, faces=[])
+    half = [W.Pipe(0, 0, x, q.astype(np.int32), full.flags, full.rowPtr, full.colPtr, p.radius, p.length) for q in ien]
+    M = [DeviceMesh(L, h) for h in half]
+    rng = np.random.default_rng(8)
+    Ag, Yg = rng.standard_normal((2, full.nNo, 4))
+    R0, V0 = oracle.construct_fluid(full, phys, Ag, Yg)
+    dA, dY = _dev(torch, Ag), _dev(torch, Yg)
+    streams = [torch.cuda.Stream() for _ in M]
+    dR, dV = _dev(torch, np.zeros_like(R0)), _dev(torch, np.zeros_like(V0))
+    for _ in range(20):
+        dR.zero_()
+        dV.zero_()
+        torch.cuda.synchronize()
+        start = threading.Barrier(2)
+        failed = []
+
+        def work(m, s):
+            try:
+                with torch.cuda.stream(s):
+                    start.wait()
+                    construct_fluid(m, phys, dA, dY, dR, dV)
+            except Exception as e:
+                failed.append(e)
+
+        t = [threading.Thread(target=work, args=a) for a in zip(M, streams)]
+        for q in t:
+            q.start()
+        for q in t:
+            q.join()
+        torch.cuda.synchronize()
+        assert not failed, failed
+        assert np.array_equal(dR.cpu().numpy(), R0) and np.array_equal(dV.cpu().numpy(), V0)
+
+
 def _one_launch(L, rows=128):
     """The lhs's solves that ran as one launch (GMRES, Schur CG) and the misses."""
     import ctypes as C
