@@ -500,12 +500,12 @@ int svg_lhs_create_dev(int nNo, int nEl, const int* d_IEN, int nFaces, svg_lhs**
   if ((unsigned long long)nNo * (unsigned long long)nNo >= (1ULL << 62))
     return set_error(SVG_ERR_ARG, "svg_lhs_create_dev: nNo too large");
   const long long K = 16LL * nEl + nNo;
-  Scratch S(sizeof(unsigned long long) * 4 * (size_t)std::min(K, 0x7fffffffLL) + ((size_t)4 << 20));
+  if (K > 0x7fffffffLL) return set_error(SVG_ERR_ARG, "svg_lhs_create_dev: too many node pairs");
+  Scratch S(sizeof(unsigned long long) * 4 * (size_t)K + ((size_t)4 << 20));
   int rc;
   int* d_err = nullptr;
   if ((rc = S.get(&d_err, 1))) return rc;
   if ((rc = check_ien(4LL * nEl, d_IEN, nNo, d_err, s, "svg_lhs_create_dev"))) return rc;
-  if (K > 0x7fffffffLL) return set_error(SVG_ERR_ARG, "svg_lhs_create_dev: too many node pairs");
   unsigned long long *keys = nullptr, *sorted = nullptr, *uniq = nullptr;
   int* d_nnz = nullptr;
   if ((rc = S.get(&keys, (size_t)K)) || (rc = S.get(&sorted, (size_t)K)) || (rc = S.get(&uniq, (size_t)K)) ||

@@ -177,3 +177,12 @@ def test_ls_create_defaults_match_reference():
         for name in ("RI", "GM", "CG"):
             for f, r in ref[name].items():
                 assert got[name][f] == (0 if r == -7777.0 else r), (t, name, f)
+
+
+def test_device_lhs_refuses_too_many_pairs_up_front():
+    """2^31 node pairs are refused by their number alone, before scratch memory is
+    taken for them (64 GB) or the connectivity is looked at."""
+    ien, h = np.zeros(64, np.int32), C.c_void_p()
+    at = (ien.ctypes.data + 15) & ~15
+    with pytest.raises(_lib.SvgError, match="too many node pairs"):
+        _lib.check(_lib.load().svg_lhs_create_dev(4, 2**27, at, 0, C.byref(h), None))
