@@ -615,7 +615,7 @@ int svg_msh_create_dev(const svg_lhs* L, int nEl, const int* d_IEN, const double
   int h[4] = {0, 1, 0, 0};
   int r = 1;
   while (h[r % 3] > 0) {
-    if (r > 100000) return set_error(SVG_ERR_ARG, "svg_msh_create_dev: colouring did not finish");
+    if (r > 400000) return set_error(SVG_ERR_ARG, "svg_msh_create_dev: colouring did not finish");
     // 32 rounds per host check: a round with an empty list does nothing
     for (int k = 0; k < 32; k++) {
       r++;

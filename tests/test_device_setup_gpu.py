@@ -117,6 +117,14 @@ def test_device_setup_rejects_bad_connectivity(torch_cuda):
         W.pattern(p.nNo, ien)
 
 
+def _priority(n):
+    """The device colouring's priorities of n elements."""
+    x = np.arange(n, dtype=np.uint32) * np.uint32(2654435761) + np.uint32(0x9E3779B9)
+    for shift, mul in ((16, 0x85EBCA6B), (13, 0xC2B2AE35)):
+        x = (x ^ (x >> np.uint32(shift))) * np.uint32(mul)
+    return (x ^ (x >> np.uint32(16))).astype(np.int64)
+
+
 @pytest.mark.parametrize("kind", ["pipe", "random"])
 def test_device_colouring_is_the_priority_greedy(torch_cuda, kind):
     """The device colouring is the sequential greedy one in decreasing element
@@ -134,13 +142,9 @@ def test_device_colouring_is_the_priority_greedy(torch_cuda, kind):
     off, ien = np.empty(M.nColors + 1, np.int32), np.empty((p.nEl, 4), np.int32)
     _lib.call("svg_msh_colors", M.h, off.ctypes.data)
     _lib.call("svg_msh_sorted_ien", M.h, ien.ctypes.data)
-    x = np.arange(p.nEl, dtype=np.uint32) * np.uint32(2654435761) + np.uint32(0x9E3779B9)
-    for shift, mul in ((16, 0x85EBCA6B), (13, 0xC2B2AE35)):
-        x = (x ^ (x >> np.uint32(shift))) * np.uint32(mul)
-    x ^= x >> np.uint32(16)
     used = [set() for _ in range(p.nNo)]
     color = np.empty(p.nEl, np.int64)
-    for e in np.argsort(-x.astype(np.int64)):
+    for e in np.argsort(-_priority(p.nEl)):
         taken = set().union(*(used[v] for v in p.IEN[e]))
         color[e] = next(c for c in range(257) if c not in taken)
         for v in p.IEN[e]:
@@ -148,3 +152,22 @@ def test_device_colouring_is_the_priority_greedy(torch_cuda, kind):
     assert M.nColors == color.max() + 1
     assert np.array_equal(np.diff(off), np.bincount(color))
     assert np.array_equal(ien, p.IEN[np.argsort(color, kind="stable")])
+
+
+def test_device_colouring_of_a_long_chain(torch_cuda):
+    """A strip of tets whose priorities fall along it takes a colouring round per
+    tet; 101 000 of them are within the rounds that a set-up may take."""
+    from svfsiplus_amd.newton import DeviceLhs, DeviceMesh, device_arrays
+    n = 101000
+    ien = np.empty((n, 4), np.int32)
+    ien[np.argsort(-_priority(n))] = np.arange(n)[:, None] + np.arange(4)
+    x = np.random.default_rng(1).standard_normal((n + 3, 3))
+    p = W.Pipe(0, 0, x, ien, np.zeros(n + 3, np.int32), *W.pattern(n + 3, ien), 0.3, 3.0)
+    d_ien, d_x = device_arrays(p)
+    M = DeviceMesh(DeviceLhs(p, d_ien=d_ien), p, d_ien=d_ien, d_x=d_x)
+    off, got = np.empty(5, np.int32), np.empty((n, 4), np.int32)
+    assert M.nColors == 4
+    _lib.call("svg_msh_colors", M.h, off.ctypes.data)
+    _lib.call("svg_msh_sorted_ien", M.h, got.ctypes.data)
+    for c in range(4):  # along the strip the colours follow each other
+        assert np.array_equal(np.sort(got[off[c]:off[c + 1], 0]), np.arange(c, n, 4))
