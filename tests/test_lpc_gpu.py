@@ -93,7 +93,8 @@ def test_lpc_gradient_of_stacked_vectors(torch_cuda, nvec):
     (6: with a remainder) gives the mean of the one-vector calls. The forward
     pass and the FP64 residuals of a vector do not depend on the stack (loss:
     FP64 summation order only); the gradient's BF16 roundings are unchanged by
-    the factor 1/8, so for 8 vectors only the FP32 summation order differs."""
+    the factor 1/8, so for 8 vectors only the FP32 summation order differs, and
+    for 6 the roundings."""
     torch = torch_cuda
     sys = _sys(torch, n=16)
     net = L.LearnedPC(_params(5))
@@ -110,9 +111,10 @@ def test_lpc_gradient_of_stacked_vectors(torch_cuda, nvec):
     loss, grad = call(R)
     want = np.mean([o[0] for o in one])
     assert abs(loss - want) <= 1e-12 * want
-    if nvec == 8:
-        g = np.mean([o[1] for o in one], axis=0)
-        assert np.linalg.norm(grad - g) <= 1e-5 * np.linalg.norm(g)
+    # under the factor 1/6 the backward pass rounds otherwise: a few BF16 roundings
+    # of 2^-9; a vector left out changes the mean by a sixth
+    g = np.mean([o[1] for o in one], axis=0)
+    assert np.linalg.norm(grad - g) <= (1e-5 if nvec == 8 else 2e-2) * np.linalg.norm(g)
 
 
 def test_lpc_training_reduces_loss(torch_cuda):
