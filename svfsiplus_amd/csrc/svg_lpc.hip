@@ -760,7 +760,7 @@ __global__ __launch_bounds__(BS) void k_layer_bwd(int rows, const float* __restr
 
 // Transposed message passing: Gin[j] += sum_{i : j in row i} A_ij^T (x) GM[i];
 // one lane per (row j, channel c), the block read as two 16-byte words (the
-// row's 16 lanes share it) and two blocks' loads issued before their sums.
+// row's 16 lanes share it) and four blocks' loads issued before their sums.
 __device__ __forceinline__ void spmmT_block(float4& e, const uint4& lo4, const uint4& hi4, const float4& g)
 {
   const unsigned r0[2] = {lo4.x, lo4.y}, r1[2] = {lo4.z, lo4.w}, r2[2] = {hi4.x, hi4.y}, r3[2] = {hi4.z, hi4.w};
@@ -1157,18 +1157,22 @@ static int lpc_loss_grad(svg_lpc* N, svg_lhs* L, const double* Val, int nvec, co
   const unsigned nbv = blocks_for((size_t)4 * n, 256);
   // Res = T - A Z (FP64, in the solver's SpMV order), GZ = -(2/B) A^T Res
   const double* Tt = T ? T : R;
-  if ((size_t)4 * rows <= NV_MIN_LANES) {
-    launch("lpc_res", k_residual_nv<1>, dim3(nbv, nvec), dim3(256), 0, s, n, nvec, (const int*)L->d_rowPtr,
-           (const int*)L->d_colPtr, Val, (const double*)N->Z, Tt, N->Res);
-    launch("lpc_spmvT", k_spmvT<1>, dim3(nbv, nvec), dim3(256), 0, s, n, nvec, (const int*)L->d_rowPtr,
-           (const int*)L->d_colPtr, (const int*)L->d_trans, Val, (const double*)N->Res, N->GZ, -2.0 / nvec);
-  } else {
-    launch("lpc_res", k_residual_nv<4>, dim3(nbv, blocks_for(nvec, 4)), dim3(256), 0, s, n, nvec,
-           (const int*)L->d_rowPtr, (const int*)L->d_colPtr, Val, (const double*)N->Z, Tt, N->Res);
-    launch("lpc_spmvT", k_spmvT<4>, dim3(nbv, blocks_for(nvec, 4)), dim3(256), 0, s, n, nvec,
-           (const int*)L->d_rowPtr, (const int*)L->d_colPtr, (const int*)L->d_trans, Val, (const double*)N->Res,
-           N->GZ, -2.0 / nvec);
-  }
+  auto residuals = [&](auto residual, auto transposed, int nv) {
+    // at most 2^16 - 1 groups of vectors a launch, the grid's limit along y
+    const int most = 0xffff * nv;
+    for (int b = 0; b < nvec; b += most) {
+      const int m = std::min(nvec - b, most);
+      const size_t o = (size_t)4 * n * b;
+      launch("lpc_res", residual, dim3(nbv, blocks_for(m, nv)), dim3(256), 0, s, n, m, (const int*)L->d_rowPtr,
+             (const int*)L->d_colPtr, Val, (const double*)(N->Z + o), Tt + o, N->Res + o);
+      launch("lpc_spmvT", transposed, dim3(nbv, blocks_for(m, nv)), dim3(256), 0, s, n, m, (const int*)L->d_rowPtr,
+             (const int*)L->d_colPtr, (const int*)L->d_trans, Val, (const double*)(N->Res + o), N->GZ + o, -2.0 / nvec);
+    }
+  };
+  if ((size_t)4 * rows <= NV_MIN_LANES)
+    residuals(k_residual_nv<1>, k_spmvT<1>, 1);
+  else
+    residuals(k_residual_nv<4>, k_spmvT<4>, 4);
   launch("lpc_loss", k_sqsum, dim3(256), dim3(256), 0, s, (size_t)rows * 4, (const double*)N->Res, N->sq);
   const unsigned ng = std::min<unsigned>(MAXGRID, blocks_for(rows, TILE));
   const bf16* pb = N->pb;

@@ -117,6 +117,31 @@ def test_lpc_gradient_of_stacked_vectors(torch_cuda, nvec):
     assert np.linalg.norm(grad - g) <= (1e-5 if nvec == 8 else 2e-2) * np.linalg.norm(g)
 
 
+def test_lpc_gradient_of_very_many_vectors(torch_cuda):
+    """More vectors than one launch of the residual kernels takes (4 * 65 535): the
+    five past it, a thousand times as large, carry most of the loss and gradient."""
+    torch = torch_cuda
+    sys = L.ScaledSystem(W.make_pipe(2, nz=1), W.Physics())
+    net = L.LearnedPC(_params(7))
+    lib, n = _lib.load(), 4 * 65535
+    g = torch.Generator(device="cuda").manual_seed(3)
+    V = torch.randn((2, sys.n, 4), dtype=torch.float64, device="cuda", generator=g)
+    V[1] *= 1e3
+
+    def call(V):
+        loss, g = C.c_double(), np.empty(L.num_params(), dtype=np.float32)
+        _lib.check(lib.svg_lpc_loss_grad(net.h, sys.lhs.h, sys.Val.data_ptr(), V.shape[0], V.data_ptr(),
+                                         C.byref(loss), g.ctypes.data, _stream()))
+        return loss.value, g.astype(np.float64)
+
+    (la, ga), (lb, gb) = call(V[:1].contiguous()), call(V[1:].contiguous())
+    loss, grad = call(torch.cat([V[:1].expand(n, -1, -1), V[1:].expand(5, -1, -1)]).contiguous())
+    want, g = (n * la + 5 * lb) / (n + 5), (n * ga + 5 * gb) / (n + 5)
+    assert 5 * lb > n * la
+    assert abs(loss - want) <= 1e-10 * want
+    assert np.linalg.norm(grad - g) <= 2e-2 * np.linalg.norm(g)
+
+
 def test_lpc_training_reduces_loss(torch_cuda):
     torch = torch_cuda
     sys = _sys(torch)
