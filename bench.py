@@ -683,7 +683,7 @@ def batch_run(a, log):
         out["twolevel"] = {"coarse": coarse, "meshes_fallen_back": fallbacks}
     u = bn.pipe
     bn.free()
-    # the union's mesh setup (block pattern, colouring, colour order, slot map): host and device builds
+    # the union's mesh setup (block pattern, colouring, colour order, the slots' entries): host and device builds
     from svfsiplus_amd.newton import DeviceLhs, DeviceMesh, device_arrays
     torch.cuda.synchronize()
     t = time.perf_counter()
@@ -700,7 +700,7 @@ def batch_run(a, log):
     td = time.perf_counter() - t
     out["setup_s"] = {"host": round(th, 3), "device": round(td, 3),
                       "colours": {"host": Mh.nColors, "device": Md.nColors},
-                      "note": "block pattern + colouring + colour order + slot map of the union (host: C++ on one "
+                      "note": "block pattern + colouring + colour order + slot entries of the union (host: C++ on one "
                               "core, then upload; device: upload of IEN and x, then svg_lhs_create_dev and "
                               "svg_msh_create_dev)"}
     log(f"# batch union setup: host {th:.3f}s, device {td:.3f}s")

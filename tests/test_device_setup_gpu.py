@@ -2,8 +2,7 @@
 block pattern equals the host build (lhsa.cpp:153-380) entry for entry; the
 Jones-Plassmann colouring is a valid colouring (no two elements of a colour
 share a node) with a stable colour order; the assembly through the device-
-built slot map equals the host-built one to rounding (only the order of the
-colour launches differs); a Newton time step on the device-built setup
+built setup equals the host-built one; a Newton time step on the device-built setup
 matches the host-built one."""
 import ctypes as C
 
