@@ -496,10 +496,12 @@ constexpr int MDOT_CB_G = 4;  // FP32 basis columns per load batch (4: 24.1 us, 
 
 // Columns a workgroup of the dots' first pass takes. With few spans a workgroup
 // a span leaves compute units waiting on one column batch's latency after the
-// other: the columns are split over up to `wgs` workgroups in all, eight columns
-// at least each (w is read again by each of them). 230 spans, FP32 basis: 10.4
-// -> 6.9 us a step; 810 spans: FP32 19.3 -> 18.7 us with two, FP64 (twice the
-// bytes in flight) 31.7 -> 33.5, so it is split only below 512 spans.
+// other: the columns are split over up to `wgs` workgroups in all, about eight
+// columns each and five at least (w is read again by each of them). 230 spans,
+// FP32 basis: 10.4 -> 6.9 us a step; 414 spans, FP64: 21.7 -> 17.4; 819 spans:
+// FP32 19.3 -> 18.7 us with two, FP64 (twice the bytes in flight) 31.7 -> 33.5, so
+// that is split up to 512 spans. A Newton iteration of 24, 64 and 128 FP32-basis
+// meshes gains 5, 3 and 0.3 %; 256 have too many spans for it.
 constexpr int DOT_WGS_F32 = 2048, DOT_WGS_F64 = 1024;
 static int dot_cols(int nblk, int mc, int wgs)
 {
@@ -539,9 +541,9 @@ __device__ __forceinline__ void mdot_body(const TWv* __restrict__ w, const T* __
 // 819 spans make four wavefronts a SIMD at most: 31.0 us, 31.5 with register
 // moves, 32.7 with the next column's loads issued ahead of the sums.
 template <int G>
-__global__ __launch_bounds__(RED_BS) __attribute__((amdgpu_waves_per_eu(1, G == 1 ? 4 : 8))) void k_mdot(int n, const double* __restrict__ w, const double* __restrict__ base,
-                                                 size_t ld, int m, int cols, double* __restrict__ partial,
-                                                 const int* __restrict__ skip)
+__global__ __launch_bounds__(RED_BS) __attribute__((amdgpu_waves_per_eu(1, G == 1 ? 4 : 8))) void k_mdot(
+    int n, const double* __restrict__ w, const double* __restrict__ base, size_t ld, int m, int cols,
+    double* __restrict__ partial, const int* __restrict__ skip)
 {
   extern __shared__ double lds[];  // [RED_NW waves][cols]
   if (skip && *skip) return;
@@ -2497,11 +2499,10 @@ static int precond_diag_dev(svg_lhs* L, int dof, double* Val, double* R, double*
 // Newton iteration of 256 FP64 meshes: 404.4 ms, 406.2 with shuffles, 410 to 412
 // with eight wavefronts a SIMD).
 template <int G>
-__global__ __launch_bounds__(RED_BS) __attribute__((amdgpu_waves_per_eu(1, G == 1 ? 4 : 8))) void k_bmdot(const int* __restrict__ spanStart, const int* __restrict__ spanEnd,
-                                                  const int* __restrict__ spanSys, int nsp,
-                                                  const double* __restrict__ w, const double* __restrict__ base,
-                                                  size_t ld, int m, int cols, double* __restrict__ partial,
-                                                  const GmState* __restrict__ st, int check)
+__global__ __launch_bounds__(RED_BS) __attribute__((amdgpu_waves_per_eu(1, G == 1 ? 4 : 8))) void k_bmdot(
+    const int* __restrict__ spanStart, const int* __restrict__ spanEnd, const int* __restrict__ spanSys, int nsp,
+    const double* __restrict__ w, const double* __restrict__ base, size_t ld, int m, int cols,
+    double* __restrict__ partial, const GmState* __restrict__ st, int check)
 {
   extern __shared__ double lds[];  // [RED_NW waves][cols]
   const int b = blockIdx.x;
@@ -2621,7 +2622,9 @@ __global__ __launch_bounds__(256) void k_bgs_update_cb(int n, double* __restrict
 // first one also records the Hessenberg column, the rotation and the state.
 // That record may set `done` while others still start: they skip then, and
 // what they would write is not read (the cycle ends at column i). 230 spans:
-// 8.2 us a step, 4.9 + 7.5 and a launch gap as two.
+// 8.2 us a step, 4.9 + 7.5 and a launch gap as two. More meshes keep the gain: a
+// Newton iteration of 24, 128 and 256 meshes of 5k to 16k tets 35.9, 100.8 and
+// 153.6 ms (39.6, 108.8 and 160.7 as two), of 256 up to 80k tets 298 (305).
 constexpr int BFU_BS = RED_SPAN / 2;
 __global__ __launch_bounds__(BFU_BS) void k_bfin_update_cb(
     FinArgs A, const int* __restrict__ spanStart, const int* __restrict__ spanEnd, const int* __restrict__ spanSys,
